@@ -94,6 +94,18 @@ int pamd_nrm2_large_f64(int64_t n, const double* x, double* result,
 int pamd_trsv_upper_f64(int trans, int64_t n, const double* R, int64_t ldr,
                         double* x, void* stream);
 
+/* The same solves from a packed copy of R (n <= 1024), for a triangle that is
+ * solved with more than once: pack writes both directions' blocks in the order
+ * the solve reads them (query the size first; R may be freed afterwards, and
+ * the packed copy serves any number of solves on any stream ordered after the
+ * packing).  x <- R^{-1} x (trans = 0) or R^{-T} x in place; same rounding
+ * bound as pamd_trsv_upper_f64.  Only R's upper triangle is read. */
+int pamd_trsv_pack_workspace(int64_t n, int64_t* bytes);
+int pamd_trsv_pack_f64(int64_t n, const double* R, int64_t ldr, void* packed,
+                       void* stream);
+int pamd_trsv_packed_f64(int trans, int64_t n, const void* packed, double* x,
+                         void* stream);
+
 /* ------------------------------------------------------------------------ */
 /* Sketching operators                                                      */
 /* ------------------------------------------------------------------------ */

@@ -46,6 +46,9 @@ SIGNATURES = {
     "pamd_gemv_workspace": (c_int, [c_int, c_i64, c_i64, ctypes.POINTER(c_i64)]),
     "pamd_nrm2_f64": (c_int, [c_i64, c_vp, c_vp, c_vp]),
     "pamd_trsv_upper_f64": (c_int, [c_int, c_i64, c_vp, c_i64, c_vp, c_vp]),
+    "pamd_trsv_pack_workspace": (c_int, [c_i64, ctypes.POINTER(c_i64)]),
+    "pamd_trsv_pack_f64": (c_int, [c_i64, c_vp, c_i64, c_vp, c_vp]),
+    "pamd_trsv_packed_f64": (c_int, [c_int, c_i64, c_vp, c_vp, c_vp]),
     "pamd_gaussian_fill_f64": (c_int, [c_i64, c_i64, c_dbl, c_u64, c_u64, c_vp, c_i64, c_vp]),
     "pamd_sjlt_draw": (c_int, [c_i64, c_i64, c_int, c_u64, c_vp, c_vp, c_vp]),
     "pamd_srct_fill_f64": (c_int, [c_i64, c_i64, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp]),

@@ -8,6 +8,7 @@
 // partials that a second kernel sums in slice order (deterministic).
 #include "common.h"
 #include "trsv_dev.h"
+#include "trsv_pack.h"
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
@@ -507,4 +508,34 @@ extern "C" int pamd_trsv_upper_f64(int trans, int64_t n, const double* R, int64_
   }
   PAMD_LAUNCH_CHECK();
   return PAMD_OK;
+}
+
+// The packed form (trsv_pack.h) for a triangle that is solved with more than
+// once, or once at n >= 192: one wide packing launch, then solves bound by the
+// chain through the diagonal.
+extern "C" int pamd_trsv_pack_workspace(int64_t n, int64_t* bytes) {
+  PAMD_ARG_CHECK(n >= 0 && n <= TP_MAX_N, 1);
+  PAMD_ARG_CHECK(bytes != nullptr, 2);
+  *bytes = 2 * tp_doubles(n) * (int64_t)sizeof(double);
+  return PAMD_OK;
+}
+
+extern "C" int pamd_trsv_pack_f64(int64_t n, const double* R, int64_t ldr, void* packed, void* stream) {
+  PAMD_ARG_CHECK(n >= 0 && n <= TP_MAX_N, 1);
+  PAMD_ARG_CHECK(R != nullptr || n == 0, 2);
+  PAMD_ARG_CHECK(ldr >= n && ldr >= 1, 3);
+  PAMD_ARG_CHECK(packed != nullptr || n == 0, 4);
+  if (n == 0) return PAMD_OK;
+  double* P = (double*)packed;
+  return tp_launch_pack((int)n, R, ldr, P, P + tp_doubles(n), (hipStream_t)stream);
+}
+
+extern "C" int pamd_trsv_packed_f64(int trans, int64_t n, const void* packed, double* x, void* stream) {
+  PAMD_ARG_CHECK(trans == 0 || trans == 1, 1);
+  PAMD_ARG_CHECK(n >= 0 && n <= TP_MAX_N, 2);
+  PAMD_ARG_CHECK(packed != nullptr || n == 0, 3);
+  PAMD_ARG_CHECK(x != nullptr || n == 0, 4);
+  if (n == 0) return PAMD_OK;
+  const double* P = (const double*)packed + (trans ? 0 : tp_doubles(n));
+  return tp_launch_solve(trans, (int)n, P, x, x, (hipStream_t)stream);
 }

@@ -2,9 +2,10 @@
 //
 // Operator: A_pc = [A; sd I] M with M = R^{-1} (sd = sqrt(delta)), or M = I.
 // M is applied by backward-stable substitution (R x = v, R^T x = y) inside the
-// tail kernel, in LDS -- an explicit inverse would be faster to apply but its
+// tail kernel -- an explicit inverse would be faster to apply but its
 // forward error grows like kappa(R) u and costs an order of magnitude in the
-// final backward error.  One LSQR iteration is two kernels:
+// final backward error.  One LSQR iteration is two or
+// three kernels:
 //
 //   lsqr_pass  (multi-workgroup, one read of A): for each row i
 //                u_i <- c1 * (A w)_i + c2 * u_i,   y_g += u_i * A[i, :]
@@ -12,7 +13,8 @@
 //              A_pc^T applied to the *normalised* new u; since
 //              A^T (u / beta) = (A^T u) / beta, both products come out of the
 //              same pass: one read of A per iteration instead of two.
-//   lsqr_tail  (one 1024-thread workgroup): sums the per-workgroup partials
+//   lsqr_reduce + lsqr_tailp (R given, n <= 1024), or lsqr_tail (otherwise; one
+//              1024-thread workgroup): sums the per-workgroup partials
 //              y_g in fixed order (plus the lifted rows sd * I), then beta,
 //              v <- R^{-T} y / beta - beta v, alpha, the Givens recurrences
 //              and stopping tests of PARLA's lsqr (comps/determiter/lsqr.py:
@@ -25,6 +27,7 @@
 // c2 = -alpha / beta.
 #include "common.h"
 #include "trsv_dev.h"
+#include "trsv_pack.h"
 
 namespace {
 
@@ -39,6 +42,7 @@ struct LsqrConst {
   int64_t m, n, lda, ldr, iter_lim;
   double sd, damp, atol, btol, ctol;
   int has_r, calc_var, has_x0, grid;
+  int packed;     // R is packed in the workspace (lsqr_packed)
   int xs_global;  // the substitution vector lives in the workspace (n too large for LDS)
 };
 
@@ -64,8 +68,13 @@ __host__ __device__ inline int lsqr_grid(int64_t m, int64_t n) {
   return (int)pamd_cdiv(lsqr_total_waves(m), lsqr_waves(m, n));
 }
 
+// The packed path (R given, n <= TP_MAX_N): R is packed once per solve
+// (trsv_pack.h), a reduction kernel sums the pass partials and
+// lsqr_tailp_kernel does the rest of the iteration.
+__host__ __device__ inline bool lsqr_packed(int64_t n) { return n <= TP_MAX_N; }
+
 struct LsqrLayout {
-  int64_t st, u, v, w, work, y, pv, pb, xs, dinv, total;
+  int64_t st, u, v, w, work, y, pv, pb, rs, xs, dinv, padj, pfwd, total;
 };
 
 __host__ __device__ inline LsqrLayout lsqr_layout(int64_t m, int64_t n) {
@@ -79,9 +88,12 @@ __host__ __device__ inline LsqrLayout lsqr_layout(int64_t m, int64_t n) {
   L.y = L.work + n;
   L.pv = (L.y + n + 31) / 32 * 32;
   L.pb = L.pv + (int64_t)G * n;
-  L.xs = (L.pb + (int64_t)G * 2 + 31) / 32 * 32;
+  L.rs = (L.pb + (int64_t)G * 2 + 31) / 32 * 32;  // (sum u'^2, sum u^2) of each reduction workgroup
+  L.xs = L.rs + 2 * TP_MAX_NB;
   L.dinv = (L.xs + (n > LSQR_LDS_MAX_N ? n : 0) + 31) / 32 * 32;  // inverses of R's 8 x 8 diagonal sub-blocks
-  L.total = L.dinv + pamd_cdiv(n, 8) * 64 + 32;
+  L.padj = L.dinv + pamd_cdiv(n, 8) * 64 + 32;                    // packed R^T and R solves
+  L.pfwd = L.padj + (lsqr_packed(n) ? tp_doubles(n) : 0);
+  L.total = L.pfwd + (lsqr_packed(n) ? tp_doubles(n) : 0);
   return L;
 }
 
@@ -360,36 +372,108 @@ __device__ inline void apply_forward(const LsqrConst& K, const double* __restric
   __syncthreads();
 }
 
-// state, x = x0 or 0, u = b (lifted part 0), work = M x0 with (c1, c2) =
-// (-1, 1), or work = 0 with (c1, c2) = (0, 1)
-__global__ __launch_bounds__(1024) void lsqr_init_kernel(LsqrConst K, const double* __restrict__ R,
-                                                         const double* __restrict__ b, const double* __restrict__ x0,
-                                                         double* __restrict__ x, double* __restrict__ var,
-                                                         double* __restrict__ ws) {
-  extern __shared__ double smem[];
+// The norm estimates, stopping tests and log entry of one iteration
+// (lsqr.py:412-526), by one thread; returns whether the iteration stops.
+__device__ inline bool lsqr_scalars(const LsqrConst& K, LsqrState* S, double* __restrict__ arnorms, double alfa,
+                                    double beta, double anorm, double rho, double rhobar, double phi, double phibar,
+                                    double psi, double tau, double theta, double ddsum) {
+  const double eps = 2.220446049250313e-16;
+  const int64_t itn_prev = S->itn;
+  arnorms[itn_prev] = S->arnorm;  // logged at the top of the iteration (lsqr.py:413)
+  const int64_t itn = itn_prev + 1;
+  const double ddnorm = S->ddnorm + ddsum;
+  const double delta = S->sn2 * rho;
+  const double gambar = -S->cs2 * rho;
+  const double rhs = phi - delta * S->z;
+  const double zbar = rhs / gambar;
+  const double xnorm = sqrt(S->xxnorm + zbar * zbar);
+  const double gamma = sqrt(gambar * gambar + theta * theta);
+  const double cs2 = gambar / gamma;
+  const double sn2 = theta / gamma;
+  const double z = rhs / gamma;
+  const double xxnorm = S->xxnorm + z * z;
+  const double acond = anorm * sqrt(ddnorm);
+  const double res1 = phibar * phibar;
+  const double res2 = S->res2 + psi * psi;
+  const double rnorm = sqrt(res1 + res2);
+  const double arnorm = alfa * fabs(tau);
+  const double r1sq = rnorm * rnorm - K.damp * K.damp * xxnorm;
+  double r1norm = sqrt(fabs(r1sq));
+  if (r1sq < 0) r1norm = -r1norm;
+  const double bnorm = S->bnorm;
+  const double test1 = rnorm / bnorm;
+  const double test2 = arnorm / (anorm * rnorm + eps);
+  const double test3 = 1.0 / (acond + eps);
+  const double tt1 = test1 / (1.0 + anorm * xnorm / bnorm);
+  const double rtol = K.btol + K.atol * anorm * xnorm / bnorm;
+  int64_t istop = 0;
+  if (itn >= K.iter_lim) istop = 7;
+  if (1.0 + test3 <= 1.0) istop = 6;
+  if (1.0 + test2 <= 1.0) istop = 5;
+  if (1.0 + tt1 <= 1.0) istop = 4;
+  if (test3 <= K.ctol) istop = 3;
+  if (test2 <= K.atol) istop = 2;
+  if (test1 <= rtol) istop = 1;
+  S->itn = itn;
+  S->istop = istop;
+  S->alfa = alfa;
+  S->beta = beta;
+  S->anorm = anorm;
+  S->acond = acond;
+  S->ddnorm = ddnorm;
+  S->res2 = res2;
+  S->xnorm = xnorm;
+  S->xxnorm = xxnorm;
+  S->z = z;
+  S->cs2 = cs2;
+  S->sn2 = sn2;
+  S->rhobar = rhobar;
+  S->phibar = phibar;
+  S->rnorm = rnorm;
+  S->r1norm = r1norm;
+  S->r2norm = rnorm;
+  S->arnorm = arnorm;
+  S->c1 = 1.0;
+  S->c2 = (beta > 0.0) ? -alfa * (1.0 / beta) : -alfa;
+  return istop != 0;
+}
+
+// state, x = x0 or 0, u = b (lifted part 0), work = 0; (c1, c2) = (0, 1), or
+// (-1, 1) with x0, when lsqr_init_work_kernel or the packed forward solve then
+// writes work = M x0.  A grid-stride copy: with one workgroup it took 119 us
+// at m = 131072.
+__global__ __launch_bounds__(256) void lsqr_init_kernel(LsqrConst K, const double* __restrict__ b,
+                                                        const double* __restrict__ x0, double* __restrict__ x,
+                                                        double* __restrict__ var, double* __restrict__ ws) {
   const LsqrLayout L = lsqr_layout(K.m, K.n);
-  LsqrState* S = reinterpret_cast<LsqrState*>(ws);
   double* u = ws + L.u;
-  for (int64_t i = threadIdx.x; i < K.m; i += blockDim.x) u[i] = b[i];
-  for (int64_t i = threadIdx.x; i < K.n; i += blockDim.x) {
+  const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = i0; i < K.m; i += step) u[i] = b[i];
+  for (int64_t i = i0; i < K.n; i += step) {
     u[K.m + i] = 0.0;
     x[i] = K.has_x0 ? x0[i] : 0.0;
     if (var) var[i] = 0.0;
+    ws[L.work + i] = 0.0;
   }
-  if (K.has_r) trsv_dinv8((int)K.n, R, K.ldr, ws + L.dinv);  // once per solve: R is fixed
-  __syncthreads();
-  if (K.has_x0) {
-    double* xs = K.xs_global ? ws + L.xs : smem;
-    apply_forward(K, R, x, ws + L.work, xs, K.xs_global ? smem : smem + K.n, ws + L.dinv);
-  } else {
-    for (int64_t i = threadIdx.x; i < K.n; i += blockDim.x) ws[L.work + i] = 0.0;
-  }
-  if (threadIdx.x == 0) {
+  if (i0 == 0) {
     LsqrState s = {};
     s.cs2 = -1.0;
     s.c1 = K.has_x0 ? -1.0 : 0.0;
     s.c2 = 1.0;
-    *S = s;
+    *reinterpret_cast<LsqrState*>(ws) = s;
+  }
+}
+
+// the unpacked path: R's 8 x 8 diagonal inverses (once per solve: R is fixed) and work = M x0
+__global__ __launch_bounds__(1024) void lsqr_init_work_kernel(LsqrConst K, const double* __restrict__ R,
+                                                              const double* __restrict__ x, double* __restrict__ ws) {
+  extern __shared__ double smem[];
+  const LsqrLayout L = lsqr_layout(K.m, K.n);
+  if (K.has_r) trsv_dinv8((int)K.n, R, K.ldr, ws + L.dinv);
+  __syncthreads();
+  if (K.has_x0) {
+    double* xs = K.xs_global ? ws + L.xs : smem;
+    apply_forward(K, R, x, ws + L.work, xs, K.xs_global ? smem : smem + K.n, ws + L.dinv);
   }
 }
 
@@ -408,7 +492,6 @@ __global__ __launch_bounds__(1024) void lsqr_tail_kernel(LsqrConst K, const doub
   double* v = ws + L.v;
   double* w = ws + L.w;
   const int64_t n = K.n;
-  const double eps = 2.220446049250313e-16;
 
   double ssq_new, ssq_in;
   gather_partials(K, ws, L, S, red, cred, ssq_new, ssq_in);
@@ -493,66 +576,9 @@ __global__ __launch_bounds__(1024) void lsqr_tail_kernel(LsqrConst K, const doub
     w[i] = v[i] + t2 * wi;
   }
   const double ddsum = block_sum(dd, red);
-  if (threadIdx.x == 0) {
-    const int64_t itn_prev = S->itn;
-    arnorms[itn_prev] = S->arnorm;  // logged at the top of the iteration (lsqr.py:413)
-    const int64_t itn = itn_prev + 1;
-    const double ddnorm = S->ddnorm + ddsum;
-    const double delta = S->sn2 * rho;
-    const double gambar = -S->cs2 * rho;
-    const double rhs = phi - delta * S->z;
-    const double zbar = rhs / gambar;
-    const double xnorm = sqrt(S->xxnorm + zbar * zbar);
-    const double gamma = sqrt(gambar * gambar + theta * theta);
-    const double cs2 = gambar / gamma;
-    const double sn2 = theta / gamma;
-    const double z = rhs / gamma;
-    const double xxnorm = S->xxnorm + z * z;
-    const double acond = anorm * sqrt(ddnorm);
-    const double res1 = phibar * phibar;
-    const double res2 = S->res2 + psi * psi;
-    const double rnorm = sqrt(res1 + res2);
-    const double arnorm = alfa * fabs(tau);
-    const double r1sq = rnorm * rnorm - damp * damp * xxnorm;
-    double r1norm = sqrt(fabs(r1sq));
-    if (r1sq < 0) r1norm = -r1norm;
-    const double bnorm = S->bnorm;
-    const double test1 = rnorm / bnorm;
-    const double test2 = arnorm / (anorm * rnorm + eps);
-    const double test3 = 1.0 / (acond + eps);
-    const double tt1 = test1 / (1.0 + anorm * xnorm / bnorm);
-    const double rtol = K.btol + K.atol * anorm * xnorm / bnorm;
-    int64_t istop = 0;
-    if (itn >= K.iter_lim) istop = 7;
-    if (1.0 + test3 <= 1.0) istop = 6;
-    if (1.0 + test2 <= 1.0) istop = 5;
-    if (1.0 + tt1 <= 1.0) istop = 4;
-    if (test3 <= K.ctol) istop = 3;
-    if (test2 <= K.atol) istop = 2;
-    if (test1 <= rtol) istop = 1;
-    S->itn = itn;
-    S->istop = istop;
-    S->alfa = alfa;
-    S->beta = beta;
-    S->anorm = anorm;
-    S->acond = acond;
-    S->ddnorm = ddnorm;
-    S->res2 = res2;
-    S->xnorm = xnorm;
-    S->xxnorm = xxnorm;
-    S->z = z;
-    S->cs2 = cs2;
-    S->sn2 = sn2;
-    S->rhobar = rhobar;
-    S->phibar = phibar;
-    S->rnorm = rnorm;
-    S->r1norm = r1norm;
-    S->r2norm = rnorm;
-    S->arnorm = arnorm;
-    S->c1 = 1.0;
-    S->c2 = (beta > 0.0) ? -alfa * (1.0 / beta) : -alfa;
-    bc[0] = (istop != 0) ? 1.0 : 0.0;
-  }
+  if (threadIdx.x == 0)
+    bc[0] = lsqr_scalars(K, S, arnorms, alfa, beta, anorm, rho, rhobar, phi, phibar, psi, tau, theta, ddsum) ? 1.0
+                                                                                                             : 0.0;
   __syncthreads();
   if (bc[0] == 0.0) apply_forward(K, R, v, ws + L.work, xs, scratch, ws + L.dinv);
   if (threadIdx.x == 0 && bc[0] != 0.0) S->done = 1;
@@ -566,6 +592,281 @@ __global__ __launch_bounds__(1024) void lsqr_xorig_kernel(LsqrConst K, const dou
   const LsqrLayout L = lsqr_layout(K.m, K.n);
   double* xs = K.xs_global ? ws + L.xs : smem;
   apply_forward(K, R, x, xo, xs, K.xs_global ? smem : smem + K.n, ws + L.dinv);
+}
+
+// ---------------------------------------------------------------------------
+// packed path
+// ---------------------------------------------------------------------------
+
+// y = sum of the pass partials (+ lifted rows) for 64 columns per workgroup,
+// and this workgroup's share of the ssq totals.  Sixteen wavefronts sum the
+// partials g = s, s + 16, ... with sixteen loads in flight each, then the
+// sixteen sums are added in order.  One workgroup reads its 64 columns of all
+// partials at one CU's rate, so spreading the columns over ceil(n / 64) CUs
+// beats gathering in the tail's one (12.3 us for 313 partials of 200 columns)
+// once there are more partials than LSQR_TAIL_GATHER.
+__global__ __launch_bounds__(1024) void lsqr_reduce_kernel(LsqrConst K, double* __restrict__ ws) {
+  constexpr int GL = 16;
+  __shared__ double cred[16][64];
+  __shared__ double red[16];
+  const LsqrState* S = reinterpret_cast<const LsqrState*>(ws);
+  if (S->done) return;
+  const LsqrLayout L = lsqr_layout(K.m, K.n);
+  const int64_t n = K.n;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t c = (int64_t)blockIdx.x * 64 + lane;
+  const double* __restrict__ pv = ws + L.pv;
+  const int ng = K.grid;
+  double a = 0.0, b = 0.0;
+  if (blockIdx.x == 0)
+    for (int g = threadIdx.x; g < ng; g += 1024) {
+      a += ws[L.pb + 2 * g];
+      b += ws[L.pb + 2 * g + 1];
+    }
+  double t = 0.0;
+  if (c < n)
+    for (int g = wave; g < ng; g += 16 * GL) {
+      double pg[GL];
+#pragma unroll
+      for (int q = 0; q < GL; ++q) pg[q] = (g + 16 * q < ng) ? pv[(int64_t)(g + 16 * q) * n + c] : 0.0;
+#pragma unroll
+      for (int q = 0; q < GL; ++q) t += pg[q];
+    }
+  cred[wave][lane] = t;
+  __syncthreads();
+  if (wave == 0 && c < n) {
+    double tot = 0.0;
+#pragma unroll
+    for (int s = 0; s < 16; ++s) tot += cred[s][lane];
+    if (K.sd > 0.0) {
+      double* ul = ws + L.u + K.m;
+      const double uin = ul[c];
+      const double un = S->c1 * (K.sd * ws[L.work + c]) + S->c2 * uin;
+      ul[c] = un;
+      tot += K.sd * un;
+      a += un * un;
+      b += uin * uin;
+    }
+    ws[L.y + c] = tot;
+  }
+  a = block_sum(a, red);
+  b = block_sum(b, red);
+  if (threadIdx.x == 0) {
+    ws[L.rs + 2 * blockIdx.x] = a;
+    ws[L.rs + 2 * blockIdx.x + 1] = b;
+  }
+}
+
+// partials the tail sums itself: at most as many as one lane keeps in flight
+// in two rounds, where a reduction launch of its own costs more
+constexpr int LSQR_TAIL_GATHER = 32;
+
+// The rest of the iteration for the packed path: v <- R^{-T} y / beta - beta v,
+// alpha, the recurrences and stopping tests, the x / w updates, work = R^{-1} v
+// (phase 0: the set-up).  One workgroup, bound by the latency of the two
+// triangular solves (trsv_pack.h); everything else is arranged off that chain:
+// the forward solve runs on the unscaled v and is divided by alpha afterwards,
+// the two norms share the barrier that hands v over, and the scalar
+// recurrences run on the wavefront that leaves the forward solve first.
+// KR block rows per wavefront (n <= 512 KR).  Per iteration, with the
+// reduction: 58 -> 18 + 6 us at n = 200, 155 -> 55 + 6 at n = 512 (m = 131072).
+template <int KR>
+__global__ __launch_bounds__(TP_THREADS) void lsqr_tailp_kernel(LsqrConst K, double* __restrict__ x,
+                                                                double* __restrict__ var,
+                                                                double* __restrict__ arnorms,
+                                                                double* __restrict__ ws) {
+  LsqrState* S = reinterpret_cast<LsqrState*>(ws);
+  if (S->done) return;
+  __shared__ double xs[64 * TP_WAVES * KR];
+  __shared__ double vs[64 * TP_WAVES * KR];
+  __shared__ double part[TP_WAVES][2], part2[TP_WAVES][2];
+  __shared__ int ready[2];
+  const LsqrLayout L = lsqr_layout(K.m, K.n);
+  const int n = (int)K.n, nb = tp_nb(n), N = 64 * nb;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const TpBuf Padj = tp_buf(ws + L.padj, nb, lane), Pfwd = tp_buf(ws + L.pfwd, nb, lane);
+  double buf[64];
+  tp_prefetch(buf, Padj, nb, wave);
+  double acc[KR], vin[KR], win[KR], xin[KR];
+  const bool inline_gather = K.grid <= LSQR_TAIL_GATHER;
+  double a = 0.0, b = 0.0;
+  if (inline_gather && wave == 0 && lane < K.grid) {
+    a = ws[L.pb + 2 * lane];
+    b = ws[L.pb + 2 * lane + 1];
+  }
+#pragma unroll
+  for (int k = 0; k < KR; ++k) {
+    const int i = 64 * (wave + TP_WAVES * k) + lane;
+    acc[k] = vin[k] = win[k] = xin[k] = 0.0;
+    if (i < n) {
+      if (inline_gather) {
+        double t = 0.0;
+        for (int g = 0; g < K.grid; g += 16) {
+          double pg[16];
+#pragma unroll
+          for (int q = 0; q < 16; ++q) pg[q] = (g + q < K.grid) ? ws[L.pv + (int64_t)(g + q) * n + i] : 0.0;
+#pragma unroll
+          for (int q = 0; q < 16; ++q) t += pg[q];
+        }
+        if (K.sd > 0.0) {
+          double* ul = ws + L.u + K.m;
+          const double uin = ul[i];
+          const double un = S->c1 * (K.sd * ws[L.work + i]) + S->c2 * uin;
+          ul[i] = un;
+          t += K.sd * un;
+          a += un * un;
+          b += uin * uin;
+        }
+        acc[k] = t;
+      } else {
+        acc[k] = ws[L.y + i];
+      }
+      vin[k] = ws[L.v + i];
+      win[k] = ws[L.w + i];
+      xin[k] = x[i];
+    }
+  }
+  if (inline_gather) {
+    a = wave_sum(a);
+    b = wave_sum(b);
+  }
+  if (lane == 0) {
+    part[wave][0] = a;
+    part[wave][1] = b;
+  }
+  if (threadIdx.x < 2) ready[threadIdx.x] = 0;
+  // every read of the state comes before the second barrier, every write after it
+  const int64_t phase = S->phase;
+  const double alfa0 = S->alfa, anorm0 = S->anorm, rhobar0 = S->rhobar, phibar0 = S->phibar;
+  __syncthreads();
+  double ssq_new = 0.0, ssq_in = 0.0;
+  if (inline_gather) {
+#pragma unroll
+    for (int w = 0; w < TP_WAVES; ++w) {
+      ssq_new += part[w][0];
+      ssq_in += part[w][1];
+    }
+  } else {
+    for (int g = 0; g < nb; ++g) {
+      ssq_new += ws[L.rs + 2 * g];
+      ssq_in += ws[L.rs + 2 * g + 1];
+    }
+  }
+  const double beta = sqrt(ssq_new);
+  const double inv = 1.0 / beta;  // used where beta > 0
+
+  tp_solve<KR>(nb, Padj, buf, acc, xs, &ready[0], wave, lane);
+  tp_prefetch(buf, Pfwd, nb, wave);
+
+  // t: v before its division by alpha; phase 0 with b = 0 takes v = x
+  double t[KR];
+  double ss = 0.0, ww = 0.0;
+#pragma unroll
+  for (int k = 0; k < KR; ++k) {
+    const int i = 64 * (wave + TP_WAVES * k) + lane;
+    t[k] = 0.0;
+    if (i < n) {
+      if (beta > 0.0)
+        t[k] = phase == 0 ? acc[k] * inv : acc[k] * inv - beta * vin[k];
+      else
+        t[k] = phase == 0 ? xin[k] : vin[k];
+    }
+    ss += t[k] * t[k];
+    ww += win[k] * win[k];
+    if (i < N) vs[i] = t[k];
+  }
+  ss = wave_sum(ss);
+  ww = wave_sum(ww);
+  if (lane == 0) {
+    part2[wave][0] = ss;
+    part2[wave][1] = ww;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < KR; ++k) {
+    const int i = 64 * (wave + TP_WAVES * k) + lane;
+    acc[k] = i < N ? vs[N - 1 - i] : 0.0;
+  }
+  tp_solve<KR>(nb, Pfwd, buf, acc, xs, &ready[1], wave, lane);
+
+  ss = 0.0;
+  ww = 0.0;
+#pragma unroll
+  for (int w = 0; w < TP_WAVES; ++w) {
+    ss += part2[w][0];
+    ww += part2[w][1];
+  }
+  double alfa = beta > 0.0 ? sqrt(ss) : (phase == 0 ? 0.0 : alfa0);
+  const double ia = (beta > 0.0 && alfa > 0.0) ? 1.0 / alfa : 1.0;
+#pragma unroll
+  for (int k = 0; k < KR; ++k) {
+    const int i = 64 * (wave + TP_WAVES * k) + lane;
+    if (i < N && N - 1 - i < n) ws[L.work + N - 1 - i] = ia * acc[k];
+  }
+
+  if (phase == 0) {
+#pragma unroll
+    for (int k = 0; k < KR; ++k) {
+      const int i = 64 * (wave + TP_WAVES * k) + lane;
+      if (i < n) {
+        ws[L.v + i] = ia * t[k];
+        ws[L.w + i] = ia * t[k];
+      }
+    }
+    if (threadIdx.x == 0) {
+      const double arnorm = alfa * beta;
+      S->bnorm = sqrt(ssq_in);
+      S->beta = beta;
+      S->alfa = alfa;
+      S->rhobar = alfa;
+      S->phibar = beta;
+      S->rnorm = S->r1norm = S->r2norm = beta;
+      S->arnorm = arnorm;
+      S->istop = 0;
+      S->itn = 0;
+      S->early = (arnorm == 0.0) ? 1 : 0;
+      S->c1 = 1.0;
+      S->c2 = -alfa * (1.0 / beta);
+      S->phase = 1;
+      S->done = ((arnorm == 0.0) || (K.iter_lim <= 0)) ? 1 : 0;
+    }
+    return;
+  }
+
+  double anorm = anorm0;
+  if (beta > 0.0) anorm = sqrt(anorm * anorm + alfa0 * alfa0 + beta * beta + K.damp * K.damp);
+  // scalar rotations (identical on every thread)
+  const double rhobar1 = sqrt(rhobar0 * rhobar0 + K.damp * K.damp);
+  const double cs1 = rhobar0 / rhobar1;
+  const double sn1 = K.damp / rhobar1;
+  const double psi = sn1 * phibar0;
+  double phibar = cs1 * phibar0;
+  double cs, sn, rho;
+  sym_ortho(rhobar1, beta, cs, sn, rho);
+  const double theta = sn * alfa;
+  const double rhobar = -cs * alfa;
+  const double phi = cs * phibar;
+  phibar = sn * phibar;
+  const double tau = sn * phi;
+  const double t1 = phi / rho;
+  const double t2 = -theta / rho;
+  const double irho = 1.0 / rho;
+#pragma unroll
+  for (int k = 0; k < KR; ++k) {
+    const int i = 64 * (wave + TP_WAVES * k) + lane;
+    if (i < n) {
+      const double vn = ia * t[k], wi = win[k];
+      const double dk = irho * wi;
+      if (K.calc_var) var[i] += dk * dk;
+      x[i] = xin[k] + t1 * wi;
+      ws[L.v + i] = vn;
+      ws[L.w + i] = vn + t2 * wi;
+    }
+  }
+  if (threadIdx.x == 0 &&
+      lsqr_scalars(K, S, arnorms, alfa, beta, anorm, rho, rhobar, phi, phibar, psi, tau, theta, irho * irho * ww))
+    S->done = 1;
 }
 
 int launch_pass(const LsqrConst& K, const double* A, double* ws, hipStream_t st) {
@@ -585,6 +886,34 @@ int launch_pass(const LsqrConst& K, const double* A, double* ws, hipStream_t st)
   else
     PAMD_PASS(0, 4);
 #undef PAMD_PASS
+  PAMD_LAUNCH_CHECK();
+  return PAMD_OK;
+}
+
+// one tail (the packed path: the reduction of the partials before it)
+int launch_tail(const LsqrConst& K, const double* R, double* x, double* var, double* arnorms, double* ws,
+                size_t shmem, hipStream_t st) {
+  if (!K.packed) {
+    lsqr_tail_kernel<<<1, 1024, shmem, st>>>(K, R, x, var, arnorms, ws);
+  } else {
+    if (K.grid > LSQR_TAIL_GATHER) {
+      lsqr_reduce_kernel<<<(unsigned)tp_nb(K.n), 1024, 0, st>>>(K, ws);
+      PAMD_LAUNCH_CHECK();
+    }
+    if (K.n <= 64 * TP_WAVES)
+      lsqr_tailp_kernel<1><<<1, TP_THREADS, 0, st>>>(K, x, var, arnorms, ws);
+    else
+      lsqr_tailp_kernel<2><<<1, TP_THREADS, 0, st>>>(K, x, var, arnorms, ws);
+  }
+  PAMD_LAUNCH_CHECK();
+  return PAMD_OK;
+}
+
+// x_orig = R^{-1} x
+int launch_xorig(const LsqrConst& K, const double* R, const double* x, double* xo, double* ws, size_t shmem,
+                 hipStream_t st) {
+  if (K.packed) return tp_launch_solve(0, (int)K.n, ws + lsqr_layout(K.m, K.n).pfwd, x, xo, st);
+  lsqr_xorig_kernel<<<1, 1024, shmem, st>>>(K, R, x, xo, ws);
   PAMD_LAUNCH_CHECK();
   return PAMD_OK;
 }
@@ -634,16 +963,28 @@ int lsqr_start(const pamd_lsqr_problem* prob, double* x, double* var, double* ar
   K.has_x0 = P.x0 != nullptr;
   K.grid = lsqr_grid(P.m, P.n);
   K.ldr = P.ldr;
+  K.packed = K.has_r && lsqr_packed(P.n);
   K.xs_global = (K.has_r && P.n > LSQR_LDS_MAX_N) ? 1 : 0;
   double* ws = (double*)workspace;
   shmem = (size_t)(K.has_r ? ((K.xs_global ? 0 : P.n) + TRSV_SCRATCH_DOUBLES) : 1) * sizeof(double);
-  lsqr_init_kernel<<<1, 1024, shmem, st>>>(K, P.R, P.b, P.x0, x, var, ws);
+  const unsigned ig = (unsigned)imax64(1, imin64(256, pamd_cdiv(imax64(P.m, P.n), 1024)));
+  lsqr_init_kernel<<<ig, 256, 0, st>>>(K, P.b, P.x0, x, var, ws);
   PAMD_LAUNCH_CHECK();
+  if (K.packed) {
+    const LsqrLayout L = lsqr_layout(K.m, K.n);
+    int rc = tp_launch_pack((int)P.n, P.R, P.ldr, ws + L.padj, ws + L.pfwd, st);
+    if (rc) return rc;
+    if (K.has_x0) {
+      rc = tp_launch_solve(0, (int)K.n, ws + L.pfwd, P.x0, ws + L.work, st);
+      if (rc) return rc;
+    }
+  } else if (K.has_r || K.has_x0) {
+    lsqr_init_work_kernel<<<1, 1024, shmem, st>>>(K, P.R, x, ws);
+    PAMD_LAUNCH_CHECK();
+  }
   int rc = launch_pass(K, P.A, ws, st);
   if (rc) return rc;
-  lsqr_tail_kernel<<<1, 1024, shmem, st>>>(K, P.R, x, var, arnorms, ws);  // phase 0: set-up
-  PAMD_LAUNCH_CHECK();
-  return PAMD_OK;
+  return launch_tail(K, P.R, x, var, arnorms, ws, shmem, st);  // phase 0: set-up
 }
 
 // the result fields from the device state (one thread)
@@ -684,15 +1025,15 @@ extern "C" int pamd_lsqr_run_f64(const pamd_lsqr_problem* prob, double* x, doubl
     for (int64_t it = 0; it < todo; ++it) {
       rc = launch_pass(K, P.A, ws, st);
       if (rc) return rc;
-      lsqr_tail_kernel<<<1, 1024, shmem, st>>>(K, P.R, x, var, arnorms, ws);
-      PAMD_LAUNCH_CHECK();
+      rc = launch_tail(K, P.R, x, var, arnorms, ws, shmem, st);
+      if (rc) return rc;
     }
     launched += todo;
     batch = imin64(batch * 2, 64);
   }
   if (x_orig) {
-    lsqr_xorig_kernel<<<1, 1024, shmem, st>>>(K, P.R, x, x_orig, ws);
-    PAMD_LAUNCH_CHECK();
+    rc = launch_xorig(K, P.R, x, x_orig, ws, shmem, st);
+    if (rc) return rc;
   }
   result->istop = hs.istop;
   result->itn = hs.itn;
@@ -719,12 +1060,12 @@ extern "C" int pamd_lsqr_launch_f64(const pamd_lsqr_problem* prob, double* x, do
   for (int64_t it = 0; it < P.iter_lim; ++it) {
     rc = launch_pass(K, P.A, ws, st);
     if (rc) return rc;
-    lsqr_tail_kernel<<<1, 1024, shmem, st>>>(K, P.R, x, var, arnorms, ws);
-    PAMD_LAUNCH_CHECK();
+    rc = launch_tail(K, P.R, x, var, arnorms, ws, shmem, st);
+    if (rc) return rc;
   }
   if (x_orig) {
-    lsqr_xorig_kernel<<<1, 1024, shmem, st>>>(K, P.R, x, x_orig, ws);
-    PAMD_LAUNCH_CHECK();
+    rc = launch_xorig(K, P.R, x, x_orig, ws, shmem, st);
+    if (rc) return rc;
   }
   lsqr_result_kernel<<<1, 64, 0, st>>>(ws, result);
   PAMD_LAUNCH_CHECK();

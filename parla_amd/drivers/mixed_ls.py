@@ -133,7 +133,8 @@ class SPOMixed(OverLstsqSolver):
         log.time_factor = clock() - tic
 
         tic = clock()
-        x = ops.trsv_(R, z)
+        tri = ops.TriSolver(R)
+        x = tri.solve_(z)
         res = ops.Residual(At)
         normal = ops.NormalOp(B32)
         anorm_d = ops.nrm2(At.reshape(-1))  # read with the first step's norms
@@ -160,13 +161,13 @@ class SPOMixed(OverLstsqSolver):
             # then at the FP64 floor of this problem's backward error
             if eta <= tol or (step > 0 and eta > 0.5 * etas[-2]) or step == self.max_refine:
                 break
-            rhs = ops.trsv_(R, g, trans=True)
+            rhs = tri.solve_(g, trans=True)
             # the inner solve only has to take eta down to tol (or to the FP64
             # floor): ask CG for a tenth of that ratio, between inner_tol and 0.1
             inner = min(0.1, max(self.inner_tol, 0.1 * tol / eta)) if eta > 0 else self.inner_tol
             dz, its = cg_normal(normal, rhs, self.max_inner, inner)
             inner_total += its
-            x.add_(ops.trsv_(R, dz))
+            x.add_(tri.solve_(dz))
         x = best_x
         if best_eta > tol:
             warnings.warn(f"SPOMixed: backward error {best_eta:.3e} stays above tol {tol:.1e} "
