@@ -311,6 +311,21 @@ int pamd_small_combine_f64(int64_t k, const double* A, int64_t lda, const double
 int pamd_cholqr_stats_f64(int64_t k, const double* G, int64_t ldg, const int* info,
                           const double* enorm, double* out, void* stream);
 
+/* R (n x n, upper with zeros below, positive diagonal) and z = Q^T S b of a
+ * sketch M = [S A | S b] (d x (n + 1), n <= 1024, not modified) by CholeskyQR2
+ * of S A, or with shifted = 1 by the shifted CholeskyQR3 (for an S A too ill
+ * conditioned for the former).  newton = 1 takes the second round's factor of
+ * I + E from two fixed-point steps (error of order ||E||^3), newton = 0 from a
+ * second Cholesky factorisation.  stats (4 doubles on the device): min and max
+ * |diag R1|, ||Q1^T Q1 - I||_F and the first failing pivot or 0; the result
+ * stands if the last is 0 and the norm is at most 1e-2 (newton = 1) or 0.25;
+ * otherwise R and z are not meaningful.  Launches only.
+ * Replaces la.qr and Q.T @ b_ske at drivers/least_squares.py:311,315. */
+int pamd_sketch_rz_workspace(int64_t d, int64_t n, int64_t* bytes);
+int pamd_sketch_rz_f64(int64_t d, int64_t n, const double* M, int64_t ldm,
+                       int shifted, int newton, double* R, int64_t ldr,
+                       double* z, double* stats, void* workspace, void* stream);
+
 /* Rinv (n x n, zeros below the diagonal) = R^{-1} for upper-triangular R
  * (n <= 2048); one triangular solve per column, all columns in parallel. */
 int pamd_trtri_upper_f64(int64_t n, const double* R, int64_t ldr, double* Rinv,

@@ -305,16 +305,7 @@ class SPOLearned:
         it = idx if isinstance(idx, torch.Tensor) else torch.from_numpy(idx).to(dev)
         st = scale if isinstance(scale, torch.Tensor) else torch.from_numpy(scale).to(dev)
         row_gather(bt.reshape(-1, 1), it, st, Mx[:, n:])
-        # R and Q^T S b of the sample: CholeskyQR2 when the sample is well enough
-        # conditioned for it (the learned or row-norm probabilities keep it
-        # near kappa(A)), else Householder
-        rz = ops.sketch_rz_cholqr2(Mx, n)
-        if rz is not None:
-            R, z = rz
-        else:
-            fac = ops.qr_r_(Mx, n)
-            R = torch.triu(fac.R_view).contiguous()
-            z = Mx[:n, n].clone()
+        R, z = ops.sketch_rz_(Mx, n)
         return R, z, kappa_estimate(At, R, self.lanczos_steps)
 
     def __call__(self, A, b, delta, tol, iter_lim, rng, logging=True, probs=None):

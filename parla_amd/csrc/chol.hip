@@ -301,24 +301,20 @@ __global__ __launch_bounds__(256) void cholqr_stats_kernel(int k, const double* 
 
 }  // namespace
 
-extern "C" int pamd_potrf_upper_f64(int64_t n, double* A, int64_t lda, int* info, void* stream) {
-  PAMD_ARG_CHECK(n >= 0 && n <= POTRF_MAX_N, 1);
-  PAMD_ARG_CHECK(A != nullptr || n == 0, 2);
-  PAMD_ARG_CHECK(lda >= n && lda >= 1, 3);
-  PAMD_ARG_CHECK(info != nullptr, 4);
+int pamd_potrf_run(int n, double* A, int64_t lda, int* info, void* stream) {
   hipStream_t st = (hipStream_t)stream;
   if (n == 0) {
     potrf_zero_info_kernel<<<1, 1, 0, st>>>(info);
     PAMD_LAUNCH_CHECK();
     return PAMD_OK;
   }
-  for (int j0 = 0; pr_width((int)n, j0) > 0; j0 += PR_LEAD) {
-    if (pr_small(pr_width((int)n, j0)))
-      potrf_reg_kernel<PR_SMALL><<<1, PR_THREADS, 0, st>>>((int)n, j0, A, lda, info);
+  for (int j0 = 0; pr_width(n, j0) > 0; j0 += PR_LEAD) {
+    if (pr_small(pr_width(n, j0)))
+      potrf_reg_kernel<PR_SMALL><<<1, PR_THREADS, 0, st>>>(n, j0, A, lda, info);
     else
-      potrf_reg_kernel<PR_LARGE><<<1, PR_THREADS, 0, st>>>((int)n, j0, A, lda, info);
+      potrf_reg_kernel<PR_LARGE><<<1, PR_THREADS, 0, st>>>(n, j0, A, lda, info);
     PAMD_LAUNCH_CHECK();
-    const int r = (int)n - j0;
+    const int r = n - j0;
     if (r <= PR_MAXN) break;
     double* Aj = A + j0 * (lda + 1);
     const int T = pr_trailing(r);
@@ -328,6 +324,14 @@ extern "C" int pamd_potrf_upper_f64(int64_t n, double* A, int64_t lda, int* info
     PAMD_LAUNCH_CHECK();
   }
   return PAMD_OK;
+}
+
+extern "C" int pamd_potrf_upper_f64(int64_t n, double* A, int64_t lda, int* info, void* stream) {
+  PAMD_ARG_CHECK(n >= 0 && n <= POTRF_MAX_N, 1);
+  PAMD_ARG_CHECK(A != nullptr || n == 0, 2);
+  PAMD_ARG_CHECK(lda >= n && lda >= 1, 3);
+  PAMD_ARG_CHECK(info != nullptr, 4);
+  return pamd_potrf_run((int)n, A, lda, info, stream);
 }
 
 #define PAMD_TRSM_MAX_N 2048
@@ -407,6 +411,16 @@ extern "C" int pamd_trtri_batched_f64(int64_t nprob, int64_t nmax, const int64_t
 
 #define PAMD_TRSM_MFMA_MAX_K 512
 
+int pamd_trsm_strip_run(int64_t m, int k, const double* R, int64_t ldr, const double* Y, int64_t ldy, double* X,
+                        int64_t ldx, double* dinv, void* stream) {
+  hipStream_t st = (hipStream_t)stream;
+  trsm_dinv_kernel<<<(unsigned)pamd_cdiv(k, TS_B), 64, 0, st>>>(k, R, ldr, dinv);
+  PAMD_LAUNCH_CHECK();
+  trsm_strip_kernel<<<(unsigned)pamd_cdiv(m, TS_B), 256, trsm_strip_lds(k), st>>>(m, k, Y, ldy, R, ldr, dinv, X, ldx);
+  PAMD_LAUNCH_CHECK();
+  return PAMD_OK;
+}
+
 extern "C" int pamd_trsm_mfma_workspace(int64_t k, int64_t* bytes) {
   PAMD_ARG_CHECK(k >= 0 && k <= PAMD_TRSM_MFMA_MAX_K, 1);
   PAMD_ARG_CHECK(bytes != nullptr, 2);
@@ -426,14 +440,7 @@ extern "C" int pamd_trsm_right_upper_mfma_f64(int64_t m, int64_t k, const double
   PAMD_ARG_CHECK(ldx >= k && ldx >= 1, 8);
   PAMD_ARG_CHECK(workspace != nullptr || k == 0, 9);
   if (m == 0 || k == 0) return PAMD_OK;
-  hipStream_t st = (hipStream_t)stream;
-  const int nb = (int)pamd_cdiv(k, TS_B);
-  trsm_dinv_kernel<<<nb, 64, 0, st>>>((int)k, R, ldr, (double*)workspace);
-  PAMD_LAUNCH_CHECK();
-  trsm_strip_kernel<<<(unsigned)pamd_cdiv(m, TS_B), 256, trsm_strip_lds((int)k), st>>>(m, (int)k, Y, ldy, R, ldr,
-                                                                     (const double*)workspace, X, ldx);
-  PAMD_LAUNCH_CHECK();
-  return PAMD_OK;
+  return pamd_trsm_strip_run(m, (int)k, R, ldr, Y, ldy, X, ldx, (double*)workspace, stream);
 }
 
 extern "C" int pamd_small_combine_f64(int64_t k, const double* A, int64_t lda, const double* B, int64_t ldb,

@@ -6,8 +6,9 @@ SPO (qr mode) on the device:
   1. S = sketch_op_gen(d, m, rng); [S A | S b] is formed in one buffer
      (dense Gaussian: MFMA GEMM; SJLT: gather kernel).  With delta > 0 the
      buffer gets the rows [sqrt(delta) I | 0] (least_squares.py:309-310).
-  2. Householder QR of the first n columns; the same reflectors turn the
-     last column into z = Q^T [S b; 0] = Q[:d].T @ S b (least_squares.py:311-315).
+  2. R of the first n columns and z = Q^T [S b; 0] = Q[:d].T @ S b from the
+     last one (least_squares.py:311-315): CholeskyQR2, its shifted form for an
+     ill-conditioned sketch, Householder QR otherwise (ops.sketch_rz_).
   3. x_ske = R^{-1} z and the presolve test ||A x_ske - b|| / ||b|| < 1
      (least_squares.py:316, 343-351) -- the one host synchronisation.
   4. PcSS2 -> device LSQR on [A; sqrt(delta) I] R^{-1} from z (or from 0).
@@ -160,7 +161,7 @@ def _sketch_into(S, X, out):
 class SPO(OverLstsqSolver):
     """Sketch-and-precondition for overdetermined least squares (least_squares.py:206-369).
 
-    mode 'qr' (Householder QR of the sketch, least_squares.py:306-316),
+    mode 'qr' (R of the sketch's QR, least_squares.py:306-316),
     'chol' (Cholesky of the sketched Gram matrix plus delta I, :317-329) or
     'svd' (the SVD right preconditioner M = V / sigma over the numerical rank,
     :330-339; rank-deficient A is handled as in the reference)."""
@@ -204,13 +205,9 @@ class SPO(OverLstsqSolver):
                 Mx[d:, :n_cols].diagonal().fill_(sqrt_delta)
             _sketch_into(S, bt, b_ske)
             Mx[:d, n_cols].copy_(b_ske)
-            fac = ops.qr_r_(Mx, n_cols)
-            # only the upper triangle of this view is R (scratch sits below); every
-            # consumer (triangular solves, LSQR) reads the upper triangle only
-            R = fac.R_view
+            R, z_ske = ops.sketch_rz_(Mx, n_cols)
             log.time_factor = clock() - tic
             tic = clock()
-            z_ske = Mx[:n_cols, n_cols].clone()
             x_ske = ops.trsv_(R, z_ske.clone())
         elif self.mode == 'chol':
             A_ske = Mx[:d, :n_cols]

@@ -478,50 +478,65 @@ def cholqr2(Y, rounds=2):
 
 
 SKETCH_NEWTON_MAX_E = 1e-2  # sketch_rz_cholqr2: second round by Newton while ||Q1^T Q1 - I||_F is below this
+SKETCH_MAX_E = 0.25         # ... and by potrf below this; beyond, the Gram matrix has lost the sketch's small directions
 
 
-def sketch_rz_cholqr2(M, n):
+def _sketch_rz(M, n, shifted, newton):
+    """One pamd_sketch_rz_f64: (R, z, ||Q1^T Q1 - I||_F), or None when a pivot
+    failed or the norm says that the first round was not good enough (the
+    call's one host read).  The norm alone decides: it is measured on the Q1
+    that was computed, and unlike R1's diagonal it does not depend on the
+    scaling of the columns."""
+    d = M.shape[0]
+    dev = M.device
+    R = torch.empty((n, n), dtype=F64, device=dev)
+    z = torch.empty(n, dtype=F64, device=dev)
+    stats = torch.empty(4, dtype=F64, device=dev)
+    ws = workspace(_query(lib().pamd_sketch_rz_workspace, d, n), dev)
+    check(lib().pamd_sketch_rz_f64(d, n, _p(M), M.stride(0), int(shifted), int(newton), _p(R), n, _p(z), _p(stats),
+                                   _p(ws), stream(dev)), "pamd_sketch_rz_f64")
+    dd = stats.cpu().numpy()
+    if dd[3] != 0 or not np.all(np.isfinite(dd)) or dd[0] <= 0 or dd[2] > SKETCH_MAX_E:
+        return None
+    return R, z, dd[2]
+
+
+SKETCH_RZ_MIN_N, SKETCH_RZ_MAX_N = 64, 1024
+
+
+def sketch_rz_cholqr2(M, n, shifted=False):
     """(R, z) of a sketch M = [S A | S b] (d x (n + 1)) by CholeskyQR2 on
     S A: R1 = chol((S A)^T S A), Q1 = S A R1^{-1}, R2 = chol(Q1^T Q1); then
     R = R2 R1 (positive diagonal) and z = R2^{-T} Q1^T S b = Q^T S b for
     Q = Q1 R2^{-1}, which is never formed.  These are a Householder QR's R
-    and Q^T S b up to the signs of R's rows, to O(u kappa) for
-    kappa(S A) << u^{-1/2}.  Q1^T Q1 = I + E with ||E|| of order
-    kappa^2 u: while ||E||_F <= SKETCH_NEWTON_MAX_E, R2 = I + X comes from
-    two fixed-point steps X = H(E - X^T X) (H: the upper triangle with the
-    diagonal halved; the error after them is O(||E||^3)), else from potrf.
-    None when S A is too ill-conditioned for it (a pivot fails or R1's
-    diagonal spread exceeds CHOLQR_MAX_COND); the caller then factors M by
-    Householder.  On sketches of a few hundred rows this is much shorter than
-    a panel-by-panel Householder QR."""
+    and Q^T S b (R up to the signs of its rows, z with them).  The second
+    round is two Newton steps while ||Q1^T Q1 - I||_F <= SKETCH_NEWTON_MAX_E
+    (their error is O(||E||^3)), else potrf.  With ``shifted``, the same on
+    S A R0^{-1} with R0 from the shifted Gram matrix, for kappa(S A) beyond
+    what the Gram matrix of S A holds.  None when S A is too ill-conditioned;
+    M is unmodified."""
     d, ncols = M.shape
-    if n < 1 or n > CHOLQR_MAX_K or d < n or ncols != n + 1:
+    if n < 1 or n > SKETCH_RZ_MAX_N or d < n or ncols != n + 1 or M.stride(1) != 1:
         return None
-    SA, Sb = M[:, :n], M[:, n:]
-    info = torch.zeros(2, dtype=torch.int32, device=M.device)
-    G1, Q1 = _chol_round(SA, info[0:1])
-    QtQ = gemm(Q1.t(), Q1)
-    E = small_combine(QtQ, sigma=-1.0)  # as in _newton_round: E, ||E||_F, H(E)
-    enorm = nrm2(E.reshape(-1))
-    X = small_combine(E, upper_half=True)
-    stats = torch.empty(4, dtype=F64, device=M.device)
-    check(lib().pamd_cholqr_stats_f64(n, _p(G1), G1.stride(0), _p(info), _p(enorm), _p(stats), stream(M.device)),
-          "pamd_cholqr_stats_f64")
-    dd = stats.cpu().numpy()  # one read: R1's diagonal spread, ||E||_F, the first pivot
-    if dd[3] != 0 or not np.all(np.isfinite(dd)) or dd[0] <= 0 or dd[1] / dd[0] > CHOLQR_MAX_COND:
-        return None
-    w = gemm(Q1.t(), Sb).reshape(n)
-    if dd[2] <= SKETCH_NEWTON_MAX_E:
-        X = small_combine(QtQ, gemm(X.t(), X), alpha=-1.0, sigma=-1.0, upper_half=True)  # H(E - X^T X)
-        R2 = small_combine(X, sigma=1.0)  # I + X (upper triangular)
-    else:
-        potrf_(QtQ, info[1:2])
-        if int(info[1].item()) != 0:
-            return None
-        R2 = torch.triu(QtQ)
-    R = gemm(R2, torch.triu(G1))
-    z = trsv_(R2, w, trans=True)
-    return R, z
+    out = _sketch_rz(M, n, shifted, True)
+    if out is not None and out[2] > SKETCH_NEWTON_MAX_E:
+        out = _sketch_rz(M, n, shifted, False)
+    return None if out is None else out[:2]
+
+
+def sketch_rz_(M, n):
+    """(R, z = Q^T S b) of a sketch M = [S A | S b] (contiguous; overwritten
+    only by the last resort): CholeskyQR2, the shifted CholeskyQR3 when S A is
+    too ill-conditioned for it, Householder (qr_r_) when that fails too or n
+    is out of range.  At n = 64 Householder takes 222 us, CholeskyQR2 110 and,
+    having failed first, the shifted form 265; at n = 32 it is 103, 91 and 219."""
+    if SKETCH_RZ_MIN_N <= n <= SKETCH_RZ_MAX_N:
+        for shifted in (False, True):
+            rz = sketch_rz_cholqr2(M, n, shifted)
+            if rz is not None:
+                return rz
+    fac = qr_r_(M, n)
+    return fac.R().contiguous(), M[:, n][:n].clone()
 
 
 def orth_q(Y, rounds=2):
