@@ -25,6 +25,8 @@
 // iterations in batches and reads the state back once per batch.  u is kept
 // unnormalised: the 1/beta of lsqr.py:425 is folded into the next pass's
 // c2 = -alpha / beta.
+#include <math.h>
+
 #include "common.h"
 #include "trsv_dev.h"
 #include "trsv_pack.h"
@@ -36,7 +38,9 @@ struct LsqrState {
   double rhobar, phibar, rnorm, r1norm, r2norm, arnorm, bnorm;
   double c1, c2;
   int64_t itn, istop, done, early, phase;
+  double hist[8];  // arnorm after iteration i at i % 8
 };
+static_assert(sizeof(LsqrState) <= 64 * sizeof(double), "the state's place in the workspace");
 
 struct LsqrConst {
   int64_t m, n, lda, ldr, iter_lim;
@@ -433,6 +437,7 @@ __device__ inline bool lsqr_scalars(const LsqrConst& K, LsqrState* S, double* __
   S->r1norm = r1norm;
   S->r2norm = rnorm;
   S->arnorm = arnorm;
+  S->hist[itn & 7] = arnorm;
   S->c1 = 1.0;
   S->c2 = (beta > 0.0) ? -alfa * (1.0 / beta) : -alfa;
   return istop != 0;
@@ -987,6 +992,18 @@ int lsqr_start(const pamd_lsqr_problem* prob, double* x, double* var, double* ar
   return launch_tail(K, P.R, x, var, arnorms, ws, shmem, st);  // phase 0: set-up
 }
 
+// iterations to launch next, from the state after the last batch
+int64_t lsqr_next_batch(const LsqrState& s, const LsqrConst& K, int64_t batch) {
+  const int64_t doubled = imin64(2 * batch, 64);
+  if (s.itn < 5 || !(K.atol > 0.0)) return doubled;
+  const double before = s.hist[(s.itn - 4) & 7];
+  const double test2 = s.arnorm / (s.anorm * s.rnorm);
+  if (!(s.arnorm > 0.0) || !(before > s.arnorm) || !(test2 > K.atol)) return doubled;
+  const double need = 4.0 * log(test2 / K.atol) / log(before / s.arnorm);
+  if (!(need < 64.0)) return doubled;
+  return imax64(2, (int64_t)ceil(need) + 1);
+}
+
 // the result fields from the device state (one thread)
 __global__ void lsqr_result_kernel(const double* __restrict__ ws, pamd_lsqr_result* __restrict__ r) {
   if (threadIdx.x != 0) return;
@@ -1014,13 +1031,15 @@ extern "C" int pamd_lsqr_run_f64(const pamd_lsqr_problem* prob, double* x, doubl
   const pamd_lsqr_problem& P = *prob;
   double* ws = (double*)workspace;
 
+  // Iterations go out in batches, the state is read back after each (a
+  // synchronisation, about 20 us).  An iteration launched after the stop still
+  // costs its launches (7 us), so after the first batch the next one is the
+  // number of iterations test2 needs at its rate over the last four, plus one;
+  // a fixed doubling launched 60 iterations where 36 were needed.
   LsqrState hs;
-  int64_t batch = 4;
+  int64_t batch = 8;
   int64_t launched = 0;
   for (;;) {
-    PAMD_HIP_CHECK(hipMemcpyAsync(&hs, ws, sizeof(LsqrState), hipMemcpyDeviceToHost, st));
-    PAMD_HIP_CHECK(hipStreamSynchronize(st));
-    if (hs.done || launched >= P.iter_lim) break;
     const int64_t todo = imin64(batch, P.iter_lim - launched);
     for (int64_t it = 0; it < todo; ++it) {
       rc = launch_pass(K, P.A, ws, st);
@@ -1028,8 +1047,11 @@ extern "C" int pamd_lsqr_run_f64(const pamd_lsqr_problem* prob, double* x, doubl
       rc = launch_tail(K, P.R, x, var, arnorms, ws, shmem, st);
       if (rc) return rc;
     }
-    launched += todo;
-    batch = imin64(batch * 2, 64);
+    launched += imax64(todo, 0);
+    PAMD_HIP_CHECK(hipMemcpyAsync(&hs, ws, sizeof(LsqrState), hipMemcpyDeviceToHost, st));
+    PAMD_HIP_CHECK(hipStreamSynchronize(st));
+    if (hs.done || launched >= P.iter_lim) break;
+    batch = lsqr_next_batch(hs, K, batch);
   }
   if (x_orig) {
     rc = launch_xorig(K, P.R, x, x_orig, ws, shmem, st);
