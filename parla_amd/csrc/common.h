@@ -101,6 +101,21 @@ __device__ __forceinline__ int pamd_opaque(int x) {
   return x;
 }
 
+// A matrix larger than the 256 MB Infinity Cache is read without displacing
+// what is small and used again: its own lines would be gone before its next
+// pass.  LSQR on 131072 x 512 (537 MB): pass 88 -> 75 us (7.1 TB/s), and the
+// one-workgroup tail, whose packed R then stays in L2, 52 -> 33.  Below that
+// size the cached pass is the faster one (20000 x 200: 7.7 against 9.0 us).
+constexpr int64_t PAMD_STREAM_BYTES = (int64_t)256 << 20;
+
+template <bool STREAM, typename T>
+__device__ __forceinline__ T pamd_load(const T* p) {
+  if constexpr (STREAM)
+    return __builtin_nontemporal_load(p);
+  else
+    return *p;
+}
+
 // value of v in lane `lane` (uniform index), for every lane
 __device__ __forceinline__ double wave_bcast(double v, int lane) {
   const long long b = __double_as_longlong(v);

@@ -54,22 +54,21 @@ struct LsqrConst {
 // scratch (<= 64 KiB of dynamic LDS)
 constexpr int64_t LSQR_LDS_MAX_N = 1900;
 
-// Pass workgroups of lsqr_waves(m, n) wavefronts, one wavefront per row at a
-// time: four, or more where that still leaves at least one workgroup per CU
-// (wider workgroups leave fewer partials for the tail to sum; the register
-// tile of 4 * NPL doubles per lane bounds the width).
+// Pass workgroups of lsqr_waves(n) wavefronts, one wavefront per row at a time:
+// as wide as the register tile of 4 * NPL doubles per lane allows, since a
+// workgroup leaves one partial for the reduction to read.
 __host__ __device__ inline int lsqr_npl(int64_t n) {
   return n <= 64 ? 1 : n <= 128 ? 2 : n <= 256 ? 4 : n <= 512 ? 8 : n <= 1024 ? 16 : 0;
 }
-// wavefronts over the rows of A: one per 16 rows, at most 4096 (16 per CU)
-__host__ __device__ inline int64_t lsqr_total_waves(int64_t m) { return imax64(1, imin64(4096, pamd_cdiv(m, 16))); }
-__host__ __device__ inline int lsqr_waves(int64_t m, int64_t n) {
+// wavefronts over the rows of A: one per 4 rows, at most 4096 (16 per CU; one
+// workgroup each)
+__host__ __device__ inline int64_t lsqr_total_waves(int64_t m) { return imax64(1, imin64(4096, pamd_cdiv(m, 4))); }
+__host__ __device__ inline int lsqr_waves(int64_t n) {
   const int npl = lsqr_npl(n);
-  const int wide = (npl >= 1 && npl <= 8) ? 16 : (npl == 16 ? 8 : 4);
-  return pamd_cdiv(lsqr_total_waves(m), wide) >= 256 ? wide : 4;
+  return (npl >= 1 && npl <= 8) ? 16 : (npl == 16 ? 8 : 4);
 }
 __host__ __device__ inline int lsqr_grid(int64_t m, int64_t n) {
-  return (int)pamd_cdiv(lsqr_total_waves(m), lsqr_waves(m, n));
+  return (int)pamd_cdiv(lsqr_total_waves(m), lsqr_waves(n));
 }
 
 // The packed path (R given, n <= TP_MAX_N): R is packed once per solve
@@ -105,10 +104,10 @@ __host__ __device__ inline LsqrLayout lsqr_layout(int64_t m, int64_t n) {
 // pass over A
 // ---------------------------------------------------------------------------
 // NPL = columns per lane held in registers (n <= 64 * NPL); NPL = 0: any n,
-// the row is read twice (the second read hits cache).  WAVES wavefronts per
+// the row is read twice (the second read hits cache, so not streamed).  WAVES wavefronts per
 // workgroup (lsqr_waves); the workgroup's partial of A^T u' is the sum of its
 // wavefronts' in wavefront order.
-template <int NPL, int WAVES>
+template <int NPL, int WAVES, bool STREAM>
 __global__ __launch_bounds__(64 * WAVES) void lsqr_pass_kernel(LsqrConst K, const double* __restrict__ A,
                                                                double* __restrict__ ws) {
   constexpr int THREADS = 64 * WAVES;
@@ -144,7 +143,7 @@ __global__ __launch_bounds__(64 * WAVES) void lsqr_pass_kernel(LsqrConst K, cons
 #pragma unroll
       for (int q = 0; q < NPL; ++q) {
         const int64_t c = lane + 64 * q;
-        a[q] = (c < n) ? A[row * K.lda + c] : 0.0;
+        a[q] = (c < n) ? pamd_load<STREAM>(A + row * K.lda + c) : 0.0;
       }
     }
     for (; row < K.m; row += gw) {
@@ -155,7 +154,7 @@ __global__ __launch_bounds__(64 * WAVES) void lsqr_pass_kernel(LsqrConst K, cons
 #pragma unroll
         for (int q = 0; q < NPL; ++q) {
           const int64_t c = lane + 64 * q;
-          an[q] = (c < n) ? A[nrow * K.lda + c] : 0.0;
+          an[q] = (c < n) ? pamd_load<STREAM>(A + nrow * K.lda + c) : 0.0;
         }
       }
       const double uin = u[row];
@@ -876,20 +875,22 @@ __global__ __launch_bounds__(TP_THREADS) void lsqr_tailp_kernel(LsqrConst K, dou
 
 int launch_pass(const LsqrConst& K, const double* A, double* ws, hipStream_t st) {
   const int npl = lsqr_npl(K.n);
-  const bool wide = lsqr_waves(K.m, K.n) > 4;
-#define PAMD_PASS(NPL, WAVES) lsqr_pass_kernel<NPL, WAVES><<<K.grid, 64 * WAVES, 0, st>>>(K, A, ws)
+  const bool stream = K.m * K.n * (int64_t)sizeof(double) > PAMD_STREAM_BYTES;
+#define PAMD_PASS(NPL, WAVES)                                                             \
+  stream ? lsqr_pass_kernel<NPL, WAVES, true><<<K.grid, 64 * WAVES, 0, st>>>(K, A, ws)    \
+         : lsqr_pass_kernel<NPL, WAVES, false><<<K.grid, 64 * WAVES, 0, st>>>(K, A, ws)
   if (npl == 1)
-    wide ? PAMD_PASS(1, 16) : PAMD_PASS(1, 4);
+    PAMD_PASS(1, 16);
   else if (npl == 2)
-    wide ? PAMD_PASS(2, 16) : PAMD_PASS(2, 4);
+    PAMD_PASS(2, 16);
   else if (npl == 4)
-    wide ? PAMD_PASS(4, 16) : PAMD_PASS(4, 4);
+    PAMD_PASS(4, 16);
   else if (npl == 8)
-    wide ? PAMD_PASS(8, 16) : PAMD_PASS(8, 4);
+    PAMD_PASS(8, 16);
   else if (npl == 16)
-    wide ? PAMD_PASS(16, 8) : PAMD_PASS(16, 4);
+    PAMD_PASS(16, 8);
   else
-    PAMD_PASS(0, 4);
+    lsqr_pass_kernel<0, 4, false><<<K.grid, 256, 0, st>>>(K, A, ws);
 #undef PAMD_PASS
   PAMD_LAUNCH_CHECK();
   return PAMD_OK;

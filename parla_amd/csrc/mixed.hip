@@ -418,7 +418,7 @@ constexpr int NP_MAX_GRID = 1024;
 // workgroups is faster (131072 x 200 FP32 with its reduction: 22.8 against
 // 27.3 us; at 20000 rows it is slower, 14.4 against 13.5).  Wider rows: 4
 // wavefronts (LDS, registers), one row ahead.
-template <typename T, int NPL, int W, int D>
+template <typename T, int NPL, int W, int D, bool STREAM>
 __global__ __launch_bounds__(64 * W) void normal_pass_kernel(int64_t m, int64_t n, const T* __restrict__ B,
                                                              int64_t ldb, const double* __restrict__ p,
                                                              double* __restrict__ part) {
@@ -441,7 +441,7 @@ __global__ __launch_bounds__(64 * W) void normal_pass_kernel(int64_t m, int64_t 
 #pragma unroll
     for (int q = 0; q < NPL; ++q) {
       const int64_t c = lane + 64 * q;
-      a[k][q] = (r < m && c < n) ? B[r * ldb + c] : T(0);
+      a[k][q] = (r < m && c < n) ? pamd_load<STREAM>(B + r * ldb + c) : T(0);
     }
   }
   for (; row < m; row += gw) {
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(64 * W) void normal_pass_kernel(int64_t m, int64_t 
 #pragma unroll
     for (int q = 0; q < NPL; ++q) {
       const int64_t c = lane + 64 * q;
-      an[q] = (nrow < m && c < n) ? B[nrow * ldb + c] : T(0);
+      an[q] = (nrow < m && c < n) ? pamd_load<STREAM>(B + nrow * ldb + c) : T(0);
     }
     double s = 0.0;
 #pragma unroll
@@ -544,7 +544,7 @@ __device__ __forceinline__ void wave_sum2(double& s, double& c) {
   }
 }
 
-template <int NPL>
+template <int NPL, bool STREAM>
 __global__ __launch_bounds__(NP_THREADS) void residual_kernel(int64_t m, int64_t n, const double* __restrict__ A,
                                                               int64_t lda, const double* __restrict__ x,
                                                               const double* __restrict__ b, double* __restrict__ r,
@@ -569,7 +569,7 @@ __global__ __launch_bounds__(NP_THREADS) void residual_kernel(int64_t m, int64_t
 #pragma unroll
     for (int q = 0; q < NPL; ++q) {
       const int64_t c = lane + 64 * q;
-      a[q] = (c < n) ? A[row * lda + c] : 0.0;
+      a[q] = (c < n) ? pamd_load<STREAM>(A + row * lda + c) : 0.0;
     }
     double s = 0.0, cs = 0.0;
 #pragma unroll
@@ -766,17 +766,26 @@ int trsm_rec(int64_t m, int64_t n, const double* R, int64_t ldr, const double* X
 inline int64_t np_grid(int64_t m) { return imax64(1, imin64(NP_MAX_GRID, pamd_cdiv(m, 64))); }
 
 // the normal pass's launch shape for rows of 64 NPL values (see normal_pass_kernel)
+template <typename T, int NPL, bool STREAM>
+void np_launch_as(unsigned grid, bool deep, hipStream_t st, int64_t m, int64_t n, const T* B, int64_t ldb,
+                  const double* p, double* part) {
+  if constexpr (NPL <= 4) {
+    if (deep)
+      normal_pass_kernel<T, NPL, 16, 4, STREAM><<<grid, 1024, 0, st>>>(m, n, B, ldb, p, part);
+    else
+      normal_pass_kernel<T, NPL, 16, 1, STREAM><<<grid, 1024, 0, st>>>(m, n, B, ldb, p, part);
+  } else {
+    normal_pass_kernel<T, NPL, 4, 1, STREAM><<<grid, 256, 0, st>>>(m, n, B, ldb, p, part);
+  }
+}
+
 template <typename T, int NPL>
 void np_launch(unsigned grid, bool deep, hipStream_t st, int64_t m, int64_t n, const T* B, int64_t ldb,
                const double* p, double* part) {
-  if constexpr (NPL <= 4) {
-    if (deep)
-      normal_pass_kernel<T, NPL, 16, 4><<<grid, 1024, 0, st>>>(m, n, B, ldb, p, part);
-    else
-      normal_pass_kernel<T, NPL, 16, 1><<<grid, 1024, 0, st>>>(m, n, B, ldb, p, part);
-  } else {
-    normal_pass_kernel<T, NPL, 4, 1><<<grid, 256, 0, st>>>(m, n, B, ldb, p, part);
-  }
+  if (m * n * (int64_t)sizeof(T) > PAMD_STREAM_BYTES)
+    np_launch_as<T, NPL, true>(grid, deep, st, m, n, B, ldb, p, part);
+  else
+    np_launch_as<T, NPL, false>(grid, deep, st, m, n, B, ldb, p, part);
 }
 
 }  // namespace
@@ -942,7 +951,10 @@ extern "C" int pamd_residual_f64(int64_t m, int64_t n, const double* A, int64_t 
   const int64_t grid = np_grid(m);
   double* part = (double*)workspace;
   const int npl = (int)pamd_cdiv(n, 64);
-#define PAMD_RK(NPL) residual_kernel<NPL><<<(unsigned)grid, NP_THREADS, 0, st>>>(m, n, A, lda, x, b, r, part)
+  const bool streamed = m * n * (int64_t)sizeof(double) > PAMD_STREAM_BYTES;
+#define PAMD_RK(NPL)                                                                                            \
+  streamed ? residual_kernel<NPL, true><<<(unsigned)grid, NP_THREADS, 0, st>>>(m, n, A, lda, x, b, r, part)     \
+           : residual_kernel<NPL, false><<<(unsigned)grid, NP_THREADS, 0, st>>>(m, n, A, lda, x, b, r, part)
   if (npl <= 1) PAMD_RK(1);
   else if (npl <= 2) PAMD_RK(2);
   else if (npl <= 4) PAMD_RK(4);

@@ -166,7 +166,7 @@ def nrm2(x):
     x = x.contiguous()
     out = torch.empty(1, dtype=F64, device=x.device)
     n = x.numel()
-    if n > (1 << 18):  # long vectors: one partial per workgroup
+    if n > (1 << 15):  # long vectors: one partial per workgroup (one workgroup: 16 us at 131072, two launches: 7)
         ws = workspace(_query(lib().pamd_nrm2_workspace, n), x.device)
         check(lib().pamd_nrm2_large_f64(n, _p(x), _p(out), _p(ws), stream(x.device)), "pamd_nrm2_large_f64")
         return out
