@@ -10,13 +10,11 @@
 // step); every product and sum is FP32.  Parameter vector layout (FP32
 // master, and the same order for gradients):
 //   W1[16][64] | b1[64] | W2[64][64] | b2[64] | w3[64] | b3        (5313)
-// One thread evaluates one row; the BF16 weights are widened once per
+// Forward: one thread evaluates one row; the BF16 weights are widened once per
 // workgroup into LDS and read there by same-address (broadcast) loads.
-// Backward recomputes the forward pass (it is cheaper than storing
-// activations), keeps each row's h1, dh2 and dh1 in that row's LDS vectors,
-// and reduces the weight gradients of the workgroup's 256 rows from LDS;
-// workgroup partials are summed in a fixed order by a second kernel, so the
-// gradients are deterministic.
+// Backward recomputes the forward pass (cheaper than storing activations) on
+// the matrix units; workgroup partials are summed in a fixed order by a second
+// kernel, so the gradients are deterministic.
 #include "common.h"
 #include "rng.h"
 
@@ -102,119 +100,271 @@ __global__ __launch_bounds__(MLP_THREADS) void mlp_fwd_kernel(int64_t rows, cons
   y[r] = mlp_eval(s, x, hrow[threadIdx.x], h2);
 }
 
-// Loss = (1 / rows_total) sum_r (y_r - t_r)^2 over this call's rows; writes
-// per-workgroup partial gradients part[blockIdx.x][0 .. MLP_NPARAM) and the
-// partial loss in part[blockIdx.x][MLP_NPARAM].  va / vb are per-row LDS
-// vectors, reused phase by phase: (h1, dh2) -> dW2, db2; (h1 mask) -> dh1;
-// (dy h2, dh1) -> dw3, db1; (x, dh1) -> dW1.
-__global__ __launch_bounds__(MLP_THREADS) void mlp_bwd_kernel(int64_t rows, double inv_total,
-                                                              const float* __restrict__ X, int64_t ldx,
-                                                              const float* __restrict__ t,
-                                                              const uint16_t* __restrict__ wb,
-                                                              const float* __restrict__ bias,
-                                                              float* __restrict__ part) {
-  __shared__ MlpLds s;
-  __shared__ float va[MLP_THREADS][MLP_H + 1];
-  __shared__ float vb[MLP_THREADS][MLP_H + 1];
-  __shared__ float red[MLP_THREADS / 64][2];
-  load_weights(s, wb, bias);
-  __syncthreads();
-  const int tid = threadIdx.x;
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + tid;
-  const bool valid = r < rows;
-  float x[MLP_IN], h2[MLP_H];
-#pragma unroll
-  for (int k = 0; k < MLP_IN; ++k) x[k] = valid ? asinhf(X[r * ldx + k]) : 0.f;
-  const float yv = mlp_eval(s, x, va[tid], h2);  // h1 -> va[tid]
-  const float diff = valid ? yv - t[r] : 0.f;
-  const float dy = (float)(2.0 * inv_total) * diff;
-  const float lossc = (float)inv_total * diff * diff;
-  // dh2 = dy w3 (h2 > 0) -> vb[tid]
-#pragma unroll
-  for (int j = 0; j < MLP_H; ++j) vb[tid][j] = (h2[j] > 0.f) ? dy * s.w3[j] : 0.f;
-  float* out = part + (int64_t)blockIdx.x * (MLP_NPARAM + 1);
-  __syncthreads();
-  {  // dW2[a][b] = sum_rows h1[a] dh2[b]: 16 (a, b) pairs per thread
-    const int a = tid >> 2, b0 = (tid & 3) * 16;
-    float acc[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = 0.f;
-    for (int rr = 0; rr < MLP_THREADS; ++rr) {
-      const float ha = va[rr][a];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) acc[q] = fmaf(ha, vb[rr][b0 + q], acc[q]);
-    }
-#pragma unroll
-    for (int q = 0; q < 16; ++q) out[OFF_W2 + a * MLP_H + b0 + q] = acc[q];
-  }
-  if (tid < MLP_H) {  // db2
-    float acc = 0.f;
-    for (int rr = 0; rr < MLP_THREADS; ++rr) acc += vb[rr][tid];
-    out[OFF_B2 + tid] = acc;
-  }
-  __syncthreads();
-  {  // dh1[a] = (h1[a] > 0) sum_b W2[a][b] dh2[b], into vb[tid] (own row)
-    float dh2[MLP_H];
-#pragma unroll
-    for (int b = 0; b < MLP_H; ++b) dh2[b] = vb[tid][b];
-    for (int a = 0; a < MLP_H; ++a) {
-      float acc = 0.f;
-#pragma unroll
-      for (int b = 0; b < MLP_H; ++b) acc = fmaf(s.w2[a][b], dh2[b], acc);
-      vb[tid][a] = (va[tid][a] > 0.f) ? acc : 0.f;
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < MLP_H; ++j) va[tid][j] = dy * h2[j];
-  __syncthreads();
-  if (tid < MLP_H) {  // db1, dw3
-    float acc1 = 0.f, acc3 = 0.f;
-    for (int rr = 0; rr < MLP_THREADS; ++rr) {
-      acc1 += vb[rr][tid];
-      acc3 += va[rr][tid];
-    }
-    out[OFF_B1 + tid] = acc1;
-    out[OFF_W3 + tid] = acc3;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < MLP_IN; ++k) va[tid][k] = x[k];
-  __syncthreads();
-  {  // dW1[k][a] = sum_rows x[k] dh1[a]: 4 entries per thread
-    const int k = tid >> 4, a0 = (tid & 15) * 4;
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int rr = 0; rr < MLP_THREADS; ++rr) {
-      const float xk = va[rr][k];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) acc[q] = fmaf(xk, vb[rr][a0 + q], acc[q]);
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) out[OFF_W1 + k * MLP_H + a0 + q] = acc[q];
-  }
-  // db3 and the loss
-  const float sdy = wave_sum(dy), sl = wave_sum(lossc);
-  if ((tid & 63) == 0) {
-    red[tid >> 6][0] = sdy;
-    red[tid >> 6][1] = sl;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    float a = 0.f, l = 0.f;
-    for (int w = 0; w < MLP_THREADS / 64; ++w) {
-      a += red[w][0];
-      l += red[w][1];
-    }
-    out[OFF_B3] = a;
-    out[MLP_NPARAM] = l;
-  }
+// ---------------------------------------------------------------------------
+// Backward.  Loss = (1 / rows_total) sum_r (y_r - t_r)^2 over this call's rows;
+// partial gradients part[blockIdx.x][0 .. MLP_NPARAM) and the partial loss in
+// part[blockIdx.x][MLP_NPARAM].
+//
+// Every product is v_mfma_f32_16x16x4f32 (FP32 products and sums), one
+// wavefront per tile of 16 rows, so that an operand value read from LDS or
+// held in a register serves sixteen products instead of one (one thread per
+// row spent 118 us at 65536 rows on LDS reads of the weights and of the rows'
+// activations; the arithmetic is 13 us at the matrix units' rate).  The result
+// layout (lane l, item r: row 4 (l / 16) + r, column l % 16) is the A and B
+// operand layout of a product whose k index runs over (4 (l / 16) + r), so with
+// the k order chosen to match, results feed the next product from registers:
+//   H1t (units x rows) = W1^T X^T   -> left operand of H2
+//   H1  (rows x units) = X W1       -> left operand (transposed) of dW2, mask of dH1
+//   H2  (rows x units) = H1 W2, dH2 -> right operand of dW2
+//   dH1 (rows x units) = dH2 W2^T   -> right operand of dW1
+// and only dH2 passes through LDS, to become dH1's left operand.  dW2, dW1 and
+// the bias gradients stay in registers over the wavefront's tiles.
+// ---------------------------------------------------------------------------
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+constexpr int BW_WAVES = 8;
+constexpr int BW_THREADS = 64 * BW_WAVES;
+constexpr int BW_MAX_GRID = 256;  // one workgroup per CU; further rows are looped over
+
+inline int64_t bw_grid(int64_t rows) {
+  return imax64(1, imin64(BW_MAX_GRID, pamd_cdiv(rows, 16 * BW_WAVES)));
 }
 
-__global__ void mlp_reduce_kernel(int64_t nparts, const float* __restrict__ part, float* __restrict__ grad) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e > MLP_NPARAM) return;
+struct BwLds {
+  f4 w2[4][4][64];    // [i][j][lane]: W2[16 i + 4 g + r][16 j + c], g = lane / 16, c = lane % 16
+  f4 w2t[4][4][64];   // [j][i][lane]: W2[16 i + c][16 j + 4 g + r]
+  float dh2[BW_WAVES][16][MLP_H + 4];
+};
+
+__device__ __forceinline__ float row16_sum(float v) {
+  v += dpp_f32<0xb1>(v);
+  v += dpp_f32<0x4e>(v);
+  v += dpp_f32<0x124>(v);
+  return v + dpp_f32<0x128>(v);
+}
+
+__global__ __launch_bounds__(BW_THREADS) void mlp_bwd_kernel(int64_t rows, double inv_total,
+                                                             const float* __restrict__ X, int64_t ldx,
+                                                             const float* __restrict__ t,
+                                                             const uint16_t* __restrict__ wb,
+                                                             const float* __restrict__ bias,
+                                                             float* __restrict__ part) {
+  __shared__ BwLds s;
+  __shared__ float sum[MLP_NPARAM + 1];
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
+  const int wave = tid >> 6;
+  const uint16_t* wb2 = wb + MLP_IN * MLP_H;
+  for (int e = tid; e < 4 * 4 * 64; e += BW_THREADS) {
+    const int hi = e >> 8, lo = (e >> 6) & 3, l = e & 63, lc = l & 15, lg = l >> 4;
+    f4 u, v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      u[r] = bf16_to_f32(wb2[(16 * hi + 4 * lg + r) * MLP_H + 16 * lo + lc]);
+      v[r] = bf16_to_f32(wb2[(16 * lo + lc) * MLP_H + 16 * hi + 4 * lg + r]);
+    }
+    s.w2[hi][lo][l] = u;
+    s.w2t[hi][lo][l] = v;
+  }
+  for (int e = tid; e <= MLP_NPARAM; e += BW_THREADS) sum[e] = 0.f;
+  // this lane's weights: W1[4 q + g][16 i + c], the biases by unit
+  float w1[4][4], b1n[4], b2n[4], w3n[4];
+  f4 b1t[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w1[q][i] = bf16_to_f32(wb[(4 * q + g) * MLP_H + 16 * i + c]);
+    b1n[i] = bias[16 * i + c];
+    b2n[i] = bias[MLP_H + 16 * i + c];
+    w3n[i] = bf16_to_f32(wb2[MLP_H * MLP_H + 16 * i + c]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) b1t[i][r] = bias[16 * i + 4 * g + r];
+  }
+  const float b3 = bias[2 * MLP_H], inv = (float)inv_total, inv2 = (float)(2.0 * inv_total);
+  __syncthreads();
+
+  f4 dw2[4][4], dw1[4];
+  float db1[4], db2[4], dw3[4], db3 = 0.f, loss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dw2[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+    dw1[i] = f4{0.f, 0.f, 0.f, 0.f};
+    db1[i] = db2[i] = dw3[i] = 0.f;
+  }
+  float(*T)[MLP_H + 4] = s.dh2[wave];
+  for (int64_t r0 = ((int64_t)blockIdx.x * BW_WAVES + wave) * 16; r0 < rows;
+       r0 += (int64_t)gridDim.x * BW_WAVES * 16) {
+    float x[4], xt[4], tr[4];  // X[c][4 q + g], X[4 g + r][c], t[4 g + r] (rows past the end: zero)
+    const bool in = r0 + c < rows;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int64_t rr = r0 + 4 * g + q;
+      x[q] = in ? asinhf(X[(r0 + c) * ldx + 4 * q + g]) : 0.f;
+      xt[q] = rr < rows ? asinhf(X[rr * ldx + c]) : 0.f;
+      tr[q] = rr < rows ? t[rr] : 0.f;
+    }
+    f4 h1t[4], h1[4], h2[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      h1t[i] = b1t[i];
+      h1[i] = f4{b1n[i], b1n[i], b1n[i], b1n[i]};
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        h1t[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[q][i], x[q], h1t[i], 0, 0, 0);
+        h1[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q], w1[q][i], h1[i], 0, 0, 0);
+      }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        h1t[i][r] = fmaxf(h1t[i][r], 0.f);
+        h1[i][r] = fmaxf(h1[i][r], 0.f);
+      }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) h2[j] = f4{b2n[j], b2n[j], b2n[j], b2n[j]};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      f4 w[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = s.w2[i][j][lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) h2[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(h1t[i][r], w[j][r], h2[j], 0, 0, 0);
+    }
+    // y of rows 4 g + r, in every lane of the row group; h2 <- relu, then dH2
+    float dy[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float y = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        h2[j][r] = fmaxf(h2[j][r], 0.f);
+        y = fmaf(h2[j][r], w3n[j], y);
+      }
+      const float diff = (r0 + 4 * g + r < rows) ? row16_sum(y) + b3 - tr[r] : 0.f;
+      dy[r] = inv2 * diff;
+      db3 += dy[r];
+      loss += inv * diff * diff;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        dw3[j] = fmaf(dy[r], h2[j][r], dw3[j]);
+        h2[j][r] = h2[j][r] > 0.f ? dy[r] * w3n[j] : 0.f;
+        db2[j] += h2[j][r];
+        T[4 * g + r][16 * j + c] = h2[j][r];
+      }
+    // dW2[16 i ..][16 j ..] += H1^T dH2 (k: the rows 4 g + r)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          dw2[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(h1[i][r], h2[j][r], dw2[i][j], 0, 0, 0);
+    PAMD_WAVE_SYNC();
+    // dH1 = dH2 W2^T, k over the units 16 j + 4 g + r of row c
+    f4 d1[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d1[i] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f4 a = *reinterpret_cast<const f4*>(&T[c][16 * j + 4 * g]);
+      f4 w[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = s.w2t[j][i][lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d1[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], w[i][r], d1[i], 0, 0, 0);
+    }
+    PAMD_WAVE_SYNC();  // T is written again by the next tile
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        d1[i][r] = h1[i][r] > 0.f ? d1[i][r] : 0.f;
+        db1[i] += d1[i][r];
+      }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dw1[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(xt[r], d1[i][r], dw1[i], 0, 0, 0);
+  }
+  // the bias sums over the four row groups; db3 and the loss are the same in a row group's lanes
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    db1[i] += __shfl_xor(db1[i], 16, 64);
+    db1[i] += __shfl_xor(db1[i], 32, 64);
+    db2[i] += __shfl_xor(db2[i], 16, 64);
+    db2[i] += __shfl_xor(db2[i], 32, 64);
+    dw3[i] += __shfl_xor(dw3[i], 16, 64);
+    dw3[i] += __shfl_xor(dw3[i], 32, 64);
+  }
+  db3 += __shfl_xor(db3, 16, 64);
+  db3 += __shfl_xor(db3, 32, 64);
+  loss += __shfl_xor(loss, 16, 64);
+  loss += __shfl_xor(loss, 32, 64);
+  // the workgroup's sums, wavefront after wavefront
+  for (int w = 0; w < BW_WAVES; ++w) {
+    __syncthreads();
+    if (w != wave) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[OFF_W2 + (16 * i + 4 * g + r) * MLP_H + 16 * j + c] += dw2[i][j][r];
+        sum[OFF_W1 + (4 * g + r) * MLP_H + 16 * i + c] += dw1[i][r];
+      }
+      if (g == 0) {
+        sum[OFF_B1 + 16 * i + c] += db1[i];
+        sum[OFF_B2 + 16 * i + c] += db2[i];
+        sum[OFF_W3 + 16 * i + c] += dw3[i];
+      }
+    }
+    if (lane == 0) {
+      sum[OFF_B3] += db3;
+      sum[MLP_NPARAM] += loss;
+    }
+  }
+  __syncthreads();
+  float* out = part + (int64_t)blockIdx.x * (MLP_NPARAM + 1);
+  for (int e = tid; e <= MLP_NPARAM; e += BW_THREADS) out[e] = sum[e];
+}
+
+// grad[e] = the workgroups' sums in FP64: 64 entries per workgroup, its four
+// wavefronts take the partials g = w, w + 4, ... with eight in flight, and
+// their sums are added in order (one thread per entry walking all 256
+// partials took 62 us)
+__global__ __launch_bounds__(256) void mlp_reduce_kernel(int nparts, const float* __restrict__ part,
+                                                         float* __restrict__ grad) {
+  constexpr int U = 8;
+  __shared__ double red[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int e = (int)blockIdx.x * 64 + lane;
   double acc = 0.0;
-  for (int64_t g = 0; g < nparts; ++g) acc += (double)part[g * (MLP_NPARAM + 1) + e];
-  grad[e] = (float)acc;
+  if (e <= MLP_NPARAM) {
+    const float* p = part + e;
+    int g = wave;
+    for (; g + (U - 1) * 4 < nparts; g += 4 * U) {
+      float v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = p[(int64_t)(g + 4 * u) * (MLP_NPARAM + 1)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) acc += (double)v[u];
+    }
+    for (; g < nparts; g += 4) acc += (double)p[(int64_t)g * (MLP_NPARAM + 1)];
+  }
+  red[wave][lane] = acc;
+  __syncthreads();
+  if (wave == 0 && e <= MLP_NPARAM)
+    grad[e] = (float)((red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]));
 }
 
 // Adam on the FP32 masters; refresh the BF16 weights and FP32 biases.
@@ -287,7 +437,7 @@ extern "C" int pamd_mlp_fwd(int64_t rows, const float* X, int64_t ldx, const uin
 extern "C" int pamd_mlp_bwd_workspace(int64_t rows, int64_t* bytes) {
   PAMD_ARG_CHECK(rows >= 0, 1);
   PAMD_ARG_CHECK(bytes != nullptr, 2);
-  *bytes = imax64(1, pamd_cdiv(rows, MLP_THREADS)) * (MLP_NPARAM + 1) * (int64_t)sizeof(float);
+  *bytes = bw_grid(rows) * (MLP_NPARAM + 1) * (int64_t)sizeof(float);
   return PAMD_OK;
 }
 
@@ -303,11 +453,11 @@ extern "C" int pamd_mlp_bwd(int64_t rows, int64_t rows_total, const float* X, in
   PAMD_ARG_CHECK(grad != nullptr, 8);
   PAMD_ARG_CHECK(workspace != nullptr, 9);
   hipStream_t st = (hipStream_t)stream;
-  const int64_t nblk = pamd_cdiv(rows, MLP_THREADS);
+  const int64_t nblk = bw_grid(rows);
   float* part = (float*)workspace;
-  mlp_bwd_kernel<<<(unsigned)nblk, MLP_THREADS, 0, st>>>(rows, 1.0 / (double)rows_total, X, ldx, t, wb, bias, part);
+  mlp_bwd_kernel<<<(unsigned)nblk, BW_THREADS, 0, st>>>(rows, 1.0 / (double)rows_total, X, ldx, t, wb, bias, part);
   PAMD_LAUNCH_CHECK();
-  mlp_reduce_kernel<<<(unsigned)pamd_cdiv(MLP_NPARAM + 1, 256), 256, 0, st>>>(nblk, part, grad);
+  mlp_reduce_kernel<<<(unsigned)pamd_cdiv(MLP_NPARAM + 1, 64), 256, 0, st>>>((int)nblk, part, grad);
   PAMD_LAUNCH_CHECK();
   return PAMD_OK;
 }
