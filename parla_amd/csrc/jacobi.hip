@@ -16,21 +16,17 @@
 // until every pair is orthogonal to tol = m * eps relative to the pair's
 // norms; the rotations accumulate in V.  Then A = W V^T, the column norms of W
 // are the singular values and its normalised columns the left singular
-// vectors.  Each rotation is computed from fresh inner products of the two
-// columns, so the result has one-sided Jacobi's accuracy (backward stable,
-// with small singular values determined to high relative accuracy for graded
-// matrices), not the squared conditioning of a Gram-matrix method.
+// vectors.  The Gram matrix of a pair of blocks is formed from the columns in
+// every round and rotated with them inside it; its relative accuracy is that of
+// the columns scaled to unit length (Demmel and Veselic 1992), so small singular
+// values of graded matrices keep theirs, unlike with one Gram matrix of A.
 //
 // Parallel order.  The n columns (padded with zero columns) form nb blocks
 // of w columns, nb even.  A sweep is nb - 1 rounds of the round-robin
 // ("circle") tournament over the blocks: in a round every block meets one
-// other block, and each block pair is one workgroup.  The workgroup copies
-// its 2w columns of W into LDS (column-major, so a column is contiguous and a
-// wavefront reads it without bank conflicts), runs one full inner sweep over
-// the 2w columns (2w - 1 steps of w disjoint column pairs, one wavefront per
-// pair: three wave-reduced dot products, the rotation, the update in LDS),
-// writes the columns back, and applies the accumulated 2w x 2w rotation J to
-// its 2w columns of V (V <- V J, read and written once).
+// other block, and each block pair is one workgroup, which runs one full inner
+// sweep over its 2w columns (2w - 1 steps of w disjoint column pairs) on their
+// Gram matrix and applies the accumulated rotation to W and V (see the kernel).
 //
 // Convergence without host synchronisation.  A workgroup that rotated any
 // pair increments the sweep's counter.  Every round kernel of sweep s > 0
@@ -39,19 +35,19 @@
 //
 // Layout in the workspace: W as np columns of m doubles (column j at
 // W + j*m), V as np columns of np doubles, then the column norms, the sorted
-// positions and the per-sweep counters.  w = 8: a round workgroup is eight
-// wavefronts, and its 16 LDS columns take 64 KiB (m <= 512) or 128 KiB
-// (m <= 1024).  Narrow blocks spread a sweep over more workgroups at once
-// (17 per round at n = 266) with fewer wavefronts per SIMD; the rotation's
-// reciprocal and square roots are hardware estimates refined by Newton steps.
+// positions and the per-sweep counters.  w = 8: narrow blocks spread a sweep
+// over more workgroups at once (17 per round at n = 266).
 #include <mutex>
 
 #include "common.h"
 
+typedef double d4 __attribute__((ext_vector_type(4)));
+
 namespace {
 
 constexpr int JAC_BW = 8;                 // columns per block: 16 per pair, one wavefront per column pair
-constexpr int JAC_THREADS = 64 * JAC_BW;  // one round workgroup
+constexpr int JAC_P = 2 * JAC_BW;         // columns of a pair
+constexpr int JAC_THREADS = 512;          // one round workgroup
 constexpr int JAC_MAX_SWEEPS = 64;
 constexpr int64_t JAC_MAX_M = 1024;
 
@@ -109,141 +105,182 @@ __global__ void jac_init_kernel(int64_t m, int64_t n, int64_t np, const double* 
   if (j == 0 && blockIdx.x == 0 && threadIdx.x < JAC_MAX_SWEEPS) cnt[threadIdx.x] = 0;
 }
 
-// 1 / x and 1 / sqrt(x) from the hardware estimates and two Newton steps
-// each (the estimates' relative errors are squared twice: a few ulps)
-__device__ __forceinline__ double rcp_nr(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  y = y * fma(-x, y, 2.0);
-  return y * fma(-x, y, 2.0);
-}
-
+// 1 / sqrt(x): hardware estimate (relative error about 2^-26) and one third-
+// order correction
 __device__ __forceinline__ double rsq_nr(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  const double h = 0.5 * x;
-  y = y * fma(-h * y, y, 1.5);
-  return y * fma(-h * y, y, 1.5);
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
-// One round of sweep `sweep`: workgroup k orthogonalises block pair k.
-// MMAX >= m rows of the pair's columns are staged in LDS.
-template <int BW, int MMAX>
-__global__ __launch_bounds__(64 * BW) void jac_round_kernel(int64_t m, int64_t n, int nb, int sweep, int round,
-                                                            double tol, double* __restrict__ ws) {
-  constexpr int P = 2 * BW;         // columns of the pair
-  constexpr int E = MMAX / 64;      // rows per lane
-  constexpr int NT = 64 * BW;       // threads
-  __shared__ double Ws[P][MMAX];    // the pair's columns of W, column-major
-  __shared__ double Js[P][P + 1];   // accumulated rotation, Js[col][row]
-  const JacLayout L = jac_layout(m, n);
-  const int* cnt = reinterpret_cast<const int*>(ws + L.cnt);
-  if (sweep > 0 && cnt[sweep - 1] == 0) return;  // an earlier sweep rotated nothing: converged
-  double* W = ws + L.W;
-  double* V = ws + L.V;
-  const int np = nb * BW;
-  const int mi = (int)m;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// c, s and t = s / c of the rotation a' = c a - s b, b' = s a + c b that makes
+// a'.b' = 0, from al = a.a, be = b.b, ga = a.b; |theta| <= pi / 4.  With d = be -
+// al, g = 2 ga, h = sqrt(d^2 + g^2): cos 2 theta = |d| / h, so c^2 = (1 + |d| / h)
+// / 2 and s = sign(d) g / (2 h c): two reciprocal square roots in a row and no
+// division (the step is a chain of latencies).  The identity unless rot.
+__device__ __forceinline__ void jac_rotation(bool rot, double al, double be, double ga, double& c, double& s,
+                                             double& t) {
+  const double d = be - al, g = 2.0 * ga;
+  const double r = rsq_nr(fma(d, d, g * g));  // 1 / h
+  const double c2 = fma(0.5 * fabs(d), r, 0.5);
+  const double w = rsq_nr(c2);                // 1 / c
+  const double ss = copysign(0.5 * g, d < 0.0 ? -ga : ga) * r * w;
+  c = rot ? c2 * w : 1.0;
+  s = rot ? ss : 0.0;
+  t = rot ? ss * w : 0.0;
+}
 
+// One round of sweep `sweep`: workgroup k orthogonalises block pair k (P = 16
+// columns, rows in chunks of 16; CH >= ceil(max(m, np) / 128) chunks per
+// wavefront).  What bounds it is the chain of 15 steps; so a step works on the
+// pair's Gram matrix G = W^T W (one MFMA product per round) instead of the
+// columns.  One wavefront holds G's 8 x 8 grid of (pair p, pair q) 2 x 2 blocks
+// in its 64 lanes: a lane reads its block and both pairs' three inner products
+// from LDS, forms both rotations and writes the rotated block, so the step has
+// no barrier and no exchange of rotations: 1000 cycles, most of them the issue of
+// one wavefront's 75 FP64 operations (reducing the inner products of the columns
+// themselves took 2500).  The accumulated rotation J is
+// then applied to the pair's columns of W and V by MFMA from registers that
+// were loaded before the steps.  G is formed afresh in every round, so what is
+// rotated and when the sweeps end is decided by the columns' own inner products.
+// A working round at m = n = 160 takes 12 us, 6.5 of them the steps; the SVD of
+// a 160 x 160 / 266 x 266 / 1000 x 1000 triangle 2.53 -> 1.45 / 5.6 -> 3.0 / 52 -> 28
+// ms.
+template <int CH>
+__global__ __launch_bounds__(JAC_THREADS) void jac_round_kernel(int m, int nb, int sweep, int round, double tol,
+                                                                double* __restrict__ W, double* __restrict__ V,
+                                                                int* __restrict__ cnt) {
+  constexpr int NW = JAC_THREADS / 64;
+  __shared__ double part[NW][JAC_P * JAC_P];
+  __shared__ double G[JAC_P][JAC_P + 8];   // the stride keeps a step's 64 accesses (nearly) off each other's banks
+  __shared__ double Jm[JAC_P][JAC_P + 8];  // Jm[k][j]: column j of the result takes Jm[k][j] of column k
+  __shared__ int any;
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int np = nb * JAC_BW;
+  if (sweep > 0 && cnt[sweep - 1] == 0) return;  // an earlier sweep rotated nothing: converged
   int bp, bq;
   circle_pair(round, blockIdx.x, nb - 1, bp, bq);
   // global column of pair column c
-  auto gcol = [&](int c) -> int64_t { return (c < BW) ? (int64_t)bp * BW + c : (int64_t)bq * BW + (c - BW); };
+  auto gcol = [&](int c) -> int64_t { return (c < JAC_BW) ? bp * JAC_BW + c : bq * JAC_BW + (c - JAC_BW); };
 
-  for (int idx = tid; idx < P * mi; idx += NT) {
-    const int c = idx / mi, i = idx - c * mi;
-    Ws[c][i] = W[gcol(c) * m + i];
+  // Gram operand: column lr, rows 16 Q + 4 lk + r; product operand: column 4 q + lk,
+  // row 16 Q + lr.  Rows past the end are read from the last one and zeroed:
+  // a branch per load made the 24 loads take 4000 cycles to issue.
+  const double* wcol = W + gcol(lr) * m;
+  const double *wprod[4], *vprod[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    wprod[q] = W + gcol(4 * q + lk) * m;
+    vprod[q] = V + gcol(4 * q + lk) * np;
   }
-  for (int idx = tid; idx < P * P; idx += NT) Js[idx / P][idx % P] = (idx / P == idx % P) ? 1.0 : 0.0;
-  __syncthreads();
-
-  const int em = (mi + 63) / 64;
-  const double tol2 = tol * tol;
-  int rotated = 0;
-  for (int t = 0; t < P - 1; ++t) {
-    int a, b;
-    circle_pair(t, wave, P - 1, a, b);
-    double xa[E], xb[E];
-    double al = 0.0, be = 0.0, ga = 0.0;
+  double wg[CH][4], wa[CH][4], va[CH][4];
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      xa[e] = 0.0;
-      xb[e] = 0.0;
-      const int i = lane + 64 * e;
-      if (e < em && i < mi) {
-        xa[e] = Ws[a][i];
-        xb[e] = Ws[b][i];
-      }
-      al = fma(xa[e], xa[e], al);
-      be = fma(xb[e], xb[e], be);
-      ga = fma(xa[e], xb[e], ga);
+  for (int u = 0; u < CH; ++u) {
+    const int r0 = 16 * (wave + NW * u);
+    const int ra = r0 + lr, rm = min(ra, m - 1), rv = min(ra, np - 1);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      wg[u][q] = wcol[min(r0 + 4 * lk + q, m - 1)];
+      wa[u][q] = wprod[q][rm];
+      va[u][q] = vprod[q][rv];
     }
-    al = wave_sum(al);
-    be = wave_sum(be);
-    ga = wave_sum(ga);
-    // rotate unless |ga| <= tol sqrt(al be) (also skips zero columns)
-    if (ga * ga > tol2 * (al * be)) {
-      // a' = c a - s b, b' = s a + c b with a'.b' = 0: t = tan(theta) is the
-      // smaller root of t^2 + 2 zeta t - 1 = 0, zeta = (be - al) / (2 ga)
-      const double zeta = (be - al) * rcp_nr(2.0 * ga);
-      const double az = fabs(zeta);
-      double tt;
-      if (az > 1e150) {
-        tt = 0.5 * rcp_nr(zeta);
-      } else {
-        const double q = fma(zeta, zeta, 1.0);
-        tt = copysign(rcp_nr(az + q * rsq_nr(q)), zeta);
-      }
-      const double c = rsq_nr(fma(tt, tt, 1.0));
-      const double s = c * tt;
+  }
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const int i = lane + 64 * e;
-        if (e < em && i < mi) {
-          Ws[a][i] = c * xa[e] - s * xb[e];
-          Ws[b][i] = s * xa[e] + c * xb[e];
+  for (int u = 0; u < CH; ++u)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) wg[u][q] = (16 * (wave + NW * u) + 4 * lk + q < m) ? wg[u][q] : 0.0;
+  d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int u = 0; u < CH; ++u)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(wg[u][q], wg[u][q], acc, 0, 0, 0);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) part[wave][(lk + 4 * r) * JAC_P + lr] = acc[r];
+  __syncthreads();
+  if (threadIdx.x < JAC_P * JAC_P) {
+    const int i = threadIdx.x / JAC_P, j = threadIdx.x % JAC_P;
+    double g = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) g += part[w][threadIdx.x];
+    G[i][j] = g;
+    Jm[i][j] = i == j ? 1.0 : 0.0;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    // pair p of step t is (15, t) for p = 0, else (t + p, t - p) modulo 15: rows
+    // a, b by p = lane / 8 and columns e, f by q = lane % 8, stepped by one
+    const int p = lane >> 3, q = lane & 7;
+    int a = p ? p : JAC_P - 1, b = p ? JAC_P - 1 - p : 0;
+    int e = q ? q : JAC_P - 1, f = q ? JAC_P - 1 - q : 0;
+    const double tol2 = tol * tol;
+    bool rotated = false;
+    double* J0 = &Jm[2 * p][0];
+    double* J1 = &Jm[2 * p + 1][0];
+    for (int t = 0; t < JAC_P - 1; ++t) {
+      double *Ga = &G[a][0], *Gb = &G[b][0];
+      const double alq = G[e][e], beq = G[f][f], gaq = G[e][f];
+      const double alp = Ga[a], bep = Gb[b], gap = Ga[b];
+      const double gae = Ga[e], gaf = Ga[f], gbe = Gb[e], gbf = Gb[f];
+      const double j0e = J0[e], j0f = J0[f], j1e = J1[e], j1f = J1[f];
+      __builtin_amdgcn_sched_barrier(0);  // every read under way before the first is waited for
+      const bool rq = gaq * gaq > tol2 * (alq * beq);
+      if (__any(rq)) {
+        double cp, sp, tp, cq, sq, tq;
+        jac_rotation(gap * gap > tol2 * (alp * bep), alp, bep, gap, cp, sp, tp);
+        jac_rotation(rq, alq, beq, gaq, cq, sq, tq);
+        rotated = true;
+        // rows (a, b) by p's rotation, then columns (e, f) by q's
+        const double rae = cp * gae - sp * gbe, raf = cp * gaf - sp * gbf;
+        const double rbe = sp * gae + cp * gbe, rbf = sp * gaf + cp * gbf;
+        double nae = cq * rae - sq * raf, naf = sq * rae + cq * raf;
+        double nbe = cq * rbe - sq * rbf, nbf = sq * rbe + cq * rbf;
+        if (p == q && tp != 0.0) {  // the pair's own block: al - t ga, be + t ga, orthogonal
+          nae = fma(-tp, gap, alp);
+          nbf = fma(tp, gap, bep);
+          naf = nbe = 0.0;
         }
+        PAMD_WAVE_SYNC();
+        Ga[e] = nae;
+        Ga[f] = naf;
+        Gb[e] = nbe;
+        Gb[f] = nbf;
+        J0[e] = cq * j0e - sq * j0f;
+        J0[f] = sq * j0e + cq * j0f;
+        J1[e] = cq * j1e - sq * j1f;
+        J1[f] = sq * j1e + cq * j1f;
+        PAMD_WAVE_SYNC();
       }
-      if (lane < P) {
-        const double ja = Js[a][lane], jb = Js[b][lane];
-        Js[a][lane] = c * ja - s * jb;
-        Js[b][lane] = s * ja + c * jb;
-      }
-      rotated = 1;
+      a = p ? (a == JAC_P - 2 ? 0 : a + 1) : a;
+      b = b == JAC_P - 2 ? 0 : b + 1;
+      e = q ? (e == JAC_P - 2 ? 0 : e + 1) : e;
+      f = f == JAC_P - 2 ? 0 : f + 1;
     }
-    __syncthreads();
+    const bool r = __any(rotated);
+    if (lane == 0) any = r;
   }
-  const int any = __syncthreads_or(rotated);
+  __syncthreads();
   if (!any) return;  // the pair was already orthogonal: W and V unchanged
-
-  for (int idx = tid; idx < P * mi; idx += NT) {
-    const int c = idx / mi, i = idx - c * mi;
-    W[gcol(c) * m + i] = Ws[c][i];
-  }
-  __syncthreads();
-  // V(:, pair) <- V(:, pair) J: the pair's V columns (np <= MMAX rows) are
-  // staged in the LDS the W columns used, then each thread forms one row's
-  // 2w outputs, eight at a time
-  for (int idx = tid; idx < P * np; idx += NT) {
-    const int c = idx / np, i = idx - c * np;
-    Ws[c][i] = V[gcol(c) * np + i];
-  }
-  __syncthreads();
-  for (int i = tid; i < np; i += NT) {
+  double jb[4];
 #pragma unroll
-    for (int j0 = 0; j0 < P; j0 += 8) {
-      double acc[8];
+  for (int q = 0; q < 4; ++q) jb[q] = Jm[4 * q + lk][lr];
 #pragma unroll
-      for (int jj = 0; jj < 8; ++jj) acc[jj] = 0.0;
-#pragma unroll 4
-      for (int c = 0; c < P; ++c) {
-        const double v = Ws[c][i];
+  for (int u = 0; u < CH; ++u) {
+    const int r0 = 16 * (wave + NW * u);
+    d4 w = {0.0, 0.0, 0.0, 0.0}, v = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj) acc[jj] = fma(v, Js[j0 + jj][c], acc[jj]);
-      }
+    for (int q = 0; q < 4; ++q) {
+      w = __builtin_amdgcn_mfma_f64_16x16x4f64(wa[u][q], jb[q], w, 0, 0, 0);
+      v = __builtin_amdgcn_mfma_f64_16x16x4f64(va[u][q], jb[q], v, 0, 0, 0);
+    }
 #pragma unroll
-      for (int jj = 0; jj < 8; ++jj) V[gcol(j0 + jj) * np + i] = acc[jj];
+    for (int r = 0; r < 4; ++r) {
+      const int row = r0 + lk + 4 * r;
+      if (row < m) W[gcol(lr) * m + row] = w[r];
+      if (row < np) V[gcol(lr) * np + row] = v[r];
     }
   }
-  if (tid == 0) atomicAdd(reinterpret_cast<int*>(ws + L.cnt) + sweep, 1);
+  if (threadIdx.x == 0) atomicAdd(cnt + sweep, 1);
 }
 
 // sigma_j = ||W(:, j)|| for the first n columns, one workgroup per column
@@ -332,12 +369,19 @@ int jac_launch_sweeps(int64_t m, int64_t n, int max_sweeps, double* ws, hipStrea
   const int w = jac_block(m);
   const int nb = (int)jac_nblocks(n, w);
   const double tol = (double)imax64(m, 16) * 2.220446049250313e-16;
+  const JacLayout L = jac_layout(m, n);
+  double *W = ws + L.W, *V = ws + L.V;
+  int* cnt = reinterpret_cast<int*>(ws + L.cnt);
+  const int64_t rows = imax64(m, (int64_t)nb * w);
   for (int sw = 0; sw < max_sweeps; ++sw) {
     for (int r = 0; r < nb - 1; ++r) {
-      if (m <= 512)
-        jac_round_kernel<JAC_BW, 512><<<nb / 2, JAC_THREADS, 0, st>>>(m, n, nb, sw, r, tol, ws);
-      else
-        jac_round_kernel<JAC_BW, 1024><<<nb / 2, JAC_THREADS, 0, st>>>(m, n, nb, sw, r, tol, ws);
+#define PAMD_JAC(CH) jac_round_kernel<CH><<<nb / 2, JAC_THREADS, 0, st>>>((int)m, nb, sw, r, tol, W, V, cnt)
+      if (rows <= 128) PAMD_JAC(1);
+      else if (rows <= 256) PAMD_JAC(2);
+      else if (rows <= 384) PAMD_JAC(3);
+      else if (rows <= 640) PAMD_JAC(5);
+      else PAMD_JAC(8);
+#undef PAMD_JAC
       PAMD_LAUNCH_CHECK();
     }
   }
