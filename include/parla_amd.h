@@ -623,6 +623,13 @@ int pamd_bt_trsv(int64_t nprob, const pamd_ls_desc* descs, int trans,
 int pamd_bt_trmv(int64_t nprob, const pamd_ls_desc* descs, int trans,
                  const double* Rinv, const double* RinvT, double* v, void* stream);
 
+/* y_i = Rinv_i x_i (trans 0) or Rinv_i^T x_i (trans 1): pamd_bt_trmv out of
+ * place, with the same sums, its columns spread over the chip.  x and y are
+ * n-vector pools that do not overlap. */
+int pamd_bt_trmv_to(int64_t nprob, const pamd_ls_desc* descs, int trans,
+                    const double* Rinv, const double* RinvT, const double* x,
+                    double* y, void* stream);
+
 /* Conjugate gradients on every problem's preconditioned normal equations,
  * recurrences on the device; state[4 i] = r.r, state[4 i + 1] = 1 while
  * problem i is active (0 freezes its vectors).  mode 0 starts from z = 0 with

@@ -103,6 +103,7 @@ SIGNATURES = {
     "pamd_bt_reduce": (c_int, [c_i64, c_vp, c_vp, c_int, c_vp, c_vp, c_vp]),
     "pamd_bt_trsv": (c_int, [c_i64, c_vp, c_int, c_vp, c_vp, c_vp]),
     "pamd_bt_trmv": (c_int, [c_i64, c_vp, c_int, c_vp, c_vp, c_vp, c_vp]),
+    "pamd_bt_trmv_to": (c_int, [c_i64, c_vp, c_int, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "pamd_bt_cg": (c_int, [c_i64, c_vp, c_int, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "pamd_bt_axpy": (c_int, [c_i64, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "pamd_bt_copy": (c_int, [c_i64, c_vp, c_vp, c_vp, c_vp]),

@@ -43,65 +43,151 @@ struct Blk {
   int32_t row0;
 };
 
+// index of this wavefront in the launch, in a scalar register
+__device__ __forceinline__ int64_t bt_wave_id() {
+  return (int64_t)blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+}
+
+// ---------------------------------------------------------------------------
+// Row-block passes, bound by the one read of A.  A wavefront holds its
+// problem's p (or x) and column sums in registers, a lane per column of each
+// 64-column group, and walks its 64 rows G at a time: the next G rows are in
+// flight while these are reduced, and four rows share one cross-lane
+// reduction.  NPL is the problem's exact number of column groups (a class
+// launch picks its body per block), so no lane group beyond the last works for
+// padding, and only the last one masks its columns: out-of-range lanes read
+// the row's last value and hold zero.  With one row reduced at a time and a
+// class's full width, a normal pass over 64 problems of up to 49805 x 512 took
+// 34, 41, 71 and 304 us in the classes 1, 2, 4, 8 (1, 77, 339, 1583 MB); it
+// takes 5, 16, 64 and 296 us, the last 5.4 TB/s.  More wavefronts (conversions
+// repeated, one set of row registers) or fewer with rows further ahead measure
+// the same there.
+// ---------------------------------------------------------------------------
+template <int NPL>
+struct BtRows {
+  static constexpr int G = NPL == 1 ? 16 : NPL <= 4 ? 8 : 4;
+};
+
+// columns lane + 64 q of one row; `last`: the in-range column this lane reads
+// in the last group, `in`: whether it is its own
+template <bool STREAM, int NPL>
+__device__ __forceinline__ void bt_load_row(const float* __restrict__ row, int lane, int last, float (&a)[NPL]) {
+#pragma unroll
+  for (int q = 0; q + 1 < NPL; ++q) a[q] = pamd_load<STREAM>(row + lane + 64 * q);
+  a[NPL - 1] = pamd_load<STREAM>(row + last);
+}
+
 // ---------------------------------------------------------------------------
 // q_i = A_i^T (A_i p_i), partial per block
 // ---------------------------------------------------------------------------
-template <int NPL>
+// acc += A_k^T (A_k p) over the G rows in a, four at a time; with NEXT, row
+// k + G (from next) is loaded over row k as soon as that is converted, so that
+// the loads are in flight while the four rows are worked on
+template <bool NEXT, bool STREAM, int G, int NPL>
+__device__ __forceinline__ void bt_normal_rows(float (&a)[G][NPL], const double (&pr)[NPL], double (&acc)[NPL],
+                                               const float* __restrict__ next, int n, int lane, int last, bool in) {
+#pragma unroll
+  for (int k0 = 0; k0 < G; k0 += 4) {
+    double v[4][NPL], s[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      float(&ak)[NPL] = a[k0 + k];
+      ak[NPL - 1] = in ? ak[NPL - 1] : 0.f;
+#pragma unroll
+      for (int q = 0; q < NPL; ++q) v[k][q] = (double)ak[q];
+      if (NEXT) bt_load_row<STREAM>(next + (int64_t)(k0 + k) * n, lane, last, ak);
+      s[k] = v[k][0] * pr[0];
+#pragma unroll
+      for (int q = 1; q < NPL; ++q) s[k] += v[k][q] * pr[q];
+    }
+    wave_sum4(s);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int q = 0; q < NPL; ++q) acc[q] += s[k] * v[k][q];
+  }
+}
+
+template <int NPL, bool STREAM>
+__device__ __forceinline__ void bt_normal_block(const Desc& d, int64_t row0, const float* __restrict__ A,
+                                                const double* __restrict__ pv, double* __restrict__ part) {
+  constexpr int G = BtRows<NPL>::G;
+  const int lane = threadIdx.x & 63;
+  const int n = (int)d.n;
+  const int cl = lane + 64 * (NPL - 1);
+  const bool in = cl < n;
+  const int last = in ? cl : n - 1;
+  const float* Ai = A + d.a_off + row0 * n;
+  const int nr = (int)imin64(BT_BLOCK_ROWS, d.m - row0);
+  double pr[NPL], acc[NPL];
+#pragma unroll
+  for (int q = 0; q < NPL; ++q) {
+    pr[q] = (q + 1 < NPL || in) ? pv[d.nv_off + lane + 64 * q] : 0.0;
+    acc[q] = 0.0;
+  }
+  const int nf = nr / G * G;
+  if (nf > 0) {
+    float a[G][NPL];  // row r in a[r % G]
+#pragma unroll
+    for (int k = 0; k < G; ++k) bt_load_row<STREAM>(Ai + (int64_t)k * n, lane, last, a[k]);
+    for (int r0 = G; r0 < nf; r0 += G)
+      bt_normal_rows<true, STREAM>(a, pr, acc, Ai + (int64_t)r0 * n, n, lane, last, in);
+    bt_normal_rows<false, STREAM>(a, pr, acc, Ai, n, lane, last, in);
+  }
+  if (nf < nr) {  // the problem's last rows, fewer than a group
+    float a[G - 1][NPL];
+#pragma unroll
+    for (int k = 0; k < G - 1; ++k)
+      if (nf + k < nr) bt_load_row<STREAM>(Ai + (int64_t)(nf + k) * n, lane, last, a[k]);
+#pragma unroll
+    for (int k = 0; k < G - 1; ++k)
+      if (nf + k < nr) {
+        a[k][NPL - 1] = in ? a[k][NPL - 1] : 0.f;
+        double s = (double)a[k][0] * pr[0];
+#pragma unroll
+        for (int q = 1; q < NPL; ++q) s += (double)a[k][q] * pr[q];
+        s = wave_sum(s);
+#pragma unroll
+        for (int q = 0; q < NPL; ++q) acc[q] += s * (double)a[k][q];
+      }
+  }
+  double* pw = part + d.part_off + (row0 / BT_BLOCK_ROWS) * (2 * d.n + 2);
+#pragma unroll
+  for (int q = 0; q < NPL; ++q)
+    if (q + 1 < NPL || in) pw[lane + 64 * q] = acc[q];
+}
+
+// runs BODY<groups of 64 columns> for a problem in a launch of class NPL (a
+// problem may also sit in a wider class than its own)
+#define PAMD_BT_CASE(N, BODY, ...)                                             \
+  case N:                                                                      \
+    if constexpr (N <= NPL) BODY<N, STREAM>(__VA_ARGS__);                      \
+    break;
+#define PAMD_BT_BODY(BODY, ...)                                                \
+  switch ((int)imin64(NPL, pamd_cdiv(d.n, 64))) {                              \
+    PAMD_BT_CASE(1, BODY, __VA_ARGS__)                                         \
+    PAMD_BT_CASE(2, BODY, __VA_ARGS__)                                         \
+    PAMD_BT_CASE(3, BODY, __VA_ARGS__)                                         \
+    PAMD_BT_CASE(4, BODY, __VA_ARGS__)                                         \
+    PAMD_BT_CASE(5, BODY, __VA_ARGS__)                                         \
+    PAMD_BT_CASE(6, BODY, __VA_ARGS__)                                         \
+    PAMD_BT_CASE(7, BODY, __VA_ARGS__)                                         \
+    PAMD_BT_CASE(8, BODY, __VA_ARGS__)                                         \
+  }
+
+template <int NPL, bool STREAM>
 __global__ __launch_bounds__(256) void bt_normal_kernel(const Desc* __restrict__ D, const Blk* __restrict__ blks,
                                                         int64_t nblk, int blocks_per_wave,
                                                         const float* __restrict__ A, const double* __restrict__ pv,
                                                         const double* __restrict__ state, double* __restrict__ part) {
-  const int lane = threadIdx.x & 63;
-  const int64_t wid = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int64_t wid = bt_wave_id();
   for (int k = 0; k < blocks_per_wave; ++k) {
     const int64_t bi = wid * blocks_per_wave + k;
     if (bi >= nblk) return;
     const Blk bk = blks[bi];
     if (state != nullptr && state[4 * bk.prob + 1] == 0.0) continue;  // frozen problem: partial stays
     const Desc d = D[bk.prob];
-    const int64_t n = d.n;
-    const float* Ai = A + d.a_off;
-    double pr[NPL], acc[NPL];
-#pragma unroll
-    for (int q = 0; q < NPL; ++q) {
-      const int64_t c = lane + 64 * q;
-      pr[q] = (c < n) ? pv[d.nv_off + c] : 0.0;
-      acc[q] = 0.0;
-    }
-    const int64_t r1 = imin64(d.m, (int64_t)bk.row0 + BT_BLOCK_ROWS);
-    float a[NPL];
-#pragma unroll
-    for (int q = 0; q < NPL; ++q) {
-      const int64_t c = lane + 64 * q;
-      a[q] = (c < n) ? Ai[(int64_t)bk.row0 * n + c] : 0.f;
-    }
-    for (int64_t row = bk.row0; row < r1; ++row) {
-      // the next row's loads are in flight while this row is reduced
-      float an[NPL];
-      if (row + 1 < r1) {
-#pragma unroll
-        for (int q = 0; q < NPL; ++q) {
-          const int64_t c = lane + 64 * q;
-          an[q] = (c < n) ? Ai[(row + 1) * n + c] : 0.f;
-        }
-      }
-      double s = 0.0;
-#pragma unroll
-      for (int q = 0; q < NPL; ++q) s += (double)a[q] * pr[q];
-      s = wave_sum(s);
-#pragma unroll
-      for (int q = 0; q < NPL; ++q) acc[q] += s * (double)a[q];
-      if (row + 1 < r1) {
-#pragma unroll
-        for (int q = 0; q < NPL; ++q) a[q] = an[q];
-      }
-    }
-    double* pw = part + d.part_off + (int64_t)(bk.row0 / BT_BLOCK_ROWS) * (2 * n + 2);
-#pragma unroll
-    for (int q = 0; q < NPL; ++q) {
-      const int64_t c = lane + 64 * q;
-      if (c < n) pw[c] = acc[q];
-    }
+    PAMD_BT_BODY(bt_normal_block, d, bk.row0, A, pv, part)
   }
 }
 
@@ -127,147 +213,190 @@ __device__ __forceinline__ double bt_add(double a, double b) {
   return a + b;
 }
 
-template <int NPL>
+// (s, c) += (so, co), compensated
+__device__ __forceinline__ void bt_fold(double& s, double& c, double so, double co) {
+  double t, e;
+  bt_two_sum(s, so, t, e);
+  s = t;
+  c = bt_add(bt_add(c, co), e);
+}
+
+// wave_sum4 of four compensated sums
+__device__ __forceinline__ void bt_wave_sum4(double (&s)[4], double (&c)[4]) {
+#pragma unroll
+  for (int k = 0; k < 4; k += 2) {
+    wave_swap<false>(s[k], s[k + 1]);
+    wave_swap<false>(c[k], c[k + 1]);
+    bt_fold(s[k], c[k], s[k + 1], c[k + 1]);
+  }
+  wave_swap<true>(s[0], s[2]);
+  wave_swap<true>(c[0], c[2]);
+  bt_fold(s[0], c[0], s[2], c[2]);
+  bt_fold(s[0], c[0], dpp_f64<0xb1>(s[0]), dpp_f64<0xb1>(c[0]));
+  bt_fold(s[0], c[0], dpp_f64<0x4e>(s[0]), dpp_f64<0x4e>(c[0]));
+  bt_fold(s[0], c[0], dpp_f64<0x124>(s[0]), dpp_f64<0x124>(c[0]));
+  bt_fold(s[0], c[0], dpp_f64<0x128>(s[0]), dpp_f64<0x128>(c[0]));
+  const double t = s[0], u = c[0];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    s[k] = wave_bcast(t, wave_sum4_lane(k));
+    c[k] = wave_bcast(u, wave_sum4_lane(k));
+  }
+}
+
+template <int NPL, bool STREAM>
+__device__ __forceinline__ void bt_residual_block(const Desc& d, int64_t row0, const float* __restrict__ A,
+                                                  const double* __restrict__ b, const double* __restrict__ xv,
+                                                  double* __restrict__ part) {
+  constexpr int G = 4;
+  const int lane = threadIdx.x & 63;
+  const int n = (int)d.n;
+  const int cl = lane + 64 * (NPL - 1);
+  const bool in = cl < n;
+  const int last = in ? cl : n - 1;
+  const float* Ai = A + d.a_off + row0 * n;
+  const double* bi = b + d.mv_off + row0;
+  const int nr = (int)imin64(BT_BLOCK_ROWS, d.m - row0);
+  double xr[NPL], gs[NPL], gc[NPL];
+#pragma unroll
+  for (int q = 0; q < NPL; ++q) {
+    xr[q] = (q + 1 < NPL || in) ? xv[d.nv_off + lane + 64 * q] : 0.0;
+    gs[q] = 0.0;
+    gc[q] = 0.0;
+  }
+  double rr = 0.0;
+  float a[G][NPL], an[G][NPL];
+#pragma unroll
+  for (int k = 0; k < G; ++k)
+    if (k < nr) bt_load_row<STREAM>(Ai + (int64_t)k * n, lane, last, a[k]);
+  for (int r0 = 0; r0 < nr; r0 += G) {
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+      if (r0 + G + k < nr) bt_load_row<STREAM>(Ai + (int64_t)(r0 + G + k) * n, lane, last, an[k]);
+      a[k][NPL - 1] = in ? a[k][NPL - 1] : 0.f;
+    }
+    double s[G], cs[G];
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+      s[k] = 0.0;
+      cs[k] = 0.0;
+      if (r0 + k < nr) {
+#pragma unroll
+        for (int q = 0; q < NPL; ++q) {
+          double p, ep;
+          bt_two_prod((double)a[k][q], xr[q], p, ep);
+          bt_fold(s[k], cs[k], p, ep);
+        }
+      }
+    }
+    bt_wave_sum4(s, cs);
+#pragma unroll
+    for (int k = 0; k < G; ++k)
+      if (r0 + k < nr) {
+        double t, e;
+        bt_two_sum(bi[r0 + k], -s[k], t, e);
+        const double ri = bt_add(t, bt_add(e, -cs[k]));
+        rr += ri * ri;
+#pragma unroll
+        for (int q = 0; q < NPL; ++q) {
+          double p, ep;
+          bt_two_prod(ri, (double)a[k][q], p, ep);
+          bt_fold(gs[q], gc[q], p, ep);
+        }
+      }
+#pragma unroll
+    for (int k = 0; k < G; ++k)
+#pragma unroll
+      for (int q = 0; q < NPL; ++q) a[k][q] = an[k][q];
+  }
+  double* pw = part + d.part_off + (row0 / BT_BLOCK_ROWS) * (2 * d.n + 2);
+#pragma unroll
+  for (int q = 0; q < NPL; ++q)
+    if (q + 1 < NPL || in) {
+      pw[lane + 64 * q] = gs[q];
+      pw[n + lane + 64 * q] = gc[q];
+    }
+  if (lane == 0) pw[2 * n] = rr;
+}
+
+template <int NPL, bool STREAM>
 __global__ __launch_bounds__(256) void bt_residual_kernel(const Desc* __restrict__ D, const Blk* __restrict__ blks,
                                                           int64_t nblk, int blocks_per_wave,
                                                           const float* __restrict__ A, const double* __restrict__ b,
                                                           const double* __restrict__ xv,
                                                           const double* __restrict__ state, double* __restrict__ part) {
-  const int lane = threadIdx.x & 63;
-  const int64_t wid = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int64_t wid = bt_wave_id();
   for (int k = 0; k < blocks_per_wave; ++k) {
     const int64_t bi = wid * blocks_per_wave + k;
     if (bi >= nblk) return;
     const Blk bk = blks[bi];
     if (state != nullptr && state[4 * bk.prob + 1] == 0.0) continue;  // frozen problem: partial stays
     const Desc d = D[bk.prob];
-    const int64_t n = d.n;
-    const float* Ai = A + d.a_off;
-    double xr[NPL], gs[NPL], gc[NPL];
-#pragma unroll
-    for (int q = 0; q < NPL; ++q) {
-      const int64_t c = lane + 64 * q;
-      xr[q] = (c < n) ? xv[d.nv_off + c] : 0.0;
-      gs[q] = 0.0;
-      gc[q] = 0.0;
-    }
-    double rr = 0.0;
-    const int64_t r1 = imin64(d.m, (int64_t)bk.row0 + BT_BLOCK_ROWS);
-    float af[NPL];
-#pragma unroll
-    for (int q = 0; q < NPL; ++q) {
-      const int64_t c = lane + 64 * q;
-      af[q] = (c < n) ? Ai[(int64_t)bk.row0 * n + c] : 0.f;
-    }
-    for (int64_t row = bk.row0; row < r1; ++row) {
-      double a[NPL];
-#pragma unroll
-      for (int q = 0; q < NPL; ++q) a[q] = (double)af[q];
-      if (row + 1 < r1) {  // prefetch the next row
-#pragma unroll
-        for (int q = 0; q < NPL; ++q) {
-          const int64_t c = lane + 64 * q;
-          af[q] = (c < n) ? Ai[(row + 1) * n + c] : 0.f;
-        }
-      }
-      double s = 0.0, cs = 0.0;
-#pragma unroll
-      for (int q = 0; q < NPL; ++q) {
-        double p, ep, t, e;
-        bt_two_prod(a[q], xr[q], p, ep);
-        bt_two_sum(s, p, t, e);
-        s = t;
-        cs = bt_add(cs, bt_add(ep, e));
-      }
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) {
-        const double so = __shfl_xor(s, off, 64);
-        const double co = __shfl_xor(cs, off, 64);
-        double t, e;
-        bt_two_sum(s, so, t, e);
-        s = t;
-        cs = bt_add(bt_add(cs, co), e);
-      }
-      double t, e;
-      bt_two_sum(b[d.mv_off + row], -s, t, e);
-      const double ri = bt_add(t, bt_add(e, -cs));
-      rr += ri * ri;
-#pragma unroll
-      for (int q = 0; q < NPL; ++q) {
-        double p, ep, u, f;
-        bt_two_prod(ri, a[q], p, ep);
-        bt_two_sum(gs[q], p, u, f);
-        gs[q] = u;
-        gc[q] = bt_add(gc[q], bt_add(ep, f));
-      }
-    }
-    double* pw = part + d.part_off + (int64_t)(bk.row0 / BT_BLOCK_ROWS) * (2 * n + 2);
-#pragma unroll
-    for (int q = 0; q < NPL; ++q) {
-      const int64_t c = lane + 64 * q;
-      if (c < n) {
-        pw[c] = gs[q];
-        pw[n + c] = gc[q];
-      }
-    }
-    if (lane == 0) pw[2 * n] = rr;
+    PAMD_BT_BODY(bt_residual_block, d, bk.row0, A, b, xv, part)
   }
 }
 
-// sum a problem's block partials in a fixed order: one workgroup per problem,
-// 64-column chunks, its 16 wavefronts take the blocks bb = w, w + 16, ... and
-// their sums are combined in wavefront order; out (n-vector pool) and, for
-// the residual, the compensation terms folded in and ||r_i||^2 in scal[prob]
+// Sum a problem's block partials in a fixed order: a workgroup per problem and
+// 64-column chunk, its 16 wavefronts take the blocks bb = w, w + 16, ...
+// (eight partials in flight each) and their sums are combined in wavefront
+// order; out (n-vector pool) and, for the residual, the compensation terms
+// folded in and ||r_i||^2 (the chunk holding column n) in scal[prob].  With one
+// workgroup per problem and a load in flight, 64 problems of up to 780 blocks
+// took 204 us; 15 so.
 constexpr int BT_RED_WAVES = 16;
+constexpr int BT_RED_DEPTH = 8;
 
+template <bool COMP>
 __global__ __launch_bounds__(64 * BT_RED_WAVES) void bt_reduce_kernel(const Desc* __restrict__ D,
                                                                       const double* __restrict__ part,
-                                                                      int compensated, double* __restrict__ out,
+                                                                      double* __restrict__ out,
                                                                       double* __restrict__ scal) {
   __shared__ double rs[BT_RED_WAVES][64];
-  __shared__ double rc[BT_RED_WAVES][64];
+  __shared__ double rc[COMP ? BT_RED_WAVES : 1][64];
   const Desc d = D[blockIdx.x];
   const int64_t n = d.n;
+  const int64_t cb = 64 * (int64_t)blockIdx.y;
+  if (cb >= n + (COMP ? 1 : 0)) return;
   const int64_t nb = pamd_cdiv(d.m, BT_BLOCK_ROWS);
-  const double* p0 = part + d.part_off;
   const int64_t ps = 2 * n + 2;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int64_t cb = 0; cb <= n; cb += 64) {  // the chunk holding column n carries ||r||^2
-    const int64_t c = cb + lane;
-    double s = 0.0, cc = 0.0;
-    if (c < n) {
-      for (int64_t bb = wave; bb < nb; bb += BT_RED_WAVES) {
-        if (compensated) {
-          double t, e;
-          bt_two_sum(s, p0[bb * ps + c], t, e);
-          s = t;
-          cc = bt_add(cc, bt_add(p0[bb * ps + n + c], e));
-        } else {
-          s += p0[bb * ps + c];
-        }
+  const int64_t c = cb + lane;
+  const bool sq = COMP && c == n;
+  const double* p0 = part + d.part_off + (sq ? 2 * n : c);
+  double s = 0.0, cc = 0.0;
+  if (c < n || sq) {
+    for (int64_t b0 = wave; b0 < nb; b0 += BT_RED_WAVES * BT_RED_DEPTH) {
+      double v[BT_RED_DEPTH], w[BT_RED_DEPTH];
+#pragma unroll
+      for (int k = 0; k < BT_RED_DEPTH; ++k) {
+        const int64_t bb = b0 + BT_RED_WAVES * k;
+        v[k] = bb < nb ? p0[bb * ps] : 0.0;
+        w[k] = (COMP && !sq && bb < nb) ? p0[bb * ps + n] : 0.0;
       }
-    } else if (c == n && compensated) {
-      for (int64_t bb = wave; bb < nb; bb += BT_RED_WAVES) s += p0[bb * ps + 2 * n];
-    }
-    rs[wave][lane] = s;
-    rc[wave][lane] = cc;
-    __syncthreads();
-    if (wave == 0) {
-      double S = 0.0, C = 0.0;
-      for (int w = 0; w < BT_RED_WAVES; ++w) {
-        if (compensated && c < n) {
-          double t, e;
-          bt_two_sum(S, rs[w][lane], t, e);
-          S = t;
-          C = bt_add(C, bt_add(rc[w][lane], e));
-        } else {
-          S += rs[w][lane];
-        }
+#pragma unroll
+      for (int k = 0; k < BT_RED_DEPTH; ++k) {
+        if (COMP && !sq)
+          bt_fold(s, cc, v[k], w[k]);
+        else
+          s += v[k];
       }
-      if (c < n) out[d.nv_off + c] = compensated ? bt_add(S, C) : S;
-      else if (c == n && compensated) scal[blockIdx.x] = S;
     }
-    __syncthreads();
+  }
+  rs[wave][lane] = s;
+  if (COMP) rc[wave][lane] = cc;
+  __syncthreads();
+  if (wave == 0 && (c < n || sq)) {
+    double S = 0.0, C = 0.0;
+    for (int w = 0; w < BT_RED_WAVES; ++w) {
+      if (COMP && !sq)
+        bt_fold(S, C, rs[w][lane], rc[w][lane]);
+      else
+        S += rs[w][lane];
+    }
+    if (sq)
+      scal[blockIdx.x] = S;
+    else
+      out[d.nv_off + c] = COMP ? bt_add(S, C) : S;
   }
 }
 
@@ -286,51 +415,58 @@ __global__ __launch_bounds__(256) void bt_trsv_kernel(const Desc* __restrict__ D
   for (int i = threadIdx.x; i < n; i += blockDim.x) v[d.nv_off + i] = xs[i];
 }
 
-// v_i <- M_i^T v_i, M_i = R_i^{-1} (upper triangular) or its transpose
-// (lower), row-major with ld n_i, so that both R^{-1} v and R^{-T} v are a
-// product with a transposed matrix: one workgroup of four wavefronts per
-// problem, each lane owning eight columns, each wavefront every fourth row
-// (two rows' coalesced segments loaded at a time), the wavefronts' column
-// sums added in wavefront order.
-__global__ __launch_bounds__(256) void bt_trmv_kernel(const Desc* __restrict__ D, int lower,
-                                                      const double* __restrict__ Mp, double* __restrict__ v) {
+// y_i = M_i^T x_i, M_i = R_i^{-1} (upper triangular) or its transpose (lower),
+// row-major with ld n_i, so that both R^{-1} x and R^{-T} x are a product with
+// a transposed matrix.  A workgroup takes the 64-column chunks blockIdx.y,
+// blockIdx.y + gridDim.y, ...: a lane per column, each of its 16 wavefronts
+// every 16th row of the chunk's triangle (eight rows in flight), the
+// wavefronts' sums added in wavefront order.  One chunk per workgroup where y
+// is not x (64 problems of up to 512 columns: 11 us, where four wavefronts per
+// problem with two rows in flight took 81); in place a problem's one workgroup
+// takes them all (x is staged first), with the same sums.
+constexpr int BT_MV_WAVES = 16;
+constexpr int BT_MV_DEPTH = 8;
+
+__global__ __launch_bounds__(64 * BT_MV_WAVES) void bt_trmv_kernel(const Desc* __restrict__ D, int lower,
+                                                                   const double* __restrict__ Mp, const double* x,
+                                                                   double* y) {
   __shared__ double xs[BT_MAXN];
-  __shared__ double red[4][BT_MAXN];
+  __shared__ double red[BT_MV_WAVES][64];
   const Desc d = D[blockIdx.x];
   const int n = (int)d.n;
+  if (64 * (int)blockIdx.y >= n) return;
   const double* M = Mp + d.r_off;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) xs[i] = v[d.nv_off + i];
-  __syncthreads();
-  double acc[BT_MAXN / 64];
+  for (int i = threadIdx.x; i < n; i += blockDim.x) xs[i] = x[d.nv_off + i];
+  for (int cb = 64 * (int)blockIdx.y; cb < n; cb += 64 * (int)gridDim.y) {
+    __syncthreads();
+    const int j = cb + lane;
+    // rows of the chunk's triangle
+    const int i_lo = lower ? cb : 0, i_hi = lower ? n : (cb + 64 < n ? cb + 64 : n);
+    double acc = 0.0;
+    for (int i0 = i_lo + wave; i0 < i_hi; i0 += BT_MV_WAVES * BT_MV_DEPTH) {
+      double mv[BT_MV_DEPTH];
 #pragma unroll
-  for (int k = 0; k < BT_MAXN / 64; ++k) acc[k] = 0.0;
-  for (int i0 = wave; i0 < n; i0 += 8) {
-    double mv[2][BT_MAXN / 64];
+      for (int k = 0; k < BT_MV_DEPTH; ++k) {
+        const int i = i0 + BT_MV_WAVES * k;
+        const bool in = i < i_hi && j < n && (lower ? (j <= i) : (j >= i));
+        mv[k] = in ? M[(int64_t)i * n + j] : 0.0;
+      }
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int i = i0 + 4 * h;
-      const double* row = M + (int64_t)(i < n ? i : 0) * n;
-#pragma unroll
-      for (int k = 0; k < BT_MAXN / 64; ++k) {
-        const int j = lane + 64 * k;
-        const bool in = i < n && j < n && (lower ? (j <= i) : (j >= i));
-        mv[h][k] = in ? row[j] : 0.0;
+      for (int k = 0; k < BT_MV_DEPTH; ++k) {
+        const int i = i0 + BT_MV_WAVES * k;
+        acc += mv[k] * (i < i_hi ? xs[i] : 0.0);
       }
     }
+    red[wave][lane] = acc;
+    __syncthreads();
+    if (wave == 0 && j < n) {
+      double t = red[0][lane];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int i = i0 + 4 * h;
-      const double xi = (i < n) ? xs[i] : 0.0;
-#pragma unroll
-      for (int k = 0; k < BT_MAXN / 64; ++k) acc[k] += mv[h][k] * xi;
+      for (int w = 1; w < BT_MV_WAVES; ++w) t += red[w][lane];
+      y[d.nv_off + j] = t;
     }
   }
-#pragma unroll
-  for (int k = 0; k < BT_MAXN / 64; ++k) red[wave][lane + 64 * k] = acc[k];
-  __syncthreads();
-  for (int j = threadIdx.x; j < n; j += blockDim.x)
-    v[d.nv_off + j] = ((red[0][j] + red[1][j]) + red[2][j]) + red[3][j];
 }
 
 __device__ inline double bt_block_dot(const double* a, const double* b, int64_t n, double* red) {
@@ -719,20 +855,32 @@ __global__ __launch_bounds__(256) void bt_trmm_kernel(const Desc* __restrict__ D
 }
 
 // ||A_i||_F^2: a partial per column chunk (rows of A_i), summed in chunk order
-__global__ __launch_bounds__(256) void bt_fro2_partial_kernel(const Desc* __restrict__ D,
-                                                              const SkDesc* __restrict__ S, int64_t nprob,
-                                                              const float* __restrict__ A,
-                                                              double* __restrict__ part) {
-  __shared__ double red[4];
+// One read of A: a chunk is 2048 rows, so a batch has a few chunks per CU, and
+// the bandwidth comes from 1024 threads with eight loads in flight each (2 GB:
+// 1829 -> 780 us against 256 threads with one).
+constexpr int FRO_THREADS = 1024;
+constexpr int FRO_DEPTH = 8;
+
+__global__ __launch_bounds__(FRO_THREADS) void bt_fro2_partial_kernel(const Desc* __restrict__ D,
+                                                                      const SkDesc* __restrict__ S, int64_t nprob,
+                                                                      const float* __restrict__ A,
+                                                                      double* __restrict__ part) {
+  __shared__ double red[FRO_THREADS / 64];
   const int64_t p = bt_find(nprob, blockIdx.x, [&](int64_t q) { return S[q].chunk0; });
   const Desc d = D[p];
   const int64_t c = blockIdx.x - S[p].chunk0;
   const int64_t e0 = c * SK_CHUNK * d.n, e1 = imin64(d.m, (c + 1) * SK_CHUNK) * d.n;
   const float* Ai = A + d.a_off;
   double t = 0.0;
-  for (int64_t e = e0 + threadIdx.x; e < e1; e += blockDim.x) {
-    const double v = (double)Ai[e];
-    t += v * v;
+  for (int64_t e = e0 + threadIdx.x; e < e1; e += FRO_THREADS * FRO_DEPTH) {
+    float v[FRO_DEPTH];
+#pragma unroll
+    for (int k = 0; k < FRO_DEPTH; ++k) {
+      const int64_t i = e + k * FRO_THREADS;
+      v[k] = i < e1 ? Ai[i] : 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k < FRO_DEPTH; ++k) t += (double)v[k] * (double)v[k];
   }
   t = block_sum(t, red);
   if (threadIdx.x == 0) part[blockIdx.x] = t;
@@ -765,12 +913,20 @@ __global__ __launch_bounds__(256) void bt_dot_kernel(const Desc* __restrict__ D,
 static_assert(sizeof(Desc) == sizeof(pamd_ls_desc), "descriptor layout");
 static_assert(sizeof(Blk) == sizeof(pamd_ls_block), "block layout");
 
+// A is streamed (see PAMD_STREAM_BYTES) where the class's blocks, taken at
+// their full width, exceed the Infinity Cache.
+#define PAMD_BT_LAUNCH(KERNEL, NPL, ...)                                       \
+  if (nblk * (NPL) * (int64_t)(BT_BLOCK_ROWS * 64 * sizeof(float)) > PAMD_STREAM_BYTES) \
+    KERNEL<NPL, true><<<grid, threads, 0, st>>>(__VA_ARGS__);                  \
+  else                                                                         \
+    KERNEL<NPL, false><<<grid, threads, 0, st>>>(__VA_ARGS__);
+
 #define PAMD_BT_NPL(KERNEL, NPL, ...)                                          \
   switch (NPL) {                                                               \
-    case 1: KERNEL<1><<<grid, threads, 0, st>>>(__VA_ARGS__); break;           \
-    case 2: KERNEL<2><<<grid, threads, 0, st>>>(__VA_ARGS__); break;           \
-    case 4: KERNEL<4><<<grid, threads, 0, st>>>(__VA_ARGS__); break;           \
-    default: KERNEL<8><<<grid, threads, 0, st>>>(__VA_ARGS__); break;          \
+    case 1: PAMD_BT_LAUNCH(KERNEL, 1, __VA_ARGS__) break;                      \
+    case 2: PAMD_BT_LAUNCH(KERNEL, 2, __VA_ARGS__) break;                      \
+    case 4: PAMD_BT_LAUNCH(KERNEL, 4, __VA_ARGS__) break;                      \
+    default: PAMD_BT_LAUNCH(KERNEL, 8, __VA_ARGS__) break;                     \
   }
 
 static int bt_shape(int npl, int64_t nblk, int waves_per_wg, int blocks_per_wave, unsigned* grid, unsigned* threads) {
@@ -829,8 +985,12 @@ extern "C" int pamd_bt_reduce(int64_t nprob, const pamd_ls_desc* descs, const do
   PAMD_ARG_CHECK(out != nullptr || nprob == 0, 5);
   PAMD_ARG_CHECK(scal != nullptr || !compensated || nprob == 0, 6);
   if (nprob == 0) return PAMD_OK;
-  bt_reduce_kernel<<<(unsigned)nprob, 64 * BT_RED_WAVES, 0, (hipStream_t)stream>>>((const Desc*)descs, part,
-                                                                                  compensated, out, scal);
+  // a chunk of 64 columns each, and column n of the residual's partials
+  const dim3 grid((unsigned)nprob, BT_MAXN / 64 + (compensated ? 1 : 0));
+  if (compensated)
+    bt_reduce_kernel<true><<<grid, 64 * BT_RED_WAVES, 0, (hipStream_t)stream>>>((const Desc*)descs, part, out, scal);
+  else
+    bt_reduce_kernel<false><<<grid, 64 * BT_RED_WAVES, 0, (hipStream_t)stream>>>((const Desc*)descs, part, out, scal);
   PAMD_LAUNCH_CHECK();
   return PAMD_OK;
 }
@@ -859,8 +1019,25 @@ extern "C" int pamd_bt_trmv(int64_t nprob, const pamd_ls_desc* descs, int trans,
   PAMD_ARG_CHECK(v != nullptr || nprob == 0, 6);
   if (nprob == 0) return PAMD_OK;
   // R^{-T} v = Rinv^T v; R^{-1} v = (Rinv^T)^T v
-  bt_trmv_kernel<<<(unsigned)nprob, 256, 0, (hipStream_t)stream>>>((const Desc*)descs, trans ? 0 : 1,
-                                                                   trans ? Rinv : RinvT, v);
+  bt_trmv_kernel<<<(unsigned)nprob, 64 * BT_MV_WAVES, 0, (hipStream_t)stream>>>((const Desc*)descs, trans ? 0 : 1,
+                                                                                trans ? Rinv : RinvT, v, v);
+  PAMD_LAUNCH_CHECK();
+  return PAMD_OK;
+}
+
+extern "C" int pamd_bt_trmv_to(int64_t nprob, const pamd_ls_desc* descs, int trans, const double* Rinv,
+                               const double* RinvT, const double* x, double* y, void* stream) {
+  PAMD_ARG_CHECK(nprob >= 0, 1);
+  PAMD_ARG_CHECK(descs != nullptr || nprob == 0, 2);
+  PAMD_ARG_CHECK(trans == 0 || trans == 1, 3);
+  PAMD_ARG_CHECK(Rinv != nullptr || nprob == 0, 4);
+  PAMD_ARG_CHECK(RinvT != nullptr || nprob == 0, 5);
+  PAMD_ARG_CHECK(x != nullptr || nprob == 0, 6);
+  PAMD_ARG_CHECK((y != nullptr && y != x) || nprob == 0, 7);
+  if (nprob == 0) return PAMD_OK;
+  const dim3 grid((unsigned)nprob, BT_MAXN / 64);
+  bt_trmv_kernel<<<grid, 64 * BT_MV_WAVES, 0, (hipStream_t)stream>>>((const Desc*)descs, trans ? 0 : 1,
+                                                                    trans ? Rinv : RinvT, x, y);
   PAMD_LAUNCH_CHECK();
   return PAMD_OK;
 }
@@ -1029,7 +1206,7 @@ extern "C" int pamd_bt_fro2(int64_t nprob, const pamd_ls_desc* descs, const pamd
   PAMD_ARG_CHECK(out != nullptr || nprob == 0, 7);
   if (nprob == 0) return PAMD_OK;
   hipStream_t st = (hipStream_t)stream;
-  bt_fro2_partial_kernel<<<(unsigned)nchunk, 256, 0, st>>>((const Desc*)descs, (const SkDesc*)sk, nprob, A, part);
+  bt_fro2_partial_kernel<<<(unsigned)nchunk, FRO_THREADS, 0, st>>>((const Desc*)descs, (const SkDesc*)sk, nprob, A, part);
   PAMD_LAUNCH_CHECK();
   bt_fro2_final_kernel<<<(unsigned)nprob, 64, 0, st>>>((const Desc*)descs, (const SkDesc*)sk, part, out);
   PAMD_LAUNCH_CHECK();

@@ -151,6 +151,45 @@ __device__ __forceinline__ float wave_sum(float v) {
   return wave_bcast(v, 63);
 }
 
+// Exchanges halves (QUARTER false: lanes 32-63 of a with lanes 0-31 of b) or
+// 16-lane rows (true: rows 1, 3 of a with rows 0, 2 of b), so that a + b then
+// holds the partial sums of both, each in its own half of the lanes.
+template <bool QUARTER>
+__device__ __forceinline__ void wave_swap(double& a, double& b) {
+  const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  unsigned u[2], v[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const unsigned xi = (unsigned)(x >> (32 * i)), yi = (unsigned)(y >> (32 * i));
+    const auto r = QUARTER ? __builtin_amdgcn_permlane16_swap(xi, yi, false, false)
+                           : __builtin_amdgcn_permlane32_swap(xi, yi, false, false);
+    u[i] = r[0];
+    v[i] = r[1];
+  }
+  a = __longlong_as_double((long long)(((unsigned long long)u[1] << 32) | u[0]));
+  b = __longlong_as_double((long long)(((unsigned long long)v[1] << 32) | v[0]));
+}
+
+// the lane of a row-wise total (wave_sum4) that belongs to value k
+__device__ __forceinline__ int wave_sum4_lane(int k) { return (k & 1) * 32 + (k >> 1) * 16; }
+
+// Full-wave sums of four values at once, each returned to every lane: after
+// two exchanges one register holds all four by 16-lane rows (0, 2, 1, 3), so
+// the four steps within a row serve them together (7 additions, not 24).
+__device__ __forceinline__ void wave_sum4(double (&s)[4]) {
+  wave_swap<false>(s[0], s[1]);
+  wave_swap<false>(s[2], s[3]);
+  double t = s[0] + s[1], u = s[2] + s[3];
+  wave_swap<true>(t, u);
+  t += u;
+  t += dpp_f64<0xb1>(t);
+  t += dpp_f64<0x4e>(t);
+  t += dpp_f64<0x124>(t);
+  t += dpp_f64<0x128>(t);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) s[k] = wave_bcast(t, wave_sum4_lane(k));
+}
+
 __device__ __forceinline__ double wave_max(double v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, PAMD_WAVE));

@@ -312,6 +312,12 @@ class BatchedSPO:
         ops.check(ops.lib().pamd_bt_trmv(B.P, ops._p(B.desc), 1 if trans else 0, ops._p(B.Rinv), ops._p(B.RinvT),
                                          ops._p(v), ops.stream(B.dev)), "pamd_bt_trmv")
 
+    def _trsv_to(self, B, v, out, trans):
+        """out_i = R_i^{-1} v_i (R_i^{-T} v_i), v and out different pools."""
+        ops.check(ops.lib().pamd_bt_trmv_to(B.P, ops._p(B.desc), 1 if trans else 0, ops._p(B.Rinv),
+                                            ops._p(B.RinvT), ops._p(v), ops._p(out), ops.stream(B.dev)),
+                  "pamd_bt_trmv_to")
+
     def _copy(self, B, a, v):
         ops.check(ops.lib().pamd_bt_copy(B.P, ops._p(B.desc), ops._p(a), ops._p(v), ops.stream(B.dev)),
                   "pamd_bt_copy")
@@ -322,17 +328,14 @@ class BatchedSPO:
 
     def refine_step(self, B):
         """x += R^{-1} CG_K(...) on every active problem, then the new residual."""
-        self._copy(B, B.g, B.rhs)
-        self._trsv(B, B.rhs, True)
+        self._trsv_to(B, B.g, B.rhs, True)
         self._cg(B, 0)
         for _ in range(self.cg_iters):
-            self._copy(B, B.p, B.t)
-            self._trsv(B, B.t, False)
-            self.normal(B, B.q)
-            self._trsv(B, B.q, True)
+            self._trsv_to(B, B.p, B.t, False)
+            self.normal(B, B.t)  # the row-block passes have read t when its sums are written
+            self._trsv_to(B, B.t, B.q, True)
             self._cg(B, 1)
-        self._copy(B, B.z, B.t)
-        self._trsv(B, B.t, False)
+        self._trsv_to(B, B.z, B.t, False)
         ops.check(ops.lib().pamd_bt_axpy(B.P, ops._p(B.desc), ops._p(B.state), ops._p(B.x), ops._p(B.t),
                                          ops.stream(B.dev)), "pamd_bt_axpy")
         self.residual(B)
@@ -351,7 +354,6 @@ class BatchedSPO:
         tic = time.perf_counter()
         B = Batch(As, bs, dev, self.sampling_factor)
         self.factor(B, rng)
-        self.residual(B)  # x = 0; also tunes the residual pass
         graph = None
         if use_graph:
             # tune the normal pass outside the capture; nothing in a step
@@ -365,9 +367,11 @@ class BatchedSPO:
                 self.refine_step(B)
                 B.state[1::4] = 1.0
                 self._warm = True
-            # the partials of frozen problems must be their residual's: a
-            # problem skipped by later passes keeps g_i and ||r_i|| this way
-            self.residual(B)
+        # x = 0; also tunes the residual pass.  After the normal pass, for the
+        # partials of frozen problems must be their residual's: a problem
+        # skipped by later passes keeps g_i and ||r_i|| this way
+        self.residual(B)
+        if use_graph:
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
                 self.refine_step(B)
