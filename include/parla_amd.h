@@ -724,6 +724,12 @@ int pamd_split_layout(int npieces, int64_t M, int64_t N, int64_t K, int64_t* kp,
 int pamd_split_bf16(int transpose, int npieces, int64_t rows, int64_t cols, const double* X,
                     int64_t ldx, int64_t rows_out, int64_t kp, uint16_t* pieces,
                     int64_t pstride, void* stream);
+/* Both orientations from one read of X, the same bytes as two calls of
+ * pamd_split_bf16: X's pieces (rows_out x kp) and X^T's (rows_out_t x kp_t). */
+int pamd_split_both_bf16(int npieces, int64_t rows, int64_t cols, const double* X, int64_t ldx,
+                         int64_t rows_out, int64_t kp, uint16_t* pieces, int64_t pstride,
+                         int64_t rows_out_t, int64_t kp_t, uint16_t* pieces_t,
+                         int64_t pstride_t, void* stream);
 /* C[i * lci + j * lcj] = sum_{p+q<npieces} sum_k L_p[i][k] R_q[j][k] for
  * i < M, j < N (lcj = 1: row-major C; lci = 1: C stored transposed); L has
  * mpad rows, R npad rows, both kp columns (pamd_split_layout). */

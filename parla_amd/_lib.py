@@ -110,6 +110,8 @@ SIGNATURES = {
     "pamd_bt_layout": (c_int, [ctypes.POINTER(c_int)] * 5),
     "pamd_split_layout": (c_int, [c_int, c_i64, c_i64, c_i64] + [ctypes.POINTER(c_i64)] * 4),
     "pamd_split_bf16": (c_int, [c_int, c_int, c_i64, c_i64, c_vp, c_i64, c_i64, c_i64, c_vp, c_i64, c_vp]),
+    "pamd_split_both_bf16": (c_int, [c_int, c_i64, c_i64, c_vp, c_i64, c_i64, c_i64, c_vp, c_i64, c_i64, c_i64, c_vp,
+                                     c_i64, c_vp]),
     "pamd_split_gemm_f64": (c_int, [c_int, c_i64, c_i64, c_i64, c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_i64, c_vp,
                                     c_vp]),
     "pamd_bt_sjlt_csr": (c_int, [c_i64, c_vp, c_vp, c_i64, c_int, c_vp, c_vp, c_vp, c_vp, c_vp]),

@@ -85,41 +85,81 @@ __global__ __launch_bounds__(256) void sg_split_rows_kernel(int64_t rows, int64_
   for (int p = 0; p < P; ++p) *reinterpret_cast<uint4*>(pieces + p * pstride + off) = blk_pack(h[p]);
 }
 
-// blocked pieces of X^T (row j of the piece array = column j of X, K = X's
-// rows): a 64 x 64 tile of X transposed through LDS, then each wavefront
-// writes two 16 x 32 blocks
-template <int P>
-__global__ __launch_bounds__(256) void sg_split_t_kernel(int64_t rows, int64_t cols, const double* __restrict__ X,
-                                                         int64_t ldx, int64_t rows_out, int64_t kp,
-                                                         uint16_t* __restrict__ pieces, int64_t pstride) {
-  __shared__ double T[64][65];
-  const int tid = threadIdx.x;
-  const int64_t i0 = (int64_t)blockIdx.x * 64, j0 = (int64_t)blockIdx.y * 64;
+// Blocked pieces of X (rows_out x kp) and of X^T (rows_out_t x kp_t) from one
+// read of X: each wavefront of a workgroup loads a quarter of the rows of a
+// TI x 64 tile (coalesced 512-byte row segments, all in flight), splits every element
+// once and leaves the pieces packed in LDS (W 32-bit words per element, two
+// pieces each); then it writes its row blocks and its share of the transposed
+// ones as whole 1 KiB blocks.  Bound by memory: 8 bytes read and 4 P written
+// per element (8192 x 4096 in two pieces: 90 us; the orientations apart, each
+// with its own read, took 92 + 100).  rows_out = 0 leaves the row pieces out:
+// the transposed split of a right factor, in tiles of 32 rows (twice as many
+// workgroups for a factor of a few hundred columns: 11.6 -> 6.8 us for 266).
+template <int P, int TI, bool STREAM>
+__global__ __launch_bounds__(256) void sg_split_both_kernel(int64_t rows, int64_t cols, const double* __restrict__ X,
+                                                            int64_t ldx, int64_t kp, uint16_t* __restrict__ pieces,
+                                                            int64_t pstride, int64_t rows_out, int64_t rows_out_t,
+                                                            int64_t kp_t, uint16_t* __restrict__ pieces_t,
+                                                            int64_t pstride_t) {
+  constexpr int W = (P + 1) / 2, LD = 68;  // rows of 68 words keep 16-byte reads aligned
+  __shared__ __attribute__((aligned(16))) uint32_t T[W][TI][LD];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t i0 = (int64_t)blockIdx.x * TI, j0 = (int64_t)blockIdx.y * 64;
+  const int64_t j = j0 + lane;
+  constexpr int RW = TI / 4;  // rows of a wavefront
+  double x[RW];
 #pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    const int ii = tid / 64 + 4 * q, jj = tid % 64;
-    const int64_t i = i0 + ii, j = j0 + jj;
-    T[ii][jj] = (i < rows && j < cols) ? X[i * ldx + j] : 0.0;
+  for (int q = 0; q < RW; ++q) {
+    const int64_t i = i0 + RW * wave + q;
+    x[q] = (i < rows && j < cols) ? pamd_load<STREAM>(X + i * ldx + j) : 0.0;
+  }
+#pragma unroll
+  for (int q = 0; q < RW; ++q) {
+    uint16_t h[P];
+    sg_split<P>(x[q], h);
+#pragma unroll
+    for (int w = 0; w < W; ++w)
+      T[w][RW * wave + q][lane] = (uint32_t)h[2 * w] | (2 * w + 1 < P ? (uint32_t)h[(2 * w + 1) % P] << 16 : 0u);
   }
   __syncthreads();
-  const int lane = tid & 63, wave = tid >> 6, r = lane >> 2, c = lane & 3;
+  const int r = lane >> 2, c = lane & 3;
+  // eight consecutive elements of piece p from their packed words
+  auto pick = [](const uint32_t (&e)[8], int p) {
+    uint16_t v[8];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int b = wave * 2 + h;  // block (jr, kr) of the tile: 4 row blocks x 2 K blocks
-    const int jr = b >> 1, kr = b & 1;
-    const int64_t j = j0 + jr * 16 + r;
-    if (j >= rows_out) continue;
-    uint16_t v[P][8];
+    for (int k = 0; k < 8; ++k) v[k] = (uint16_t)(e[k] >> (16 * (p & 1)));
+    return blk_pack(v);
+  };
+  uint32_t e[W][8];
+  // row blocks b: rows 16 (b / 2) + r, K = 32 (b % 2) + 8 c ..
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      uint16_t t[P];
-      sg_split<P>(T[kr * 32 + 8 * c + e][jr * 16 + r], t);
+  for (int b = wave; b < TI / 8; b += 4) {
+    const int ri = 16 * (b >> 1) + r, kj = 32 * (b & 1) + 8 * c;
+    const int64_t i = i0 + ri, k = j0 + kj;
+    if (i < rows_out && k < kp) {
 #pragma unroll
-      for (int p = 0; p < P; ++p) v[p][e] = t[p];
+      for (int w = 0; w < W; ++w)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) e[w][q] = T[w][ri][kj + q];
+      const int64_t off = blk_off(i, k, kp);
+#pragma unroll
+      for (int p = 0; p < P; ++p) *reinterpret_cast<uint4*>(pieces + p * pstride + off) = pick(e[p / 2], p);
     }
-    const int64_t off = blk_off(j, i0 + kr * 32 + 8 * c, kp);
+  }
+  // transposed blocks: columns 16 wave + r as rows, K = rows 32 h + 8 c ..
 #pragma unroll
-    for (int p = 0; p < P; ++p) *reinterpret_cast<uint4*>(pieces + p * pstride + off) = blk_pack(v[p]);
+  for (int h = 0; h < TI / 32; ++h) {
+    const int64_t jt = j0 + 16 * wave + r, kt = i0 + 32 * h + 8 * c;
+    if (jt < rows_out_t && kt < kp_t) {
+#pragma unroll
+      for (int w = 0; w < W; ++w)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) e[w][q] = T[w][32 * h + 8 * c + q][16 * wave + r];
+      const int64_t off = blk_off(jt, kt, kp_t);
+#pragma unroll
+      for (int p = 0; p < P; ++p) *reinterpret_cast<uint4*>(pieces_t + p * pstride_t + off) = pick(e[p / 2], p);
+    }
   }
 }
 
@@ -360,12 +400,59 @@ extern "C" int pamd_split_bf16(int transpose, int npieces, int64_t rows, int64_t
       sg_split_rows_kernel<3><<<grid, 256, 0, st>>>(rows, cols, X, ldx, nblk, kbn, pieces, pstride);
   } else {
     PAMD_ARG_CHECK(pamd_cdiv(rows_out, 64) <= 65535, 7);
-    dim3 grid((unsigned)(kp / 64), (unsigned)pamd_cdiv(rows_out, 64));
+    dim3 grid((unsigned)(kp / 32), (unsigned)pamd_cdiv(rows_out, 64));
     if (npieces == 2)
-      sg_split_t_kernel<2><<<grid, 256, 0, st>>>(rows, cols, X, ldx, rows_out, kp, pieces, pstride);
+      sg_split_both_kernel<2, 32, false><<<grid, 256, 0, st>>>(rows, cols, X, ldx, 0, nullptr, 0, 0, rows_out, kp, pieces,
+                                                              pstride);
     else
-      sg_split_t_kernel<3><<<grid, 256, 0, st>>>(rows, cols, X, ldx, rows_out, kp, pieces, pstride);
+      sg_split_both_kernel<3, 32, false><<<grid, 256, 0, st>>>(rows, cols, X, ldx, 0, nullptr, 0, 0, rows_out, kp, pieces,
+                                                              pstride);
   }
+  PAMD_LAUNCH_CHECK();
+  return PAMD_OK;
+}
+
+extern "C" int pamd_split_both_bf16(int npieces, int64_t rows, int64_t cols, const double* X, int64_t ldx,
+                                    int64_t rows_out, int64_t kp, uint16_t* pieces, int64_t pstride,
+                                    int64_t rows_out_t, int64_t kp_t, uint16_t* pieces_t, int64_t pstride_t,
+                                    void* stream) {
+  PAMD_ARG_CHECK(npieces == 2 || npieces == 3, 1);
+  PAMD_ARG_CHECK(rows >= 0, 2);
+  PAMD_ARG_CHECK(cols >= 0, 3);
+  PAMD_ARG_CHECK(X != nullptr || rows * cols == 0, 4);
+  PAMD_ARG_CHECK(ldx >= cols && ldx >= 1, 5);
+  PAMD_ARG_CHECK(rows_out >= rows && rows_out % 16 == 0, 6);
+  PAMD_ARG_CHECK(kp % SG_KALIGN == 0 && kp >= cols, 7);
+  PAMD_ARG_CHECK(pieces != nullptr, 8);
+  PAMD_ARG_CHECK(pstride >= rows_out * kp && pstride % 8 == 0, 9);
+  PAMD_ARG_CHECK(rows_out_t >= cols && rows_out_t % 16 == 0, 10);
+  PAMD_ARG_CHECK(kp_t % SG_KALIGN == 0 && kp_t >= rows, 11);
+  PAMD_ARG_CHECK(pieces_t != nullptr, 12);
+  PAMD_ARG_CHECK(pstride_t >= rows_out_t * kp_t && pstride_t % 8 == 0, 13);
+  // the tiles cover both arrays, their padding included
+  const int64_t ti = pamd_cdiv(imax64(rows_out, kp_t), 64), tj = pamd_cdiv(imax64(kp, rows_out_t), 64);
+  PAMD_ARG_CHECK(ti < (1LL << 31), 6);
+  PAMD_ARG_CHECK(tj <= 65535, 10);
+  if (ti == 0 || tj == 0) return PAMD_OK;
+  hipStream_t st = (hipStream_t)stream;
+  const dim3 grid((unsigned)ti, (unsigned)tj);
+  // X and its pieces (about as many bytes) pass the Infinity Cache once
+  const bool nt = 2 * rows * cols * (int64_t)sizeof(double) > PAMD_STREAM_BYTES;
+#define SG_BOTH(P, NT)                                                                                        \
+  sg_split_both_kernel<P, 64, NT><<<grid, 256, 0, st>>>(rows, cols, X, ldx, kp, pieces, pstride, rows_out, rows_out_t, \
+                                                    kp_t, pieces_t, pstride_t)
+  if (npieces == 2) {
+    if (nt)
+      SG_BOTH(2, true);
+    else
+      SG_BOTH(2, false);
+  } else {
+    if (nt)
+      SG_BOTH(3, true);
+    else
+      SG_BOTH(3, false);
+  }
+#undef SG_BOTH
   PAMD_LAUNCH_CHECK();
   return PAMD_OK;
 }

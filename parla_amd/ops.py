@@ -985,6 +985,20 @@ def split_bf16(X, npieces, transpose=False, rows_out=None, kp=None):
     return SplitPieces(P, out_rows, K)
 
 
+def split_both_bf16(X, npieces):
+    """(pieces of X, pieces of X^T), as split_bf16 gives them for a left
+    operand in either orientation, from one read of X."""
+    Xc = X if X.stride(-1) == 1 else X.contiguous()
+    rows, cols = Xc.shape
+    kp, kpt = _round_up(max(cols, 1), 64), _round_up(max(rows, 1), 64)
+    ro, rot = _round_up(max(rows, 1), 128), _round_up(max(cols, 1), 128)
+    P = torch.empty((npieces, ro, kp), dtype=torch.uint16, device=X.device)
+    Pt = torch.empty((npieces, rot, kpt), dtype=torch.uint16, device=X.device)
+    check(lib().pamd_split_both_bf16(npieces, rows, cols, _p(Xc), max(Xc.stride(0), cols, 1), ro, kp, _p(P), ro * kp,
+                                     rot, kpt, _p(Pt), rot * kpt, stream(X.device)), "pamd_split_both_bf16")
+    return SplitPieces(P, rows, cols), SplitPieces(Pt, cols, rows)
+
+
 def split_gemm(L, R, out=None, transpose_out=False):
     """C = sum_{p+q<P} L_p R_q^T (M x N, FP64) from SplitPieces L (M x K) and
     R (N x K, its piece array with the layout's npad rows); with

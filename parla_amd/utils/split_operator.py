@@ -26,7 +26,7 @@ class SplitOperator:
             raise ValueError("npieces must be 2 or 3")
         if _parts is None:
             Ad = ops.as_device(A)
-            _parts = (Ad, ops.split_bf16(Ad, npieces), ops.split_bf16(Ad, npieces, transpose=True))
+            _parts = (Ad, *ops.split_both_bf16(Ad, npieces))
         self._parts = _parts
         self.npieces = npieces
         self._transposed = _transposed
