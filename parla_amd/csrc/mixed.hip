@@ -36,13 +36,11 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 constexpr int OZ_CHUNK = 256;       // K rows per exact FP32 accumulation
 constexpr int OZ_MAX_PIECES = 5;
 constexpr int OZ_TM = 128, OZ_TN = 64;
-// 16-row blocks per wavefront: 4 (M) x 2 (N) wavefronts of 32 x 32 outputs.  Four
-// wavefronts of 64 x 32 read less LDS per MFMA but, one per SIMD, hide no
-// latency (1.6x slower at 4096 x 262144 x 1025).
-constexpr int OZ_WAVE_MB = 2;
-constexpr int OZ_THREADS = 64 * 2 * (OZ_TM / (16 * OZ_WAVE_MB));
+// 4 (M) x 2 (N) wavefronts; a workgroup's tile is T row tiles high
+constexpr int OZ_THREADS = 512;
 constexpr int OZ_TARGET_WG = 4096;  // K groups until the grid has about this many workgroups
 constexpr int OZ_BAND = 8;          // row tiles per band of the tile order
+constexpr int OZ_TALL_WG = 1024;    // workgroups from which the tiles are two row tiles high
 
 __device__ __forceinline__ uint16_t bf16_bits_of_int(double a) {
   // a is an integer with |a| <= 256: exact in BF16 (8 significant bits)
@@ -195,9 +193,15 @@ __global__ __launch_bounds__(256) void oz_split_kernel(int64_t m, int64_t n, con
 //                   sum_p 2^(e_cj - 8 - 9p) Q[i, chunk c] . a_p[chunk c, j]
 // and out = scale * sum_g part[g] (groups in order).  Q (rows padded to 128)
 // and the pieces (rows = columns of [A | b], padded to 64) are blocked
-// (blocked.h).  One 512-thread workgroup per 128 x 64 tile and K group.
+// (blocked.h).  One 512-thread workgroup per 128 T x 64 tile and K group.
 //
-// The K steps of 32 stream through LDS in batches of oz_batch(P) steps by
+// Bound by LDS: a wavefront of 32 T x 32 outputs reads 2 T + 2 P blocks a step
+// for 4 T P MFMAs, so where there are enough tiles to fill the chip twice the
+// height halves the reads of the pieces (4096 x 262144 x 1025, P = 4:
+// 10.2 -> 8.8 ms, 1.06 PFLOP/s; three batches in flight instead of two measure
+// 10.0).  The chunks, and so the sums and their order, do not depend on T.
+//
+// The K steps of 32 stream through LDS in batches of oz_batch steps by
 // direct global -> LDS loads, with the 64 chunk exponents of the tile's
 // columns beside each batch.  Direct-to-LDS loads of one wavefront can
 // complete out of issue order, so a partial vmcnt does not say which of them
@@ -207,31 +211,31 @@ __global__ __launch_bounds__(256) void oz_split_kernel(int64_t m, int64_t n, con
 // the batch to all eight wavefronts.  Three buffers keep two batches in
 // flight while one is multiplied.
 // ---------------------------------------------------------------------------
-constexpr int oz_batch(int P) { return P <= 4 ? 2 : 1; }  // three buffers of 8 + 4 P KiB per step fit in LDS
+// three buffers of 8 T + 4 P KiB per step fit in LDS
+constexpr int oz_batch(int P, int T) { return 3 * 2 * (8 * T + 4 * P) <= 150 ? 2 : 1; }
 
-template <int P>
+template <int P, int T>
 struct OzBuf {
-  uint4 blk[oz_batch(P)][OZ_TM / 16 + P * (OZ_TN / 16)][64];
+  uint4 blk[oz_batch(P, T)][T * OZ_TM / 16 + P * (OZ_TN / 16)][64];
   int e[OZ_TN];
 };
 
-template <int P>
-__global__ __launch_bounds__(OZ_THREADS) void oz_gemm_kernel(int64_t kp, int64_t group_chunks, int mtiles,
-                                                             int ntiles, int ngroups,
+template <int P, int T>
+__global__ __launch_bounds__(OZ_THREADS) void oz_gemm_kernel(int64_t kp, int64_t group_chunks, int qblocks,
+                                                             int mtiles, int ntiles, int ngroups,
                                                              const uint16_t* __restrict__ Q,
                                                              const uint16_t* __restrict__ pieces,
                                                              int64_t pstride, const int* __restrict__ exps,
                                                              int64_t lde, int64_t d, int64_t ncols,
                                                              int64_t ncp, double* __restrict__ part) {
-  constexpr int LB = OZ_TM / 16, RB = OZ_TN / 16;  // 1 KiB blocks per K step: Q rows, piece rows
-  constexpr int NBLK = LB + P * RB;
-  constexpr int MB = OZ_WAVE_MB, WM = LB / MB;    // row blocks per wavefront, wavefronts along M
+  constexpr int LB = T * OZ_TM / 16, RB = OZ_TN / 16;  // 1 KiB blocks per K step: Q rows, piece rows
+  constexpr int MB = 2 * T, WM = LB / MB;              // row blocks per wavefront, wavefronts along M
   constexpr int G = 2, NWG = (OZ_THREADS / 64) / G;  // loading groups, wavefronts per group
   static_assert(LB % NWG == 0 && RB % NWG == 0, "row blocks split evenly over a group");
-  constexpr int B = oz_batch(P);
+  constexpr int B = oz_batch(P, T);
   constexpr int CS = OZ_CHUNK / 32;  // K steps per chunk
   static_assert(CS % B == 0, "a batch lies within one chunk");
-  __shared__ OzBuf<P> S[3];
+  __shared__ OzBuf<P, T> S[3];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: block choices are scalar
   const int wm = wave % WM, wn = wave / WM;
@@ -265,14 +269,16 @@ __global__ __launch_bounds__(OZ_THREADS) void oz_gemm_kernel(int64_t kp, int64_t
   // the calling wavefront (of the group owning batch j) loads rows wl,
   // wl + NWG, ... of Q and of every piece for each step of the batch, and
   // wavefront 0 of the group the batch's chunk exponents
-  auto issue = [&](int j, OzBuf<P>& dst) {
+  auto issue = [&](int j, OzBuf<P, T>& dst) {
 #pragma unroll
     for (int u = 0; u < B; ++u) {
       const int64_t kb = kb0 + (int64_t)j * B + u;
 #pragma unroll
       for (int r = 0; r < LB / NWG; ++r) {
         const int rb = wl + NWG * r;
-        blk_load_lds(Qg + (((int64_t)mt * LB + rb) * kbn + kb) * 64, &dst.blk[u][rb][0], lane);
+        // row blocks past Q's last (T = 2) repeat it; their sums are not stored
+        const int qb = T == 1 ? mt * LB + rb : (int)imin64((int64_t)mt * LB + rb, qblocks - 1);
+        blk_load_lds(Qg + ((int64_t)qb * kbn + kb) * 64, &dst.blk[u][rb][0], lane);
       }
 #pragma unroll
       for (int p = 0; p < P; ++p)
@@ -306,7 +312,7 @@ __global__ __launch_bounds__(OZ_THREADS) void oz_gemm_kernel(int64_t kp, int64_t
 
   // batch j from buffer cur; ahead is the buffer read in batch j - 1, which
   // the barrier frees for the owner's loads of batch j + 2
-  auto batch = [&](int j, const OzBuf<P>& cur, OzBuf<P>& ahead) {
+  auto batch = [&](int j, const OzBuf<P, T>& cur, OzBuf<P, T>& ahead) {
     const bool own = (j % G) == grp;
     if (own) __builtin_amdgcn_s_waitcnt(0x3F70);  // vmcnt(0): this batch's blocks and exponents are in
     asm volatile("s_barrier" ::: "memory");
@@ -366,7 +372,7 @@ __global__ __launch_bounds__(OZ_THREADS) void oz_gemm_kernel(int64_t kp, int64_t
     for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int64_t i = (int64_t)mt * OZ_TM + 16 * (MB * wm + mb) + 4 * lk + r;
+        const int64_t i = (int64_t)mt * (T * OZ_TM) + 16 * (MB * wm + mb) + 4 * lk + r;
         const int64_t j = (int64_t)nt * OZ_TN + 32 * wn + 16 * nb + lr;
         if (i < d) w[i * ncp + j] = acc64[mb][nb][r];
       }
@@ -861,20 +867,29 @@ extern "C" int pamd_ozaki_sketch_f64(int64_t d, int64_t m, int64_t ncols, int np
   PAMD_ARG_CHECK(out != nullptr, 11);
   PAMD_ARG_CHECK(ldo >= ncols && ldo >= 1, 12);
   PAMD_ARG_CHECK(workspace != nullptr, 13);
-  const int64_t total = (int64_t)s.mtiles * s.ntiles * s.ngroups;
-  PAMD_ARG_CHECK(total < (1LL << 31), 1);
+  PAMD_ARG_CHECK((int64_t)s.mtiles * s.ntiles * s.ngroups < (1LL << 31), 1);
+  // Two row tiles high where that still gives each CU several workgroups.  us, one against two high: 640 tall
+  // workgroups (20000 x 201, P = 4) 73 / 73; 1024 (262144 x 65) 310 / 289; 1944 (20000 x 513) 321 / 280; 2088
+  // (262144 x 513) P = 2 1655 / 1580, P = 3 2244 / 1907; one piece has few reads to save (1121 / 1220), five do
+  // not fit the registers.
+  const bool tall = npieces >= 2 && npieces <= 4 && (int64_t)pamd_cdiv(s.mtiles, 2) * s.ntiles * s.ngroups >= OZ_TALL_WG;
+  const int mt = tall ? (int)pamd_cdiv(s.mtiles, 2) : s.mtiles;
+  const unsigned total = (unsigned)((int64_t)mt * s.ntiles * s.ngroups);
+  const int qb = (int)(s.mpad / 16);
   hipStream_t st = (hipStream_t)stream;
   double* part = (double*)workspace;
-#define PAMD_OZ(P)                                                                                       \
-  oz_gemm_kernel<P><<<(unsigned)total, OZ_THREADS, 0, st>>>(s.kp, s.group_chunks, s.mtiles, s.ntiles,    \
-                                                            s.ngroups, Q, pieces, pstride, exps, lde, d,  \
-                                                            ncols, s.ncp, part)
-  switch (npieces) {
-    case 1: PAMD_OZ(1); break;
-    case 2: PAMD_OZ(2); break;
-    case 3: PAMD_OZ(3); break;
-    case 4: PAMD_OZ(4); break;
-    default: PAMD_OZ(5); break;
+#define PAMD_OZ(P, T)                                                                                     \
+  oz_gemm_kernel<P, T><<<total, OZ_THREADS, 0, st>>>(s.kp, s.group_chunks, qb, mt, s.ntiles, s.ngroups, Q, pieces, \
+                                                     pstride, exps, lde, d, ncols, s.ncp, part)
+  switch (tall ? 8 + npieces : npieces) {
+    case 1: PAMD_OZ(1, 1); break;
+    case 2: PAMD_OZ(2, 1); break;
+    case 3: PAMD_OZ(3, 1); break;
+    case 4: PAMD_OZ(4, 1); break;
+    case 5: PAMD_OZ(5, 1); break;
+    case 10: PAMD_OZ(2, 2); break;
+    case 11: PAMD_OZ(3, 2); break;
+    default: PAMD_OZ(4, 2); break;
   }
 #undef PAMD_OZ
   PAMD_LAUNCH_CHECK();
