@@ -355,7 +355,7 @@ def main():
     ls_chosen_roof["refinement_steps"] = int(lgc.refinement_steps)
     ls_chosen_roof["cg_iterations"] = int(lgc.inner_iterations)
     ls_chosen_roof["dominant_kernels"] = "normal_pass_kernel + its partial reduction and CG update per CG step " \
-                                         "(three launches), the 200 x 200 triangular solves, potrf_la; see " \
+                                         "(three launches), the 200 x 200 triangular solves, potrf_reg; see " \
                                          "profiles/ls_chosen_20000x200_kernel_stats.md"
 
     # ------------------------------------------------------------- mixed LS

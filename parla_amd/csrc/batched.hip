@@ -13,8 +13,9 @@
 //     only thing the autotuned launch shape changes: results are bit-equal
 //     for every tile choice.  Blocks are grouped by NPL = ceil(n_i / 64) so a
 //     launch is specialised to its row length.
-//   * per-problem kernels (triangular solves with R_i, the CG recurrences):
-//     one workgroup per problem.
+//   * per-problem kernels: the partials' sums and the products with R_i^{-1}
+//     by a workgroup per problem and 64 columns, triangular solves and the CG
+//     recurrences by one workgroup per problem.
 // Nothing here allocates or synchronises with the host, so a whole
 // refinement step can be captured in one HIP graph and replayed.
 #include "common.h"

@@ -16,7 +16,7 @@ n_i <= 512, b_i FP64) is solved the SPO way, all problems at once:
               x_i += R_i^{-1} z_i
           One refinement step (residual, K CG iterations, update) is a fixed
           sequence of batched kernels -- row-block passes over all problems
-          plus one-workgroup-per-problem solves and recurrences -- captured
+          plus each problem's triangular products and recurrences -- captured
           once in a HIP graph and replayed; the host reads the backward errors
           between replays and freezes converged problems.
   tuning  the launch shape of the row-block passes (workgroup size, blocks
