@@ -318,7 +318,7 @@ int pamd_cholqr_stats_f64(int64_t k, const double* G, int64_t ldg, const int* in
  * I + E from two fixed-point steps (error of order ||E||^3), newton = 0 from a
  * second Cholesky factorisation.  stats (4 doubles on the device): min and max
  * |diag R1|, ||Q1^T Q1 - I||_F and the first failing pivot or 0; the result
- * stands if the last is 0 and the norm is at most 1e-2 (newton = 1) or 0.25;
+ * stands if the last is 0 and the norm is at most 1e-4 (newton = 1) or 0.25;
  * otherwise R and z are not meaningful.  Launches only.
  * Replaces la.qr and Q.T @ b_ske at drivers/least_squares.py:311,315. */
 int pamd_sketch_rz_workspace(int64_t d, int64_t n, int64_t* bytes);

@@ -477,7 +477,10 @@ def cholqr2(Y, rounds=2):
     return Q
 
 
-SKETCH_NEWTON_MAX_E = 1e-2  # sketch_rz_cholqr2: second round by Newton while ||Q1^T Q1 - I||_F is below this
+# sketch_rz_cholqr2: second round by Newton while ||Q1^T Q1 - I||_F is below this.  The two steps leave ||E||^3,
+# which at 1e-4 is far below u kappa (E is of order u kappa^2); at 800 x 200 with kappa 1.7e7 and a consistent right-hand
+# side x = R^{-1} z was off by 1.1e-7 with them and stays within 4 u kappa with potrf
+SKETCH_NEWTON_MAX_E = 1e-4
 SKETCH_MAX_E = 0.25         # ... and by potrf below this; beyond, the Gram matrix has lost the sketch's small directions
 
 

@@ -58,6 +58,26 @@ def test_forms_match_householder(ops, d, n, cond, shifted):
     assert la.norm(z - zl) <= tol * la.norm(M[:, n])
 
 
+@pytest.mark.parametrize("cond", [5e6, 1e7, 1.5e7])
+@pytest.mark.parametrize("seed", [1, 2])
+def test_solution_between_the_second_rounds(ops, cond, seed):
+    """One small singular value, so that ||Q1^T Q1 - I|| is 1e-3 to 1e-2: x =
+    R^{-1} z of a consistent system has a backward stable solver's error, a few
+    u kappa (the two fixed-point steps alone are off by ||E||^3)."""
+    d, n = 800, 200
+    print(f"[gpu-sketch-rz] second round cond={cond:g} seed={seed}", flush=True)
+    rng = np.random.default_rng(seed)
+    V = la.qr(rng.standard_normal((n, n)))[0]
+    SA = (rng.standard_normal((d, n)) / np.sqrt(d) * np.r_[np.ones(n - 1), 1.0 / cond]) @ V.T
+    x = rng.standard_normal(n)
+    M = np.hstack([SA, (SA @ x)[:, None]])
+    rz = ops.sketch_rz_cholqr2(torch.from_numpy(M).cuda(), n)
+    assert rz is not None
+    R, z = (t.cpu().numpy() for t in rz)
+    err = la.norm(la.solve_triangular(R, z) - x) / la.norm(x)
+    assert err <= 4 * EPS * np.linalg.cond(SA), err
+
+
 def test_graded_columns_stay_on_the_plain_form(ops):
     """Cholesky is invariant under column scaling, so scales from 1e-9 to 1e9
     do not matter (R1's diagonal spread is 1e18)."""
