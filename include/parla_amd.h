@@ -316,7 +316,9 @@ int pamd_cholqr_stats_f64(int64_t k, const double* G, int64_t ldg, const int* in
  * of S A, or with shifted = 1 by the shifted CholeskyQR3 (for an S A too ill
  * conditioned for the former).  newton = 1 takes the second round's factor of
  * I + E from two fixed-point steps (error of order ||E||^3), newton = 0 from a
- * second Cholesky factorisation.  stats (4 doubles on the device): min and max
+ * second Cholesky factorisation; newton = 2 does the latter without the first
+ * round, which it takes from the workspace as a call with newton = 1 and the
+ * same arguments left it (once: it overwrites part of it).  stats (4 doubles on the device): min and max
  * |diag R1|, ||Q1^T Q1 - I||_F and the first failing pivot or 0; the result
  * stands if the last is 0 and the norm is at most 1e-4 (newton = 1) or 0.25;
  * otherwise R and z are not meaningful.  Launches only.

@@ -184,7 +184,7 @@ extern "C" int pamd_sketch_rz_f64(int64_t d, int64_t n, const double* M, int64_t
   PAMD_ARG_CHECK(M != nullptr, 3);
   PAMD_ARG_CHECK(ldm >= n + 1, 4);
   PAMD_ARG_CHECK(shifted == 0 || shifted == 1, 5);
-  PAMD_ARG_CHECK(newton == 0 || newton == 1, 6);
+  PAMD_ARG_CHECK(newton >= 0 && newton <= 2, 6);
   PAMD_ARG_CHECK(R != nullptr, 7);
   PAMD_ARG_CHECK(ldr >= n, 8);
   PAMD_ARG_CHECK(z != nullptr, 9);
@@ -201,27 +201,30 @@ extern "C" int pamd_sketch_rz_f64(int64_t d, int64_t n, const double* M, int64_t
                   double* C, int64_t ldc) {
     return pamd_gemm_f64(ta, 0, m, nn, k, 1.0, A, lda, B, ldb, 0.0, C, ldc, ws + L.gw, L.gw_bytes, stream);
   };
-  rz_init_kernel<<<(unsigned)pamd_cdiv(d, 256), 256, 0, st>>>(d, n, M, ldm, Q, info);
-  PAMD_LAUNCH_CHECK();
-  const double* Y = M;
-  int64_t ldy = ldm;
-  if (shifted) {
-    double* G0 = ws + L.G0;
-    RZ_TRY(gemm(1, n, n, d, M, ldm, M, ldm, G0, n));
-    rz_shift_kernel<<<1, 256, 0, st>>>(d, n, G0);
+  if (newton != 2) {
+    rz_init_kernel<<<(unsigned)pamd_cdiv(d, 256), 256, 0, st>>>(d, n, M, ldm, Q, info);
     PAMD_LAUNCH_CHECK();
-    RZ_TRY(pamd_potrf_run((int)n, G0, n, info + 2, stream));
-    RZ_TRY(pamd_trsm_strip_run(d, (int)n, G0, n, M, ldm, ws + L.Y, n, ws + L.dinv, stream));
-    Y = ws + L.Y;
-    ldy = n;
+    const double* Y = M;
+    int64_t ldy = ldm;
+    if (shifted) {
+      double* G0 = ws + L.G0;
+      RZ_TRY(gemm(1, n, n, d, M, ldm, M, ldm, G0, n));
+      rz_shift_kernel<<<1, 256, 0, st>>>(d, n, G0);
+      PAMD_LAUNCH_CHECK();
+      RZ_TRY(pamd_potrf_run((int)n, G0, n, info + 2, stream));
+      RZ_TRY(pamd_trsm_strip_run(d, (int)n, G0, n, M, ldm, ws + L.Y, n, ws + L.dinv, stream));
+      Y = ws + L.Y;
+      ldy = n;
+    }
+    RZ_TRY(gemm(1, n, n, d, Y, ldy, Y, ldy, G, n));
+    RZ_TRY(pamd_potrf_run((int)n, G, n, info, stream));
+    RZ_TRY(pamd_trsm_strip_run(d, (int)n, G, n, Y, ldy, Q, n + 1, ws + L.dinv, stream));
+    RZ_TRY(gemm(1, n, n + 1, d, Q, n + 1, Q, n + 1, QtQ, n + 1));
+    rz_newton_kernel<<<eg, 256, 0, st>>>((int)n, QtQ, G, T, ws + L.part);  // T = X = H(E)
+    PAMD_LAUNCH_CHECK();
   }
-  RZ_TRY(gemm(1, n, n, d, Y, ldy, Y, ldy, G, n));
-  RZ_TRY(pamd_potrf_run((int)n, G, n, info, stream));
-  RZ_TRY(pamd_trsm_strip_run(d, (int)n, G, n, Y, ldy, Q, n + 1, ws + L.dinv, stream));
-  RZ_TRY(gemm(1, n, n + 1, d, Q, n + 1, Q, n + 1, QtQ, n + 1));
-  rz_newton_kernel<<<eg, 256, 0, st>>>((int)n, QtQ, G, T, ws + L.part);  // T = X = H(E)
-  PAMD_LAUNCH_CHECK();
-  if (newton) {
+  // the first round stays in the workspace (G = R1, QtQ, the norm's parts) for a second call with newton = 2
+  if (newton == 1) {
     RZ_TRY(gemm(1, n, n, n, T, n, T, n, U, n));
     rz_r2_kernel<<<eg, 256, 0, st>>>((int)n, QtQ, U, T);  // T = R2
     PAMD_LAUNCH_CHECK();
@@ -232,14 +235,14 @@ extern "C" int pamd_sketch_rz_f64(int64_t d, int64_t n, const double* M, int64_t
   }
   rz_stats_kernel<<<1, 256, 0, st>>>((int)n, G, QtQ, (int)eg, ws + L.part, info, z, stats);
   PAMD_LAUNCH_CHECK();
+  RZ_TRY(pamd_trsv_pack_f64(n, T, n, ws + L.tri, stream));
   if (shifted) {
     RZ_TRY(gemm(0, n, n, n, T, n, G, n, U, n));
-    rz_triu_kernel<<<eg, 256, 0, st>>>((int)n, ws + L.G0, n, G);
+    rz_triu_kernel<<<eg, 256, 0, st>>>((int)n, ws + L.G0, n, T);
     PAMD_LAUNCH_CHECK();
-    RZ_TRY(gemm(0, n, n, n, U, n, G, n, R, ldr));
+    RZ_TRY(gemm(0, n, n, n, U, n, T, n, R, ldr));
   } else {
     RZ_TRY(gemm(0, n, n, n, T, n, G, n, R, ldr));
   }
-  RZ_TRY(pamd_trsv_pack_f64(n, T, n, ws + L.tri, stream));
   return pamd_trsv_packed_f64(1, n, ws + L.tri, z, stream);
 }

@@ -484,24 +484,12 @@ SKETCH_NEWTON_MAX_E = 1e-4
 SKETCH_MAX_E = 0.25         # ... and by potrf below this; beyond, the Gram matrix has lost the sketch's small directions
 
 
-def _sketch_rz(M, n, shifted, newton):
-    """One pamd_sketch_rz_f64: (R, z, ||Q1^T Q1 - I||_F), or None when a pivot
-    failed or the norm says that the first round was not good enough (the
-    call's one host read).  The norm alone decides: it is measured on the Q1
-    that was computed, and unlike R1's diagonal it does not depend on the
-    scaling of the columns."""
-    d = M.shape[0]
-    dev = M.device
-    R = torch.empty((n, n), dtype=F64, device=dev)
-    z = torch.empty(n, dtype=F64, device=dev)
-    stats = torch.empty(4, dtype=F64, device=dev)
-    ws = workspace(_query(lib().pamd_sketch_rz_workspace, d, n), dev)
-    check(lib().pamd_sketch_rz_f64(d, n, _p(M), M.stride(0), int(shifted), int(newton), _p(R), n, _p(z), _p(stats),
-                                   _p(ws), stream(dev)), "pamd_sketch_rz_f64")
-    dd = stats.cpu().numpy()
-    if dd[3] != 0 or not np.all(np.isfinite(dd)) or dd[0] <= 0 or dd[2] > SKETCH_MAX_E:
-        return None
-    return R, z, dd[2]
+def _sketch_rz_stands(dd):
+    """Whether the figures of pamd_sketch_rz_f64 say that no pivot failed and
+    the first round was good enough.  The norm alone decides: it is measured on
+    the Q1 that was computed, and unlike R1's diagonal it does not depend on
+    the scaling of the columns."""
+    return dd[3] == 0 and np.all(np.isfinite(dd)) and dd[0] > 0 and dd[2] <= SKETCH_MAX_E
 
 
 SKETCH_RZ_MIN_N, SKETCH_RZ_MAX_N = 64, 1024
@@ -514,17 +502,28 @@ def sketch_rz_cholqr2(M, n, shifted=False):
     Q = Q1 R2^{-1}, which is never formed.  These are a Householder QR's R
     and Q^T S b (R up to the signs of its rows, z with them).  The second
     round is two Newton steps while ||Q1^T Q1 - I||_F <= SKETCH_NEWTON_MAX_E
-    (their error is O(||E||^3)), else potrf.  With ``shifted``, the same on
-    S A R0^{-1} with R0 from the shifted Gram matrix, for kappa(S A) beyond
-    what the Gram matrix of S A holds.  None when S A is too ill-conditioned;
+    (their error is O(||E||^3)), else potrf on the same first round.  With
+    ``shifted``, the same on S A R0^{-1} with R0 from the shifted Gram matrix,
+    for kappa(S A) beyond what the Gram matrix of S A holds.  None when S A is too ill-conditioned;
     M is unmodified."""
     d, ncols = M.shape
     if n < 1 or n > SKETCH_RZ_MAX_N or d < n or ncols != n + 1 or M.stride(1) != 1:
         return None
-    out = _sketch_rz(M, n, shifted, True)
-    if out is not None and out[2] > SKETCH_NEWTON_MAX_E:
-        out = _sketch_rz(M, n, shifted, False)
-    return None if out is None else out[:2]
+    dev = M.device
+    R = torch.empty((n, n), dtype=F64, device=dev)
+    z = torch.empty(n, dtype=F64, device=dev)
+    stats = torch.empty(4, dtype=F64, device=dev)
+    ws = workspace(_query(lib().pamd_sketch_rz_workspace, d, n), dev)
+
+    def figures(newton):
+        check(lib().pamd_sketch_rz_f64(d, n, _p(M), M.stride(0), int(shifted), newton, _p(R), n, _p(z), _p(stats),
+                                       _p(ws), stream(dev)), "pamd_sketch_rz_f64")
+        return stats.cpu().numpy()
+
+    dd = figures(1)
+    if _sketch_rz_stands(dd) and dd[2] > SKETCH_NEWTON_MAX_E:
+        dd = figures(2)
+    return (R, z) if _sketch_rz_stands(dd) else None
 
 
 def sketch_rz_(M, n):

@@ -78,6 +78,31 @@ def test_solution_between_the_second_rounds(ops, cond, seed):
     assert err <= 4 * EPS * np.linalg.cond(SA), err
 
 
+@pytest.mark.parametrize("shifted", [0, 1])
+@pytest.mark.parametrize("d,n", [(120, 64), (700, 209), (1100, 513)])
+def test_second_round_reuses_the_first(ops, d, n, shifted):
+    """newton = 2 gives newton = 0's bits from the workspace that newton = 1
+    left, without reading the sketch again."""
+    print(f"[gpu-sketch-rz] second round only d={d} n={n} shifted={shifted}", flush=True)
+    M = torch.from_numpy(_sketch(d, n, 1e3, 5)).cuda()
+    dev = M.device
+    L, st = ops.lib(), ops.stream(dev)
+
+    def run(A, newton, ws):
+        R, z, stats = (torch.full(s, float("nan"), dtype=torch.float64, device=dev) for s in ((n, n), (n,), (4,)))
+        ops.check(L.pamd_sketch_rz_f64(d, n, ops._p(A), n + 1, shifted, newton, ops._p(R), n, ops._p(z),
+                                       ops._p(stats), ops._p(ws), st), "pamd_sketch_rz_f64")
+        return R, z, stats
+
+    size = ops._query(L.pamd_sketch_rz_workspace, d, n)
+    want = run(M, 0, ops.workspace(size, dev))
+    ws = ops.workspace(size, dev)
+    run(M, 1, ws)
+    got = run(torch.full_like(M, float("nan")), 2, ws)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 def test_graded_columns_stay_on_the_plain_form(ops):
     """Cholesky is invariant under column scaling, so scales from 1e-9 to 1e9
     do not matter (R1's diagonal spread is 1e18)."""
