@@ -26,7 +26,7 @@ constexpr int64_t RZ_MAX_N = 1024;  // the strip solve and the packed triangular
 constexpr int RZ_PARTS = 256;      // workgroups of the ||E|| partial sums
 
 struct RzLayout {
-  int64_t Y, Q, G0, G, QtQ, T, U, dinv, gw, tri, part, info, total;  // offsets in doubles
+  int64_t Q, G0, G, QtQ, T, U, dinv, gw, tri, part, info, total;  // offsets in doubles
   int64_t gw_bytes;
 };
 
@@ -46,8 +46,7 @@ int rz_layout(int64_t d, int64_t n, RzLayout* L) {
     o += rz_round(doubles);
     return at;
   };
-  L->Y = take(d * n);              // S A R0^{-1} of the shifted form
-  L->Q = take(d * (n + 1));        // [Q1 | S b]
+  L->Q = take(d * (n + 1));        // [Q1 | S b]; before, S A R0^{-1} of the shifted form in Q1's place
   L->G0 = take(n * n);             // R0 (shifted form)
   L->G = take(n * n);              // R1
   L->QtQ = take(n * (n + 1));      // [Q1^T Q1 | w]
@@ -212,9 +211,9 @@ extern "C" int pamd_sketch_rz_f64(int64_t d, int64_t n, const double* M, int64_t
       rz_shift_kernel<<<1, 256, 0, st>>>(d, n, G0);
       PAMD_LAUNCH_CHECK();
       RZ_TRY(pamd_potrf_run((int)n, G0, n, info + 2, stream));
-      RZ_TRY(pamd_trsm_strip_run(d, (int)n, G0, n, M, ldm, ws + L.Y, n, ws + L.dinv, stream));
-      Y = ws + L.Y;
-      ldy = n;
+      RZ_TRY(pamd_trsm_strip_run(d, (int)n, G0, n, M, ldm, Q, n + 1, ws + L.dinv, stream));
+      Y = Q;  // the next strip solve is in place: a workgroup holds its 16 rows in LDS before it stores them
+      ldy = n + 1;
     }
     RZ_TRY(gemm(1, n, n, d, Y, ldy, Y, ldy, G, n));
     RZ_TRY(pamd_potrf_run((int)n, G, n, info, stream));
