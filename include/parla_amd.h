@@ -321,7 +321,9 @@ int pamd_cholqr_stats_f64(int64_t k, const double* G, int64_t ldg, const int* in
  * same arguments left it (once: it overwrites part of it).  stats (4 doubles on the device): min and max
  * |diag R1|, ||Q1^T Q1 - I||_F and the first failing pivot or 0; the result
  * stands if the last is 0 and the norm is at most 1e-4 (newton = 1) or 0.25;
- * otherwise R and z are not meaningful.  Launches only.
+ * otherwise z is not meaningful, and neither is R, which after a failed pivot of
+ * the first round is not written (the rest of the work is left out on the
+ * device).  Launches only.
  * Replaces la.qr and Q.T @ b_ske at drivers/least_squares.py:311,315. */
 int pamd_sketch_rz_workspace(int64_t d, int64_t n, int64_t* bytes);
 int pamd_sketch_rz_f64(int64_t d, int64_t n, const double* M, int64_t ldm,

@@ -102,13 +102,16 @@ __device__ __forceinline__ void store_b(double (*Bs)[BN + 1], const double (&r)[
 // grid: (ceil(N/BN), ceil(M/BM), splits).  Slice z covers K range
 // [z*kchunk, min(K, (z+1)*kchunk)).  With splits > 1 the raw product of each
 // slice goes to part[z] (M x N, ld N); otherwise C = alpha*prod + beta*Cin
-// (Cin, ldcin: the input C, which may be C itself).
-template <int TA, int TB, int BM, int BN>
+// (Cin, ldcin: the input C, which may be C itself).  SKIP: nothing is done when
+// *skip is not zero (an instantiation of its own: the test in every product
+// made the power iteration's 1% slower).
+template <int TA, int TB, int BM, int BN, bool SKIP>
 __global__ __launch_bounds__(256) void gemm_f64_kernel(int64_t M, int64_t N, int64_t K, int64_t kchunk,
                                                        double alpha, const double* __restrict__ A, int64_t lda,
                                                        const double* __restrict__ B, int64_t ldb, double beta,
                                                        const double* Cin, int64_t ldcin, double* C, int64_t ldc,
-                                                       double* __restrict__ part) {
+                                                       double* __restrict__ part, const int* __restrict__ skip) {
+  if (SKIP && *skip != 0) return;
   constexpr int IM = BM / 32, JN = BN / 32;  // MFMA blocks per wavefront
   __shared__ double As[GBK][BM + 1];
   __shared__ double Bs[GBK][BN + 1];
@@ -201,8 +204,11 @@ inline int gemm_edge(int64_t d) {
 }
 
 // C = alpha * sum_z part[z] + beta * Cin, summed in slice order.
+template <bool SKIP>
 __global__ void splitk_reduce_kernel(int64_t M, int64_t N, int splits, double alpha, const double* __restrict__ part,
-                                     double beta, const double* Cin, int64_t ldcin, double* C, int64_t ldc) {
+                                     double beta, const double* Cin, int64_t ldcin, double* C, int64_t ldc,
+                                     const int* __restrict__ skip) {
+  if (SKIP && *skip != 0) return;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= M * N) return;
   const int64_t row = idx / N, col = idx % N;
@@ -422,10 +428,13 @@ extern "C" int pamd_gemm_f64(int transA, int transB, int64_t M, int64_t N, int64
 }
 
 // C = alpha op(A) op(B) + beta Cin with the input C read from Cin (which may
-// be C): the library's own out-of-place updates (recursive TRSM) use it.
+// be C): the library's own out-of-place updates (recursive TRSM) use it.  With
+// skip, a device flag that an earlier launch may have set, C is left alone
+// when it is set (transB = 0 only).
 int pamd_gemm_cin_f64(int transA, int transB, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
                       int64_t lda, const double* B, int64_t ldb, double beta, const double* Cin, int64_t ldcin,
-                      double* C, int64_t ldc, void* workspace, int64_t workspace_bytes, void* stream) {
+                      double* C, int64_t ldc, void* workspace, int64_t workspace_bytes, void* stream,
+                      const int* skip) {
   PAMD_ARG_CHECK(transA == 0 || transA == 1, 1);
   PAMD_ARG_CHECK(transB == 0 || transB == 1, 2);
   PAMD_ARG_CHECK(M >= 0, 3);
@@ -438,6 +447,7 @@ int pamd_gemm_cin_f64(int transA, int transB, int64_t M, int64_t N, int64_t K, d
   PAMD_ARG_CHECK(C != nullptr || M * N == 0, 12);
   PAMD_ARG_CHECK(ldc >= N && ldc >= 1, 13);
   PAMD_ARG_CHECK(Cin != nullptr || M * N == 0 || beta == 0.0, 12);
+  PAMD_ARG_CHECK(skip == nullptr || transB == 0, 2);
   PAMD_ARG_CHECK(ldcin >= N && ldcin >= 1, 13);
   if (M == 0 || N == 0) return PAMD_OK;
   hipStream_t st = (hipStream_t)stream;
@@ -449,15 +459,14 @@ int pamd_gemm_cin_f64(int transA, int transB, int64_t M, int64_t N, int64_t K, d
   double* part = splits > 1 ? (double*)workspace : nullptr;
   const int bm = gemm_edge(M), bn = gemm_edge(N);
   dim3 grid((unsigned)pamd_cdiv(N, bn), (unsigned)pamd_cdiv(M, bm), (unsigned)splits);
-#define PAMD_GEMM(TA, TB, BM, BN) \
-  gemm_f64_kernel<TA, TB, BM, BN><<<grid, 256, 0, st>>>(M, N, K, kchunk, alpha, A, lda, B, ldb, beta, Cin, ldcin, \
-                                                        C, ldc, part)
-#define PAMD_GEMM_T(BM, BN)                                  \
-  do {                                                       \
-    if (transA == 0 && transB == 0) PAMD_GEMM(0, 0, BM, BN); \
-    else if (transA == 0) PAMD_GEMM(0, 1, BM, BN);           \
-    else if (transB == 0) PAMD_GEMM(1, 0, BM, BN);           \
-    else PAMD_GEMM(1, 1, BM, BN);                            \
+#define PAMD_GEMM(TA, TB, BM, BN, SKIP) \
+  gemm_f64_kernel<TA, TB, BM, BN, SKIP><<<grid, 256, 0, st>>>(M, N, K, kchunk, alpha, A, lda, B, ldb, beta, Cin, ldcin, \
+                                                        C, ldc, part, skip)
+#define PAMD_GEMM_T(BM, BN)                                                                          \
+  do {                                                                                               \
+    if (transB != 0) transA == 0 ? PAMD_GEMM(0, 1, BM, BN, false) : PAMD_GEMM(1, 1, BM, BN, false);  \
+    else if (skip) transA == 0 ? PAMD_GEMM(0, 0, BM, BN, true) : PAMD_GEMM(1, 0, BM, BN, true);      \
+    else transA == 0 ? PAMD_GEMM(0, 0, BM, BN, false) : PAMD_GEMM(1, 0, BM, BN, false);              \
   } while (0)
   if (bm == 64 && bn == 64) PAMD_GEMM_T(64, 64);
   else if (bm == 64) PAMD_GEMM_T(64, 96);
@@ -468,8 +477,11 @@ int pamd_gemm_cin_f64(int transA, int transB, int64_t M, int64_t N, int64_t K, d
   PAMD_LAUNCH_CHECK();
   if (splits > 1) {
     const int64_t tot = M * N;
-    splitk_reduce_kernel<<<(unsigned)pamd_cdiv(tot, 256), 256, 0, st>>>(M, N, splits, alpha, part, beta, Cin, ldcin,
-                                                                        C, ldc);
+    const unsigned rg = (unsigned)pamd_cdiv(tot, 256);
+    if (skip)
+      splitk_reduce_kernel<true><<<rg, 256, 0, st>>>(M, N, splits, alpha, part, beta, Cin, ldcin, C, ldc, skip);
+    else
+      splitk_reduce_kernel<false><<<rg, 256, 0, st>>>(M, N, splits, alpha, part, beta, Cin, ldcin, C, ldc, nullptr);
     PAMD_LAUNCH_CHECK();
   }
   return PAMD_OK;

@@ -131,7 +131,8 @@ __global__ __launch_bounds__(64) void trsm_dinv_kernel(int k, const double* __re
 __global__ __launch_bounds__(256) void trsm_strip_kernel(int64_t m, int k, const double* __restrict__ Y, int64_t ldy,
                                                          const double* __restrict__ R, int64_t ldr,
                                                          const double* __restrict__ Dinv, double* __restrict__ X,
-                                                         int64_t ldx) {
+                                                         int64_t ldx, const int* __restrict__ skip) {
+  if (skip != nullptr && *skip != 0) return;
   trsm_strip_body(blockIdx.x, m, k, Y, ldy, R, ldr, Dinv, X, ldx);
 }
 
@@ -412,11 +413,12 @@ extern "C" int pamd_trtri_batched_f64(int64_t nprob, int64_t nmax, const int64_t
 #define PAMD_TRSM_MFMA_MAX_K 512
 
 int pamd_trsm_strip_run(int64_t m, int k, const double* R, int64_t ldr, const double* Y, int64_t ldy, double* X,
-                        int64_t ldx, double* dinv, void* stream) {
+                        int64_t ldx, double* dinv, void* stream, const int* skip) {
   hipStream_t st = (hipStream_t)stream;
   trsm_dinv_kernel<<<(unsigned)pamd_cdiv(k, TS_B), 64, 0, st>>>(k, R, ldr, dinv);
   PAMD_LAUNCH_CHECK();
-  trsm_strip_kernel<<<(unsigned)pamd_cdiv(m, TS_B), 256, trsm_strip_lds(k), st>>>(m, k, Y, ldy, R, ldr, dinv, X, ldx);
+  trsm_strip_kernel<<<(unsigned)pamd_cdiv(m, TS_B), 256, trsm_strip_lds(k), st>>>(m, k, Y, ldy, R, ldr, dinv, X, ldx,
+                                                                                         skip);
   PAMD_LAUNCH_CHECK();
   return PAMD_OK;
 }

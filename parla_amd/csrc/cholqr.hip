@@ -15,9 +15,12 @@
 // stands: the failing pivots and ||Q1^T Q1 - I||_F, which measures what the
 // first round lost.
 //
-// With that read, R and z of 400 x 101 / 800 x 201 / 2048 x 513 take 135 / 189
-// / 448 us (Householder: 378 / 806 / 2469); in the shifted form, after the
-// first form has failed, 336 / 488 / 1212.
+// With that read, R and z of 400 x 101 / 800 x 201 / 2048 x 513 take 172 / 227
+// / 495 us (Householder: 408 / 842 / 2498); in the shifted form, after the
+// first form has failed, 345 / 487 / 1095; Householder after both 680 / 1223 /
+// 3343.  A form that fails costs its Gram matrix and the pivots before the
+// failing one; with the rest of its chain run to the end the last two rows were
+// 395 / 539 / 1250 and 754 / 1344 / 3683.
 #include "common.h"
 
 namespace {
@@ -196,9 +199,12 @@ extern "C" int pamd_sketch_rz_f64(int64_t d, int64_t n, const double* M, int64_t
   double *Q = ws + L.Q, *G = ws + L.G, *QtQ = ws + L.QtQ, *T = ws + L.T, *U = ws + L.U;
   int* info = (int*)(ws + L.info);
   const unsigned eg = (unsigned)imin64(RZ_PARTS, pamd_cdiv(n * n, 1024));
+  // Everything after the first round's potrf is left out on the device when a pivot failed there (info[0]), so that a
+  // sketch that has to be factored otherwise pays for its Gram matrix and the pivots before the failing one
   auto gemm = [&](int ta, int64_t m, int64_t nn, int64_t k, const double* A, int64_t lda, const double* B, int64_t ldb,
-                  double* C, int64_t ldc) {
-    return pamd_gemm_f64(ta, 0, m, nn, k, 1.0, A, lda, B, ldb, 0.0, C, ldc, ws + L.gw, L.gw_bytes, stream);
+                  double* C, int64_t ldc, const int* skip) {
+    return pamd_gemm_cin_f64(ta, 0, m, nn, k, 1.0, A, lda, B, ldb, 0.0, C, ldc, C, ldc, ws + L.gw, L.gw_bytes, stream,
+                             skip);
   };
   if (newton != 2) {
     rz_init_kernel<<<(unsigned)pamd_cdiv(d, 256), 256, 0, st>>>(d, n, M, ldm, Q, info);
@@ -207,7 +213,7 @@ extern "C" int pamd_sketch_rz_f64(int64_t d, int64_t n, const double* M, int64_t
     int64_t ldy = ldm;
     if (shifted) {
       double* G0 = ws + L.G0;
-      RZ_TRY(gemm(1, n, n, d, M, ldm, M, ldm, G0, n));
+      RZ_TRY(gemm(1, n, n, d, M, ldm, M, ldm, G0, n, nullptr));
       rz_shift_kernel<<<1, 256, 0, st>>>(d, n, G0);
       PAMD_LAUNCH_CHECK();
       RZ_TRY(pamd_potrf_run((int)n, G0, n, info + 2, stream));
@@ -215,16 +221,16 @@ extern "C" int pamd_sketch_rz_f64(int64_t d, int64_t n, const double* M, int64_t
       Y = Q;  // the next strip solve is in place: a workgroup holds its 16 rows in LDS before it stores them
       ldy = n + 1;
     }
-    RZ_TRY(gemm(1, n, n, d, Y, ldy, Y, ldy, G, n));
+    RZ_TRY(gemm(1, n, n, d, Y, ldy, Y, ldy, G, n, nullptr));
     RZ_TRY(pamd_potrf_run((int)n, G, n, info, stream));
-    RZ_TRY(pamd_trsm_strip_run(d, (int)n, G, n, Y, ldy, Q, n + 1, ws + L.dinv, stream));
-    RZ_TRY(gemm(1, n, n + 1, d, Q, n + 1, Q, n + 1, QtQ, n + 1));
+    RZ_TRY(pamd_trsm_strip_run(d, (int)n, G, n, Y, ldy, Q, n + 1, ws + L.dinv, stream, info));
+    RZ_TRY(gemm(1, n, n + 1, d, Q, n + 1, Q, n + 1, QtQ, n + 1, info));
     rz_newton_kernel<<<eg, 256, 0, st>>>((int)n, QtQ, G, T, ws + L.part);  // T = X = H(E)
     PAMD_LAUNCH_CHECK();
   }
   // the first round stays in the workspace (G = R1, QtQ, the norm's parts) for a second call with newton = 2
   if (newton == 1) {
-    RZ_TRY(gemm(1, n, n, n, T, n, T, n, U, n));
+    RZ_TRY(gemm(1, n, n, n, T, n, T, n, U, n, info));
     rz_r2_kernel<<<eg, 256, 0, st>>>((int)n, QtQ, U, T);  // T = R2
     PAMD_LAUNCH_CHECK();
   } else {
@@ -236,12 +242,12 @@ extern "C" int pamd_sketch_rz_f64(int64_t d, int64_t n, const double* M, int64_t
   PAMD_LAUNCH_CHECK();
   RZ_TRY(pamd_trsv_pack_f64(n, T, n, ws + L.tri, stream));
   if (shifted) {
-    RZ_TRY(gemm(0, n, n, n, T, n, G, n, U, n));
+    RZ_TRY(gemm(0, n, n, n, T, n, G, n, U, n, info));
     rz_triu_kernel<<<eg, 256, 0, st>>>((int)n, ws + L.G0, n, T);
     PAMD_LAUNCH_CHECK();
-    RZ_TRY(gemm(0, n, n, n, U, n, T, n, R, ldr));
+    RZ_TRY(gemm(0, n, n, n, U, n, T, n, R, ldr, info));
   } else {
-    RZ_TRY(gemm(0, n, n, n, T, n, G, n, R, ldr));
+    RZ_TRY(gemm(0, n, n, n, T, n, G, n, R, ldr, info));
   }
   return pamd_trsv_packed_f64(1, n, ws + L.tri, z, stream);
 }

@@ -46,14 +46,16 @@
 // C = alpha op(A) op(B) + beta Cin, the input C read from Cin (blas.hip).
 int pamd_gemm_cin_f64(int transA, int transB, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
                       int64_t lda, const double* B, int64_t ldb, double beta, const double* Cin, int64_t ldcin,
-                      double* C, int64_t ldc, void* workspace, int64_t workspace_bytes, void* stream);
+                      double* C, int64_t ldc, void* workspace, int64_t workspace_bytes, void* stream,
+                      const int* skip = nullptr);
 
 // The Cholesky factorisation and the strip solve X = Y R^{-1} without the
 // entry points' limit of 512 (arguments checked by the caller; chol.hip): any n
-// for potrf, k <= 1024 for the solve (LDS); dinv: ceil(k / 16) * 256 doubles.
+// for potrf, k <= 1024 for the solve (LDS); dinv: ceil(k / 16) * 256 doubles;
+// skip: a device flag (potrf's info) that, when set, leaves X alone.
 int pamd_potrf_run(int n, double* A, int64_t lda, int* info, void* stream);
 int pamd_trsm_strip_run(int64_t m, int k, const double* R, int64_t ldr, const double* Y, int64_t ldy, double* X,
-                        int64_t ldx, double* dinv, void* stream);
+                        int64_t ldx, double* dinv, void* stream, const int* skip = nullptr);
 
 __host__ __device__ static inline int64_t pamd_cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 __host__ __device__ static inline int64_t imin64(int64_t a, int64_t b) { return a < b ? a : b; }

@@ -504,8 +504,8 @@ def sketch_rz_cholqr2(M, n, shifted=False):
     round is two Newton steps while ||Q1^T Q1 - I||_F <= SKETCH_NEWTON_MAX_E
     (their error is O(||E||^3)), else potrf on the same first round.  With
     ``shifted``, the same on S A R0^{-1} with R0 from the shifted Gram matrix,
-    for kappa(S A) beyond what the Gram matrix of S A holds.  None when S A is too ill-conditioned;
-    M is unmodified."""
+    for kappa(S A) beyond what the Gram matrix of S A holds.  None when S A is
+    too ill-conditioned; M is unmodified."""
     d, ncols = M.shape
     if n < 1 or n > SKETCH_RZ_MAX_N or d < n or ncols != n + 1 or M.stride(1) != 1:
         return None
@@ -529,9 +529,12 @@ def sketch_rz_cholqr2(M, n, shifted=False):
 def sketch_rz_(M, n):
     """(R, z = Q^T S b) of a sketch M = [S A | S b] (contiguous; overwritten
     only by the last resort): CholeskyQR2, the shifted CholeskyQR3 when S A is
-    too ill-conditioned for it, Householder (qr_r_) when that fails too or n
-    is out of range.  At n = 64 Householder takes 222 us, CholeskyQR2 110 and,
-    having failed first, the shifted form 265; at n = 32 it is 103, 91 and 219."""
+    too ill-conditioned for it (kappa past about 1e8), Householder (qr_r_) when
+    that fails too (past about 1e12) or n is out of range.  us at n = 64 / 200 /
+    512 / 1024, d = 4 n: Householder 255 / 842 / 2498 / 5254, CholeskyQR2 152 /
+    227 / 495 / 1416, the shifted form after it 298 / 487 / 1095 / 3086,
+    Householder after both 497 / 1223 / 3343 / 7467.  At n = 32 Householder
+    takes 103 and CholeskyQR2 91."""
     if SKETCH_RZ_MIN_N <= n <= SKETCH_RZ_MAX_N:
         for shifted in (False, True):
             rz = sketch_rz_cholqr2(M, n, shifted)

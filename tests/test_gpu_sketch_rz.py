@@ -118,6 +118,21 @@ def test_graded_columns_stay_on_the_plain_form(ops):
     assert la.norm(z - zl) <= 1e-12 * la.norm(M[:, n])
 
 
+@pytest.mark.parametrize("d,n", [(400, 100), (1100, 513)])
+def test_nothing_follows_a_failed_pivot(ops, d, n):
+    """kappa 1e12 is beyond the Gram matrix: its factorisation fails, which the
+    figures report, and the products after it are left out (R is not written)."""
+    print(f"[gpu-sketch-rz] failed pivot d={d} n={n}", flush=True)
+    M = torch.from_numpy(_sketch(d, n, 1e12, 6)).cuda()
+    R = torch.full((n, n), 7.0, dtype=torch.float64, device="cuda")
+    z, stats = torch.empty_like(R[0]), torch.empty(4, dtype=torch.float64, device="cuda")
+    ws = ops.workspace(ops._query(ops.lib().pamd_sketch_rz_workspace, d, n), M.device)
+    ops.check(ops.lib().pamd_sketch_rz_f64(d, n, ops._p(M), n + 1, 0, 1, ops._p(R), n, ops._p(z), ops._p(stats),
+                                           ops._p(ws), ops.stream(M.device)), "pamd_sketch_rz_f64")
+    assert 1 <= float(stats[3]) <= n
+    assert bool((R == 7.0).all())
+
+
 def test_rank_deficient_sketch_ends_at_householder(ops):
     n, d = 100, 400
     M = _sketch(d, n, 10.0, 4)
