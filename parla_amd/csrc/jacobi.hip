@@ -38,6 +38,7 @@
 // positions and the per-sweep counters.  w = 8: narrow blocks spread a sweep
 // over more workgroups at once (17 per round at n = 266).
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 
@@ -117,17 +118,42 @@ __device__ __forceinline__ double rsq_nr(double x) {
 // a'.b' = 0, from al = a.a, be = b.b, ga = a.b; |theta| <= pi / 4.  With d = be -
 // al, g = 2 ga, h = sqrt(d^2 + g^2): cos 2 theta = |d| / h, so c^2 = (1 + |d| / h)
 // / 2 and s = sign(d) g / (2 h c): two reciprocal square roots in a row and no
-// division (the step is a chain of latencies).  The identity unless rot.
-__device__ __forceinline__ void jac_rotation(bool rot, double al, double be, double ga, double& c, double& s,
+// division (the step is a chain of latencies).  The identity unless rot.  h2 =
+// d^2 + g^2 (d and g may share any factor).
+__device__ __forceinline__ void jac_rotation(bool rot, double d, double g, double h2, double& c, double& s,
                                              double& t) {
-  const double d = be - al, g = 2.0 * ga;
-  const double r = rsq_nr(fma(d, d, g * g));  // 1 / h
+  const double r = rsq_nr(h2);                // 1 / h
   const double c2 = fma(0.5 * fabs(d), r, 0.5);
   const double w = rsq_nr(c2);                // 1 / c
-  const double ss = copysign(0.5 * g, d < 0.0 ? -ga : ga) * r * w;
+  const double ss = copysign(0.5 * g, d < 0.0 ? -g : g) * r * w;
   c = rot ? c2 * w : 1.0;
   s = rot ? ss : 0.0;
   t = rot ? ss * w : 0.0;
+}
+
+// Squared lengths whose products and squares (h^2 is of fourth order in the
+// lengths) keep to FP64's range, down to what cancels in a round; 0 is a zero
+// column.  Outside, h^2 loses its last bits or overflows, and c, s would not be
+// a rotation.
+__device__ __forceinline__ bool jac_in_range(double al) { return !(al > 0x1p480 || (al > 0.0 && al < 0x1p-400)); }
+
+// The slow path for a round with columns outside that (1e-60 .. 1e72 in
+// length): whether the pair is to be rotated, with al, be and ga scaled by a
+// power of two where their products do not fit, and d, g by the one that makes
+// the larger of them about 1, with their h^2.
+__device__ __forceinline__ bool jac_wide(double al, double be, double ga, double tol2, double& d, double& g,
+                                         double& h2) {
+  d = be - al;
+  g = 2.0 * ga;
+  const double p = al * be;
+  int e = (p > 0x1p-800 && p < 0x1p1000) ? 0 : -__builtin_amdgcn_frexp_exp(fmax(al, be));
+  const double c = ldexp(ga, e);
+  const bool rot = c * c > tol2 * (ldexp(al, e) * ldexp(be, e));
+  e = -__builtin_amdgcn_frexp_exp(fmax(fabs(d), fabs(g)));
+  d = ldexp(d, e);
+  g = ldexp(g, e);
+  h2 = fma(d, d, g * g);
+  return rot;
 }
 
 // One round of sweep `sweep`: workgroup k orthogonalises block pair k (P = 16
@@ -215,47 +241,66 @@ __global__ __launch_bounds__(JAC_THREADS) void jac_round_kernel(int m, int nb, i
     int e = q ? q : JAC_P - 1, f = q ? JAC_P - 1 - q : 0;
     const double tol2 = tol * tol;
     bool rotated = false;
+    const bool wide = __any(!jac_in_range(G[lr][lr]));
     double* J0 = &Jm[2 * p][0];
     double* J1 = &Jm[2 * p + 1][0];
-    for (int t = 0; t < JAC_P - 1; ++t) {
-      double *Ga = &G[a][0], *Gb = &G[b][0];
-      const double alq = G[e][e], beq = G[f][f], gaq = G[e][f];
-      const double alp = Ga[a], bep = Gb[b], gap = Ga[b];
-      const double gae = Ga[e], gaf = Ga[f], gbe = Gb[e], gbf = Gb[f];
-      const double j0e = J0[e], j0f = J0[f], j1e = J1[e], j1f = J1[f];
-      __builtin_amdgcn_sched_barrier(0);  // every read under way before the first is waited for
-      const bool rq = gaq * gaq > tol2 * (alq * beq);
-      if (__any(rq)) {
-        double cp, sp, tp, cq, sq, tq;
-        jac_rotation(gap * gap > tol2 * (alp * bep), alp, bep, gap, cp, sp, tp);
-        jac_rotation(rq, alq, beq, gaq, cq, sq, tq);
-        rotated = true;
-        // rows (a, b) by p's rotation, then columns (e, f) by q's
-        const double rae = cp * gae - sp * gbe, raf = cp * gaf - sp * gbf;
-        const double rbe = sp * gae + cp * gbe, rbf = sp * gaf + cp * gbf;
-        double nae = cq * rae - sq * raf, naf = sq * rae + cq * raf;
-        double nbe = cq * rbe - sq * rbf, nbf = sq * rbe + cq * rbf;
-        if (p == q && tp != 0.0) {  // the pair's own block: al - t ga, be + t ga, orthogonal
-          nae = fma(-tp, gap, alp);
-          nbf = fma(tp, gap, bep);
-          naf = nbe = 0.0;
+    auto steps = [&](auto WIDE) {
+      for (int t = 0; t < JAC_P - 1; ++t) {
+        double *Ga = &G[a][0], *Gb = &G[b][0];
+        const double alq = G[e][e], beq = G[f][f], gaq = G[e][f];
+        const double alp = Ga[a], bep = Gb[b], gap = Ga[b];
+        const double gae = Ga[e], gaf = Ga[f], gbe = Gb[e], gbf = Gb[f];
+        const double j0e = J0[e], j0f = J0[f], j1e = J1[e], j1f = J1[f];
+        __builtin_amdgcn_sched_barrier(0);  // every read under way before the first is waited for
+        double dp, gp, hp, dq, gq, hq;
+        bool rp, rq;
+        if constexpr (WIDE.value) {
+          rp = jac_wide(alp, bep, gap, tol2, dp, gp, hp);
+          rq = jac_wide(alq, beq, gaq, tol2, dq, gq, hq);
+        } else {
+          rq = gaq * gaq > tol2 * (alq * beq);
         }
-        PAMD_WAVE_SYNC();
-        Ga[e] = nae;
-        Ga[f] = naf;
-        Gb[e] = nbe;
-        Gb[f] = nbf;
-        J0[e] = cq * j0e - sq * j0f;
-        J0[f] = sq * j0e + cq * j0f;
-        J1[e] = cq * j1e - sq * j1f;
-        J1[f] = sq * j1e + cq * j1f;
-        PAMD_WAVE_SYNC();
+        if (__any(rq)) {
+          double cp, sp, tp, cq, sq, tq;
+          if constexpr (!WIDE.value) {
+            rp = gap * gap > tol2 * (alp * bep);
+            dp = bep - alp, gp = 2.0 * gap, hp = fma(dp, dp, gp * gp);
+            dq = beq - alq, gq = 2.0 * gaq, hq = fma(dq, dq, gq * gq);
+          }
+          jac_rotation(rp, dp, gp, hp, cp, sp, tp);
+          jac_rotation(rq, dq, gq, hq, cq, sq, tq);
+          rotated = true;
+          // rows (a, b) by p's rotation, then columns (e, f) by q's
+          const double rae = cp * gae - sp * gbe, raf = cp * gaf - sp * gbf;
+          const double rbe = sp * gae + cp * gbe, rbf = sp * gaf + cp * gbf;
+          double nae = cq * rae - sq * raf, naf = sq * rae + cq * raf;
+          double nbe = cq * rbe - sq * rbf, nbf = sq * rbe + cq * rbf;
+          if (p == q && tp != 0.0) {  // the pair's own block: al - t ga, be + t ga, orthogonal
+            nae = fma(-tp, gap, alp);
+            nbf = fma(tp, gap, bep);
+            naf = nbe = 0.0;
+          }
+          PAMD_WAVE_SYNC();
+          Ga[e] = nae;
+          Ga[f] = naf;
+          Gb[e] = nbe;
+          Gb[f] = nbf;
+          J0[e] = cq * j0e - sq * j0f;
+          J0[f] = sq * j0e + cq * j0f;
+          J1[e] = cq * j1e - sq * j1f;
+          J1[f] = sq * j1e + cq * j1f;
+          PAMD_WAVE_SYNC();
+        }
+        a = p ? (a == JAC_P - 2 ? 0 : a + 1) : a;
+        b = b == JAC_P - 2 ? 0 : b + 1;
+        e = q ? (e == JAC_P - 2 ? 0 : e + 1) : e;
+        f = f == JAC_P - 2 ? 0 : f + 1;
       }
-      a = p ? (a == JAC_P - 2 ? 0 : a + 1) : a;
-      b = b == JAC_P - 2 ? 0 : b + 1;
-      e = q ? (e == JAC_P - 2 ? 0 : e + 1) : e;
-      f = f == JAC_P - 2 ? 0 : f + 1;
-    }
+    };
+    if (wide)
+      steps(std::true_type{});
+    else
+      steps(std::false_type{});
     const bool r = __any(rotated);
     if (lane == 0) any = r;
   }

@@ -54,6 +54,24 @@ def test_graded_columns_keep_relative_accuracy(ops):
     assert np.max(np.abs(s - scale) / scale) <= 200 * EPS * n
 
 
+@pytest.mark.parametrize("scale", [[1e80, 1e50, 1e20, 1.0], [1e76], [1e-74], [1e-78], [1e-80], [1e70, 1e-70]])
+def test_rotations_over_a_wide_range(ops, scale):
+    """Column lengths far from 1, alone and side by side: the accumulated
+    rotation is one (the squared lengths stay inside FP64, their products'
+    squares do not), and so are the singular vectors that do not need lengths
+    whose squares underflow."""
+    print(f"[gpu-jacobi-rounds] scale {scale}", flush=True)
+    m, n = 24, 16
+    A = np.random.default_rng(0).standard_normal((m, n)) * np.resize(np.asarray(scale), n)
+    U, s, Vt = (t.cpu().numpy() for t in ops.svd_jacobi(torch.from_numpy(A).cuda()))
+    tol = 50 * EPS * max(m, 16)
+    assert np.linalg.norm(Vt @ Vt.T - np.eye(n)) <= tol * n
+    if min(scale) >= 1e-70:
+        assert np.linalg.norm(U.T @ U - np.eye(n)) <= tol * n
+        ref = np.linalg.svd(A, compute_uv=False)
+        assert abs(s[0] - ref[0]) <= tol * ref[0]
+
+
 def test_orthogonal_columns_are_left_alone(ops):
     n = 40
     A = np.zeros((n + 3, n))
