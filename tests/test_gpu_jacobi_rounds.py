@@ -40,18 +40,52 @@ def test_round_edges(ops, m, n):
     assert np.linalg.norm(U * s @ Vt - A) <= tol * np.linalg.norm(A)
 
 
-def test_graded_columns_keep_relative_accuracy(ops):
-    """Columns scaled from 1 to 1e-14: sigma = D-scaled, well conditioned
-    after scaling, so every singular value has relative accuracy."""
-    n = 48
+def _singular_values_extended(A):
+    """One-sided Jacobi in extended precision (64 bits): relative accuracy of order 1e-19 times the condition
+    number of A's columns scaled to unit length."""
+    W = A.astype(np.longdouble)
+    n = W.shape[1]
+    tol = 16 * np.finfo(np.longdouble).eps
+    for _ in range(40):
+        rotated = False
+        for p in range(n - 1):
+            for q in range(p + 1, n):
+                al, be, ga = W[:, p] @ W[:, p], W[:, q] @ W[:, q], W[:, p] @ W[:, q]
+                if abs(ga) <= tol * np.sqrt(al * be):
+                    continue
+                rotated = True
+                zeta = (be - al) / (2 * ga)
+                t = (1 if zeta >= 0 else -1) / (abs(zeta) + np.sqrt(1 + zeta * zeta))
+                c = 1 / np.sqrt(1 + t * t)
+                W[:, p], W[:, q] = c * W[:, p] - c * t * W[:, q], c * t * W[:, p] + c * W[:, q]
+        if not rotated:
+            return np.sort(np.sqrt((W * W).sum(0)))[::-1].astype(np.float64)
+    raise AssertionError("no convergence")
+
+
+@pytest.mark.parametrize("m,n,order", [(57, 48, "permuted"), (57, 48, "descending"), (57, 48, "ascending"),
+                                       (24, 16, "permuted")])
+def test_graded_columns_keep_relative_accuracy(ops, m, n, order):
+    """Gaussian columns scaled from 1 to 1e-14: every pair is rotated, and as
+    the columns are well conditioned once scaled to unit length, one-sided
+    Jacobi determines every singular value to high relative accuracy (Demmel
+    and Veselic 1992)."""
+    print(f"[gpu-jacobi-rounds] graded {m} x {n} {order}", flush=True)
     rng = np.random.default_rng(2)
-    Q = np.linalg.qr(rng.standard_normal((n + 9, n)))[0]
-    # orthogonal columns times a diagonal, mixed by a unit upper triangle close to I
+    G = rng.standard_normal((m, n))
     scale = np.logspace(0, -14, n)
-    A = Q * scale
-    perm = rng.permutation(n)
-    s = ops.svd_jacobi(torch.from_numpy(np.ascontiguousarray(A[:, perm])).cuda())[1].cpu().numpy()
-    assert np.max(np.abs(s - scale) / scale) <= 200 * EPS * n
+    scale = {"permuted": rng.permutation(scale), "descending": scale, "ascending": scale[::-1]}[order]
+    A = G * scale
+    C = np.abs((A.T @ A) / np.outer(np.linalg.norm(A, axis=0), np.linalg.norm(A, axis=0)) - np.eye(n))
+    assert np.median(C) > 1e-2                  # the angles are far above the rotation threshold m eps
+    U, s, Vt = (t.cpu().numpy() for t in ops.svd_jacobi(torch.from_numpy(np.ascontiguousarray(A)).cuda()))
+    ref = _singular_values_extended(A)
+    # one-sided Jacobi: a few rounding errors per round and column, times the scaled condition number
+    kappa = np.linalg.cond(G / np.linalg.norm(G, axis=0))
+    assert np.max(np.abs(s - ref) / ref) <= n * EPS * kappa
+    tol = 50 * EPS * max(m, 16)
+    assert np.linalg.norm(U.T @ U - np.eye(n)) <= tol * n
+    assert np.linalg.norm(Vt @ Vt.T - np.eye(n)) <= tol * n
 
 
 @pytest.mark.parametrize("scale", [[1e80, 1e50, 1e20, 1.0], [1e76], [1e-74], [1e-78], [1e-80], [1e70, 1e-70]])
