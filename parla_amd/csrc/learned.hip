@@ -118,13 +118,19 @@ __global__ __launch_bounds__(MLP_THREADS) void mlp_fwd_kernel(int64_t rows, cons
 //   H2  (rows x units) = H1 W2, dH2 -> right operand of dW2
 //   dH1 (rows x units) = dH2 W2^T   -> right operand of dW1
 // and only dH2 passes through LDS, to become dH1's left operand.  dW2, dW1 and
-// the bias gradients stay in registers over the wavefront's tiles.
+// the bias gradients stay in registers over the wavefront's tiles, with more
+// than BW_TILES of them (LONG) over that many; then the eight wavefronts' are
+// added and the workgroup goes on in FP64, so that no FP32 sum runs over more
+// than 256 rows and eight terms however many rows there are (2^24 equal rows:
+// the largest relative error of an entry 1.2e-4 without, 3.9e-6 with; LONG on
+// every call would add 2 us to the 44 of 65536 rows).
 // ---------------------------------------------------------------------------
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int BW_WAVES = 8;
 constexpr int BW_THREADS = 64 * BW_WAVES;
 constexpr int BW_MAX_GRID = 256;  // one workgroup per CU; further rows are looped over
+constexpr int BW_TILES = 16;      // tiles of 16 rows per wavefront that are summed in FP32
 
 inline int64_t bw_grid(int64_t rows) {
   return imax64(1, imin64(BW_MAX_GRID, pamd_cdiv(rows, 16 * BW_WAVES)));
@@ -143,6 +149,7 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v + dpp_f32<0x128>(v);
 }
 
+template <bool LONG>
 __global__ __launch_bounds__(BW_THREADS) void mlp_bwd_kernel(int64_t rows, double inv_total,
                                                              const float* __restrict__ X, int64_t ldx,
                                                              const float* __restrict__ t,
@@ -150,7 +157,8 @@ __global__ __launch_bounds__(BW_THREADS) void mlp_bwd_kernel(int64_t rows, doubl
                                                              const float* __restrict__ bias,
                                                              float* __restrict__ part) {
   __shared__ BwLds s;
-  __shared__ float sum[MLP_NPARAM + 1];
+  __shared__ float sum[MLP_NPARAM + 1];                // the wavefronts' sums over up to BW_TILES tiles each
+  __shared__ double tot[LONG ? MLP_NPARAM + 1 : 1];    // the sums before those
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int wave = tid >> 6;
   const uint16_t* wb2 = wb + MLP_IN * MLP_H;
@@ -165,7 +173,10 @@ __global__ __launch_bounds__(BW_THREADS) void mlp_bwd_kernel(int64_t rows, doubl
     s.w2[hi][lo][l] = u;
     s.w2t[hi][lo][l] = v;
   }
-  for (int e = tid; e <= MLP_NPARAM; e += BW_THREADS) sum[e] = 0.f;
+  for (int e = tid; e <= MLP_NPARAM; e += BW_THREADS) {
+    sum[e] = 0.f;
+    if (LONG) tot[e] = 0.0;
+  }
   // this lane's weights: W1[4 q + g][16 i + c], the biases by unit
   float w1[4][4], b1n[4], b2n[4], w3n[4];
   f4 b1t[4];
@@ -183,17 +194,61 @@ __global__ __launch_bounds__(BW_THREADS) void mlp_bwd_kernel(int64_t rows, doubl
   __syncthreads();
 
   f4 dw2[4][4], dw1[4];
-  float db1[4], db2[4], dw3[4], db3 = 0.f, loss = 0.f;
+  float db1[4], db2[4], dw3[4], db3, loss;
+  auto clear = [&] {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < 4; ++i) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) dw2[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-    dw1[i] = f4{0.f, 0.f, 0.f, 0.f};
-    db1[i] = db2[i] = dw3[i] = 0.f;
-  }
+      for (int j = 0; j < 4; ++j) dw2[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+      dw1[i] = f4{0.f, 0.f, 0.f, 0.f};
+      db1[i] = db2[i] = dw3[i] = 0.f;
+    }
+    db3 = loss = 0.f;
+  };
+  // the registers of the workgroup's wavefronts to sum, wavefront after wavefront
+  auto add_up = [&] {
+    // the bias sums over the four row groups; db3 and the loss are the same in a row group's lanes
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      db1[i] += __shfl_xor(db1[i], 16, 64);
+      db1[i] += __shfl_xor(db1[i], 32, 64);
+      db2[i] += __shfl_xor(db2[i], 16, 64);
+      db2[i] += __shfl_xor(db2[i], 32, 64);
+      dw3[i] += __shfl_xor(dw3[i], 16, 64);
+      dw3[i] += __shfl_xor(dw3[i], 32, 64);
+    }
+    db3 += __shfl_xor(db3, 16, 64);
+    db3 += __shfl_xor(db3, 32, 64);
+    loss += __shfl_xor(loss, 16, 64);
+    loss += __shfl_xor(loss, 32, 64);
+    for (int w = 0; w < BW_WAVES; ++w) {
+      __syncthreads();
+      if (w != wave) continue;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) sum[OFF_W2 + (16 * i + 4 * g + r) * MLP_H + 16 * j + c] += dw2[i][j][r];
+          sum[OFF_W1 + (4 * g + r) * MLP_H + 16 * i + c] += dw1[i][r];
+        }
+        if (g == 0) {
+          sum[OFF_B1 + 16 * i + c] += db1[i];
+          sum[OFF_B2 + 16 * i + c] += db2[i];
+          sum[OFF_W3 + 16 * i + c] += dw3[i];
+        }
+      }
+      if (lane == 0) {
+        sum[OFF_B3] += db3;
+        sum[MLP_NPARAM] += loss;
+      }
+    }
+    __syncthreads();
+  };
+  clear();
   float(*T)[MLP_H + 4] = s.dh2[wave];
-  for (int64_t r0 = ((int64_t)blockIdx.x * BW_WAVES + wave) * 16; r0 < rows;
-       r0 += (int64_t)gridDim.x * BW_WAVES * 16) {
+  const int64_t step = (int64_t)gridDim.x * BW_WAVES * 16;
+  auto tile = [&](int64_t r0) {
     float x[4], xt[4], tr[4];  // X[c][4 q + g], X[4 g + r][c], t[4 g + r] (rows past the end: zero)
     const bool in = r0 + c < rows;
 #pragma unroll
@@ -295,47 +350,28 @@ __global__ __launch_bounds__(BW_THREADS) void mlp_bwd_kernel(int64_t rows, doubl
     for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int i = 0; i < 4; ++i) dw1[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(xt[r], d1[i][r], dw1[i], 0, 0, 0);
-  }
-  // the bias sums over the four row groups; db3 and the loss are the same in a row group's lanes
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    db1[i] += __shfl_xor(db1[i], 16, 64);
-    db1[i] += __shfl_xor(db1[i], 32, 64);
-    db2[i] += __shfl_xor(db2[i], 16, 64);
-    db2[i] += __shfl_xor(db2[i], 32, 64);
-    dw3[i] += __shfl_xor(dw3[i], 16, 64);
-    dw3[i] += __shfl_xor(dw3[i], 32, 64);
-  }
-  db3 += __shfl_xor(db3, 16, 64);
-  db3 += __shfl_xor(db3, 32, 64);
-  loss += __shfl_xor(loss, 16, 64);
-  loss += __shfl_xor(loss, 32, 64);
-  // the workgroup's sums, wavefront after wavefront
-  for (int w = 0; w < BW_WAVES; ++w) {
-    __syncthreads();
-    if (w != wave) continue;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sum[OFF_W2 + (16 * i + 4 * g + r) * MLP_H + 16 * j + c] += dw2[i][j][r];
-        sum[OFF_W1 + (4 * g + r) * MLP_H + 16 * i + c] += dw1[i][r];
+  };
+  const int64_t first = ((int64_t)blockIdx.x * BW_WAVES + wave) * 16;
+  if constexpr (LONG) {
+    // as many rounds for every wavefront (some of the last one past the end), for the barriers of add_up
+    const int rounds = (int)pamd_cdiv(imax64(0, rows - (int64_t)blockIdx.x * BW_WAVES * 16), step);
+    for (int it = 0; it < rounds; ++it) {
+      if (it && it % BW_TILES == 0) {
+        add_up();
+        clear();
+        for (int e = tid; e <= MLP_NPARAM; e += BW_THREADS) {  // seen by the others after the next add_up's barrier
+          tot[e] += (double)sum[e];
+          sum[e] = 0.f;
+        }
       }
-      if (g == 0) {
-        sum[OFF_B1 + 16 * i + c] += db1[i];
-        sum[OFF_B2 + 16 * i + c] += db2[i];
-        sum[OFF_W3 + 16 * i + c] += dw3[i];
-      }
+      if (first + it * step < rows) tile(first + it * step);
     }
-    if (lane == 0) {
-      sum[OFF_B3] += db3;
-      sum[MLP_NPARAM] += loss;
-    }
+  } else {
+    for (int64_t r0 = first; r0 < rows; r0 += step) tile(r0);
   }
-  __syncthreads();
+  add_up();
   float* out = part + (int64_t)blockIdx.x * (MLP_NPARAM + 1);
-  for (int e = tid; e <= MLP_NPARAM; e += BW_THREADS) out[e] = sum[e];
+  for (int e = tid; e <= MLP_NPARAM; e += BW_THREADS) out[e] = LONG ? (float)(tot[e] + (double)sum[e]) : sum[e];
 }
 
 // grad[e] = the workgroups' sums in FP64: 64 entries per workgroup, its four
@@ -455,7 +491,11 @@ extern "C" int pamd_mlp_bwd(int64_t rows, int64_t rows_total, const float* X, in
   hipStream_t st = (hipStream_t)stream;
   const int64_t nblk = bw_grid(rows);
   float* part = (float*)workspace;
-  mlp_bwd_kernel<<<(unsigned)nblk, BW_THREADS, 0, st>>>(rows, 1.0 / (double)rows_total, X, ldx, t, wb, bias, part);
+  const double inv = 1.0 / (double)rows_total;
+  if (rows > nblk * BW_WAVES * 16 * BW_TILES)
+    mlp_bwd_kernel<true><<<(unsigned)nblk, BW_THREADS, 0, st>>>(rows, inv, X, ldx, t, wb, bias, part);
+  else
+    mlp_bwd_kernel<false><<<(unsigned)nblk, BW_THREADS, 0, st>>>(rows, inv, X, ldx, t, wb, bias, part);
   PAMD_LAUNCH_CHECK();
   mlp_reduce_kernel<<<(unsigned)pamd_cdiv(MLP_NPARAM + 1, 64), 256, 0, st>>>((int)nblk, part, grad);
   PAMD_LAUNCH_CHECK();
