@@ -308,7 +308,8 @@ class BatchedSPO:
                                            ops.stream(B.dev)), "pamd_bt_reduce")
 
     def _trsv(self, B, v, trans):
-        """v_i <- R_i^{-1} v_i (R_i^{-T} v_i), as products with R_i^{-1} (formed in factor)."""
+        """v_i <- R_i^{-1} v_i (R_i^{-T} v_i), as products with R_i^{-1} (formed in factor): the in-place form,
+        which the refinement does not need (_trsv_to)."""
         ops.check(ops.lib().pamd_bt_trmv(B.P, ops._p(B.desc), 1 if trans else 0, ops._p(B.Rinv), ops._p(B.RinvT),
                                          ops._p(v), ops.stream(B.dev)), "pamd_bt_trmv")
 
@@ -359,17 +360,21 @@ class BatchedSPO:
             # tune the normal pass outside the capture; nothing in a step
             # allocates or synchronises.  The first call also runs one step
             # with every problem frozen (every pass skips them, x stays) so
-            # that each kernel has been launched once before the capture.
+            # that each kernel has been launched once before the capture; the
+            # residual pass before it, so that its launch shapes are timed
+            # with the problems active.
             self._copy(B, B.p, B.t)
             self.normal(B, B.q)
             if not self._warm:
+                self.residual(B)
                 B.state[1::4] = 0.0
                 self.refine_step(B)
                 B.state[1::4] = 1.0
                 self._warm = True
-        # x = 0; also tunes the residual pass.  After the normal pass, for the
-        # partials of frozen problems must be their residual's: a problem
-        # skipped by later passes keeps g_i and ||r_i|| this way
+        # x = 0 (chooses the residual's launch shapes where they are not known
+        # yet).  After the normal pass, for the partials of frozen problems
+        # must be their residual's: a problem skipped by later passes keeps g_i
+        # and ||r_i|| this way
         self.residual(B)
         if use_graph:
             graph = torch.cuda.CUDAGraph()

@@ -106,3 +106,33 @@ def test_triangular_products_in_and_out_of_place(batch, trans):
         T, t = (M.T if trans else M), B.vec(B.t, i).cpu().numpy()
         bound = (M.shape[0] + 2) * U * (np.abs(T) @ np.abs(t))
         assert (np.abs(B.vec(y, i).cpu().numpy() - T @ t) <= 2 * bound).all(), M.shape
+
+
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_launch_shapes_are_timed_on_active_problems(use_graph):
+    """Every shape that a fresh solver's first call, and a second call with
+    other sizes, puts into its cache was timed with all problems active."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import parla_amd.drivers.batched_ls as bl
+    print("[bt-passes] launch shapes", use_graph, flush=True)
+    solver = bl.BatchedSPO()
+    inner, misses = solver._pass, []
+
+    def spy(B, kind):
+        if torch.cuda.is_current_stream_capturing():
+            known = set(solver.tuner.cache)
+            inner(B, kind)
+            assert known == set(solver.tuner.cache)
+            return
+        active, known = bool((B.state[1::4] == 1).all()), set(solver.tuner.cache)
+        inner(B, kind)
+        misses.extend((kind, key, active) for key in set(solver.tuner.cache) - known)
+
+    solver._pass = spy
+    rng = np.random.default_rng(4)
+    for shapes in ([(900, 40), (1500, 100), (2000, 200)], [(3000, 300), (700, 30)]):
+        As = [rng.standard_normal(s).astype(np.float32) for s in shapes]
+        solver(As, [rng.standard_normal(s[0]) for s in shapes], 1e-10, 1, use_graph=use_graph)
+    assert {k for k, _, _ in misses} == {"normal", "residual"}
+    assert all(active for _, _, active in misses), misses
