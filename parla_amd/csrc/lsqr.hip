@@ -54,21 +54,30 @@ struct LsqrConst {
 // scratch (<= 64 KiB of dynamic LDS)
 constexpr int64_t LSQR_LDS_MAX_N = 1900;
 
-// Pass workgroups of lsqr_waves(n) wavefronts, one wavefront per row at a time:
+// Pass workgroups of lsqr_shape's wavefronts, one wavefront per row at a time:
 // as wide as the register tile of 4 * NPL doubles per lane allows, since a
 // workgroup leaves one partial for the reduction to read.
 __host__ __device__ inline int lsqr_npl(int64_t n) {
   return n <= 64 ? 1 : n <= 128 ? 2 : n <= 256 ? 4 : n <= 512 ? 8 : n <= 1024 ? 16 : 0;
 }
-// wavefronts over the rows of A: one per 4 rows, at most 4096 (16 per CU; one
-// workgroup each)
-__host__ __device__ inline int64_t lsqr_total_waves(int64_t m) { return imax64(1, imin64(4096, pamd_cdiv(m, 4))); }
-__host__ __device__ inline int lsqr_waves(int64_t n) {
+struct LsqrShape {
+  int waves, grid;
+};
+// One wavefront per 4 rows of A, at most 4096 (16 per CU).  Rows of 513..1024
+// columns leave the widest partials in the most workgroups (8 wavefronts each):
+// where the one-workgroup tail sums them (packed false) and they would be more
+// than 128, a wavefront takes 16 rows, and 4 make a workgroup while 8 would be
+// fewer workgroups than CUs.  us per iteration without R, one wavefront per 4
+// rows against that: 3000 x 800 28.4 / 30.3, 8000 x 600 39.6 / 35.4, 16000 x
+// 1000 96 / 63, 40000 x 800 105 / 93.  Narrower and wider rows gain from 4 rows
+// there too (60000 x 500 103 -> 62, 8000 x 1500 408 -> 241).
+__host__ __device__ inline LsqrShape lsqr_shape(int64_t m, int64_t n, bool packed) {
   const int npl = lsqr_npl(n);
-  return (npl >= 1 && npl <= 8) ? 16 : (npl == 16 ? 8 : 4);
-}
-__host__ __device__ inline int lsqr_grid(int64_t m, int64_t n) {
-  return (int)pamd_cdiv(lsqr_total_waves(m), lsqr_waves(n));
+  const bool few = npl == 16 && !packed && m > 4096;
+  const int64_t total = imax64(1, imin64(4096, pamd_cdiv(m, few ? 16 : 4)));
+  int waves = (npl >= 1 && npl <= 8) ? 16 : (npl == 16 ? 8 : 4);
+  if (few && pamd_cdiv(total, waves) < 256) waves = 4;
+  return LsqrShape{waves, (int)pamd_cdiv(total, waves)};
 }
 
 // The packed path (R given, n <= TP_MAX_N): R is packed once per solve
@@ -82,7 +91,7 @@ struct LsqrLayout {
 
 __host__ __device__ inline LsqrLayout lsqr_layout(int64_t m, int64_t n) {
   LsqrLayout L;
-  const int G = lsqr_grid(m, n);
+  const int G = lsqr_shape(m, n, true).grid;  // the other rule's is at most this
   L.st = 0;
   L.u = 64;
   L.v = L.u + m + n;
@@ -105,7 +114,7 @@ __host__ __device__ inline LsqrLayout lsqr_layout(int64_t m, int64_t n) {
 // ---------------------------------------------------------------------------
 // NPL = columns per lane held in registers (n <= 64 * NPL); NPL = 0: any n,
 // the row is read twice (the second read hits cache, so not streamed).  WAVES wavefronts per
-// workgroup (lsqr_waves); the workgroup's partial of A^T u' is the sum of its
+// workgroup (lsqr_shape); the workgroup's partial of A^T u' is the sum of its
 // wavefronts' in wavefront order.
 template <int NPL, int WAVES, bool STREAM>
 __global__ __launch_bounds__(64 * WAVES) void lsqr_pass_kernel(LsqrConst K, const double* __restrict__ A,
@@ -877,8 +886,8 @@ int launch_pass(const LsqrConst& K, const double* A, double* ws, hipStream_t st)
   const int npl = lsqr_npl(K.n);
   const bool stream = K.m * K.n * (int64_t)sizeof(double) > PAMD_STREAM_BYTES;
 #define PAMD_PASS(NPL, WAVES)                                                             \
-  stream ? lsqr_pass_kernel<NPL, WAVES, true><<<K.grid, 64 * WAVES, 0, st>>>(K, A, ws)    \
-         : lsqr_pass_kernel<NPL, WAVES, false><<<K.grid, 64 * WAVES, 0, st>>>(K, A, ws)
+  (stream ? lsqr_pass_kernel<NPL, WAVES, true><<<K.grid, 64 * WAVES, 0, st>>>(K, A, ws)   \
+          : lsqr_pass_kernel<NPL, WAVES, false><<<K.grid, 64 * WAVES, 0, st>>>(K, A, ws))
   if (npl == 1)
     PAMD_PASS(1, 16);
   else if (npl == 2)
@@ -888,7 +897,7 @@ int launch_pass(const LsqrConst& K, const double* A, double* ws, hipStream_t st)
   else if (npl == 8)
     PAMD_PASS(8, 16);
   else if (npl == 16)
-    PAMD_PASS(16, 8);
+    lsqr_shape(K.m, K.n, K.packed).waves == 8 ? PAMD_PASS(16, 8) : PAMD_PASS(16, 4);
   else
     lsqr_pass_kernel<0, 4, false><<<K.grid, 256, 0, st>>>(K, A, ws);
 #undef PAMD_PASS
@@ -967,9 +976,9 @@ int lsqr_start(const pamd_lsqr_problem* prob, double* x, double* var, double* ar
   K.has_r = P.R != nullptr;
   K.calc_var = P.calc_var != 0;
   K.has_x0 = P.x0 != nullptr;
-  K.grid = lsqr_grid(P.m, P.n);
   K.ldr = P.ldr;
   K.packed = K.has_r && lsqr_packed(P.n);
+  K.grid = lsqr_shape(P.m, P.n, K.packed).grid;
   K.xs_global = (K.has_r && P.n > LSQR_LDS_MAX_N) ? 1 : 0;
   double* ws = (double*)workspace;
   shmem = (size_t)(K.has_r ? ((K.xs_global ? 0 : P.n) + TRSV_SCRATCH_DOUBLES) : 1) * sizeof(double);

@@ -80,3 +80,17 @@ def test_lsqr_normal_and_residual_passes(ops, m, n):
     assert float((r - rr).norm()) <= tol
     assert float((gr - A.t() @ rr).norm()) <= tol * float(A.norm()) * 4
     assert abs(float(rss.item()) - float(rr.square().sum())) <= 4 * tol * float(rr.norm()) + 64 * EPS * float(rss.item())
+
+
+@pytest.mark.parametrize("m,n", [(4096, 513), (4097, 513), (16384, 1024), (32640, 700), (32641, 700), (65537, 600)])
+@pytest.mark.parametrize("sqrt_delta", [0.0, 0.3])
+def test_lsqr_pass_shapes_without_r(ops, m, n, sqrt_delta):
+    """The first iteration without R where the rule for 513..1024 columns
+    changes its workgroups, with and without lifted rows."""
+    print(f"[gpu-passes] lsqr shape {m} x {n} delta={sqrt_delta}", flush=True)
+    A, b = _randn(m, n), _randn(m, seed=1)
+    x, _, _, res = ops.lsqr_run(A, b, sqrt_delta=sqrt_delta, atol=0.0, btol=0.0, conlim=0.0, iter_lim=1)
+    g = A.t() @ b
+    v = g / g.norm()
+    ref = (g @ v) / ((A @ v).square().sum() + sqrt_delta ** 2) * v
+    assert float((x - ref).norm()) <= 64 * EPS * (m + n) * float(ref.norm())
