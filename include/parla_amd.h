@@ -556,12 +556,17 @@ int pamd_sample_rows_f64(int64_t m, const double* p, int64_t d, uint64_t seed,
 
 /* Batched potrf / trtri: problem i is the n[i] x n[i] matrix (ld n[i]) at
  * element offset off[i] of the pool (n and off are device arrays; n[i] <= 512
- * for potrf, nmax = max n[i]).  One workgroup per problem (per column for
- * trtri), one launch for the whole batch; info[i] as pamd_potrf_upper_f64.
+ * for potrf).  potrf: the launches that problems of up to nmax = max n[i] rows
+ * need, or without nmax those for 512 rows (the same bits; for a batch of small
+ * problems most of the time).  trtri: a workgroup per column, one launch (nmax
+ * = max n[i]).  info[i] as pamd_potrf_upper_f64.
  * The factorisations behind the per-problem CholeskyQR of a batch of
  * sketches (drivers/least_squares.py:311, one problem per call there). */
 int pamd_potrf_batched_f64(int64_t nprob, const int64_t* n, const int64_t* off,
                            double* pool, int* info, void* stream);
+int pamd_potrf_batched_nmax_f64(int64_t nprob, int64_t nmax, const int64_t* n,
+                                const int64_t* off, double* pool, int* info,
+                                void* stream);
 int pamd_trtri_batched_f64(int64_t nprob, int64_t nmax, const int64_t* n,
                            const int64_t* off, const double* R, double* Rinv,
                            double* RinvT, void* stream);  /* RinvT: the transposes, or NULL */

@@ -251,8 +251,8 @@ class BatchedSPO:
 
         def round_(G, r, shifted, update):
             ops.check(L.pamd_bt_gram(P, D, S, tot["tiles"], shifted, ops._p(Y), ops._p(G), st), "pamd_bt_gram")
-            ops.check(L.pamd_potrf_batched_f64(P, ops._p(B.n_dev), ops._p(B.roff_dev), ops._p(G),
-                                               ops._p(info[r * P:(r + 1) * P]), st), "pamd_potrf_batched_f64")
+            ops.check(L.pamd_potrf_batched_nmax_f64(P, nmax, ops._p(B.n_dev), ops._p(B.roff_dev), ops._p(G),
+                                                    ops._p(info[r * P:(r + 1) * P]), st), "pamd_potrf_batched_nmax_f64")
             if update:
                 ops.check(L.pamd_bt_trsm(P, D, S, tot["strips"], tot["dblk"], nmax, ops._p(G), ops._p(dinv),
                                          ops._p(Y), st), "pamd_bt_trsm")

@@ -88,3 +88,34 @@ def test_potrf_batched_mixed_sizes(ops):
         assert inf[i] == fail.get(i, 0)
         if i not in fail:
             _check(host[off[i]:off[i + 1]].reshape(n, n), Gs[i], n)
+
+
+@pytest.mark.parametrize("ns", [[0, 1, 16, 128], [129, 128, 5], [208, 130, 0, 208], [209, 3], [336, 337, 128, 129, 210],
+                                [512, 1, 465, 400, 209, 208], [512] * 3])
+def test_potrf_batched_with_the_largest_size(ops, ns):
+    """The form that is given the largest size launches the steps it needs and
+    gives the bits of the other one, failing pivots included."""
+    print(f"[gpu-potrf] batched ns={ns}", flush=True)
+    rng = np.random.default_rng(len(ns))
+    Gs = [_gram(n, rng, 2) if n else np.zeros((0, 0)) for n in ns]
+    if ns[0] > 200:
+        Gs[0][180, 180] = -1.0
+    off = np.concatenate([[0], np.cumsum([n * n for n in ns])])
+    start = torch.from_numpy(np.concatenate([np.triu(G).reshape(-1) for G in Gs])).cuda()
+    nv, od = torch.tensor(ns, dtype=torch.int64, device="cuda"), torch.from_numpy(off[:-1].copy()).cuda()
+    L, st, out = ops.lib(), ops.stream(start.device), []
+    for nmax in (None, max(ns)):
+        pool, info = start.clone(), torch.full((len(ns),), 7, dtype=torch.int32, device="cuda")
+        if nmax is None:
+            ops.check(L.pamd_potrf_batched_f64(len(ns), ops._p(nv), ops._p(od), ops._p(pool), ops._p(info), st),
+                      "pamd_potrf_batched_f64")
+        else:
+            ops.check(L.pamd_potrf_batched_nmax_f64(len(ns), nmax, ops._p(nv), ops._p(od), ops._p(pool),
+                                                    ops._p(info), st), "pamd_potrf_batched_nmax_f64")
+        out.append((pool, info))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    for i, n in enumerate(ns):
+        bad = 181 if i == 0 and ns[0] > 200 else 0
+        assert int(out[0][1][i]) == bad
+        if not bad:
+            _check(out[0][0][off[i]:off[i + 1]].reshape(n, n).cpu().numpy(), Gs[i], n)
