@@ -166,7 +166,10 @@ def nrm2(x):
     x = x.contiguous()
     out = torch.empty(1, dtype=F64, device=x.device)
     n = x.numel()
-    if n > (1 << 15):  # long vectors: one partial per workgroup (one workgroup: 16 us at 131072, two launches: 7)
+    # long vectors: one partial per workgroup.  A call takes 7.5 us up to n = 50000 and 12.5 at 100000 with one
+    # workgroup (bound by the host, then by the kernel: 16 us at 131072), 12.5 with the two launches, which take 6 on
+    # the device, and their scratch
+    if n > 100000:
         ws = workspace(_query(lib().pamd_nrm2_workspace, n), x.device)
         check(lib().pamd_nrm2_large_f64(n, _p(x), _p(out), _p(ws), stream(x.device)), "pamd_nrm2_large_f64")
         return out

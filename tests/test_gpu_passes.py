@@ -43,7 +43,7 @@ def test_gemv(ops, m, n):
     assert float((ops.gemv(A, y, trans=True) - A.t() @ y).norm()) <= 8 * EPS * m * scale * float(y.norm()) * np.sqrt(n)
 
 
-@pytest.mark.parametrize("n", [1, 1024, 8191, 8192, 8193, 32768, 32769, 100001, 36_000_000])
+@pytest.mark.parametrize("n", [1, 1024, 8191, 8192, 8193, 32768, 32769, 100000, 100001, 36_000_000])
 def test_nrm2(ops, n):
     print(f"[gpu-passes] nrm2 {n}", flush=True)
     sys.stdout.flush()
