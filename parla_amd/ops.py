@@ -6,6 +6,7 @@ allocator.  torch is used for memory and streams only; all arithmetic happens
 in libparla_amd.so.
 """
 import ctypes
+import math
 
 import numpy as np
 import torch
@@ -486,15 +487,6 @@ def cholqr2(Y, rounds=2):
 SKETCH_NEWTON_MAX_E = 1e-4
 SKETCH_MAX_E = 0.25         # ... and by potrf below this; beyond, the Gram matrix has lost the sketch's small directions
 
-
-def _sketch_rz_stands(dd):
-    """Whether the figures of pamd_sketch_rz_f64 say that no pivot failed and
-    the first round was good enough.  The norm alone decides: it is measured on
-    the Q1 that was computed, and unlike R1's diagonal it does not depend on
-    the scaling of the columns."""
-    return dd[3] == 0 and np.all(np.isfinite(dd)) and dd[0] > 0 and dd[2] <= SKETCH_MAX_E
-
-
 SKETCH_RZ_MIN_N, SKETCH_RZ_MAX_N = 64, 1024
 
 
@@ -518,15 +510,18 @@ def sketch_rz_cholqr2(M, n, shifted=False):
     stats = torch.empty(4, dtype=F64, device=dev)
     ws = workspace(_query(lib().pamd_sketch_rz_workspace, d, n), dev)
 
-    def figures(newton):
+    def run(newton):  # whether the result stands, and ||Q1^T Q1 - I||_F
         check(lib().pamd_sketch_rz_f64(d, n, _p(M), M.stride(0), int(shifted), newton, _p(R), n, _p(z), _p(stats),
                                        _p(ws), stream(dev)), "pamd_sketch_rz_f64")
-        return stats.cpu().numpy()
+        lo, hi, e, pivot = stats.tolist()
+        # the norm alone decides: it is measured on the Q1 that was computed,
+        # and unlike R1's diagonal it does not depend on the columns' scaling
+        return pivot == 0 and lo > 0 and math.isfinite(hi) and e <= SKETCH_MAX_E, e
 
-    dd = figures(1)
-    if _sketch_rz_stands(dd) and dd[2] > SKETCH_NEWTON_MAX_E:
-        dd = figures(2)
-    return (R, z) if _sketch_rz_stands(dd) else None
+    ok, e = run(1)
+    if ok and e > SKETCH_NEWTON_MAX_E:
+        ok, _ = run(2)
+    return (R, z) if ok else None
 
 
 def sketch_rz_(M, n):
