@@ -871,8 +871,13 @@ extern "C" int pamd_ozaki_sketch_f64(int64_t d, int64_t m, int64_t ncols, int np
   // Two row tiles high where that still gives each CU several workgroups.  us, one against two high: 640 tall
   // workgroups (20000 x 201, P = 4) 73 / 73; 1024 (262144 x 65) 310 / 289; 1944 (20000 x 513) 321 / 280; 2088
   // (262144 x 513) P = 2 1655 / 1580, P = 3 2244 / 1907; one piece has few reads to save (1121 / 1220), five do
-  // not fit the registers.
-  const bool tall = npieces >= 2 && npieces <= 4 && (int64_t)pamd_cdiv(s.mtiles, 2) * s.ntiles * s.ngroups >= OZ_TALL_WG;
+  // not fit the registers.  An odd number of row tiles leaves half a tall tile empty, which the saved reads outweigh
+  // from 5 row tiles; with two pieces 5 gain, 7 lose, and 9 and more gain.  P = 2, then 4: d = 300 (200000 x 65) 200 /
+  // 217, 256 / 261; d = 600 (150000 x 151) 217 / 209, 284 / 259; d = 896 (262144 x 225) 429 / 452, 648 / 602; d = 1100
+  // (100000 x 276) 275 / 250, 395 / 351.
+  const bool filled = s.mtiles % 2 == 0 || s.mtiles >= (npieces == 2 ? 9 : 5);
+  const bool tall = npieces >= 2 && npieces <= 4 && filled &&
+                    (int64_t)pamd_cdiv(s.mtiles, 2) * s.ntiles * s.ngroups >= OZ_TALL_WG;
   const int mt = tall ? (int)pamd_cdiv(s.mtiles, 2) : s.mtiles;
   const unsigned total = (unsigned)((int64_t)mt * s.ntiles * s.ngroups);
   const int qb = (int)(s.mpad / 16);

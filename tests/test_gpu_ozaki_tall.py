@@ -1,6 +1,7 @@
 """The exact BF16 sketch product in tiles of two row tiles: bit for bit the
 integer chunk sums added in FP64 in the documented order, with an odd number of
-row tiles (the last tile half empty) and an even one."""
+row tiles (the last tile half empty: 9, and 5 with more than two pieces; one
+high below) and an even one."""
 import numpy as np
 import pytest
 import torch
@@ -11,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("P", [2, 3, 4])
-@pytest.mark.parametrize("d,n", [(300, 500), (200, 1000)])
+@pytest.mark.parametrize("d,n", [(300, 500), (200, 1000), (600, 400), (1100, 250)])
 def test_tall_tiles_exact(P, d, n):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
