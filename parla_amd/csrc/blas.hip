@@ -287,15 +287,20 @@ __global__ __launch_bounds__(256) void gemv_n_kernel(int64_t m, int64_t n, doubl
   if (SPLIT ? threadIdx.x == 0 : lane == 0) y[row] = (beta == 0.0) ? alpha * s : alpha * s + beta * y[row];
 }
 
-// Column block of 64 (lanes) x row slice (grid.y); 4 waves split the rows,
-// eight rows in flight each.  With part != NULL, slice sums go to
-// part[slice * n + col].
-template <bool STREAM>
+// Column block of 64 (lanes) x row slice (grid.y); 4 waves split the rows, U
+// rows in flight each.  With part != NULL, slice sums go to part[slice * n +
+// col].  U = 8 where the rows are split, or A is streamed; a matrix so wide
+// that its column blocks alone are GEMV_T_BLOCKS or more has the loads in
+// flight by its wavefronts, and bursts of rows a multiple of 64 KB apart only
+// crowd the same channels (us for U = 8 and 1: 128 x 65536 16.7 / 12.1, 100 x
+// 100000 14.7 / 13.0, 300 x 100000 38.7 / 35.1; 300 x 20000 13.0 / 16.4).
+constexpr int64_t GEMV_T_BLOCKS = 1024;
+
+template <bool STREAM, int U>
 __global__ __launch_bounds__(256) void gemv_t_kernel(int64_t m, int64_t n, int64_t rows_per_slice,
                                                      double alpha, const double* __restrict__ A, int64_t lda,
                                                      const double* __restrict__ x, double beta,
                                                      double* __restrict__ y, double* __restrict__ part) {
-  constexpr int U = 8;
   __shared__ double red[4][64];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -305,7 +310,7 @@ __global__ __launch_bounds__(256) void gemv_t_kernel(int64_t m, int64_t n, int64
   double s = 0.0;
   if (col < n) {
     int64_t i = r0 + wave;
-    for (; i + (U - 1) * 4 < r1; i += U * 4) {
+    for (; U > 1 && i + (U - 1) * 4 < r1; i += U * 4) {
       double v[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) v[u] = pamd_load<STREAM>(A + (i + 4 * u) * lda + col);
@@ -336,7 +341,7 @@ __global__ void gemv_t_reduce_kernel(int64_t n, int slices, double alpha, const 
 
 int gemv_t_slices(int64_t m, int64_t n) {
   const int64_t cb = pamd_cdiv(n, 64);
-  int64_t s = pamd_cdiv(1024, cb);
+  int64_t s = pamd_cdiv(GEMV_T_BLOCKS, cb);
   s = imin64(s, pamd_cdiv(m, 256));
   return (int)imax64(1, imin64(s, 1024));
 }
@@ -528,9 +533,11 @@ extern "C" int pamd_gemv_f64(int trans, int64_t m, int64_t n, double alpha, cons
   double* part = slices > 1 ? (double*)workspace : nullptr;
   dim3 grid((unsigned)pamd_cdiv(n, 64), (unsigned)slices);
   if (m * n * (int64_t)sizeof(double) > PAMD_STREAM_BYTES)
-    gemv_t_kernel<true><<<grid, 256, 0, st>>>(m, n, rps, alpha, A, lda, x, beta, y, part);
+    gemv_t_kernel<true, 8><<<grid, 256, 0, st>>>(m, n, rps, alpha, A, lda, x, beta, y, part);
+  else if (pamd_cdiv(n, 64) < GEMV_T_BLOCKS)
+    gemv_t_kernel<false, 8><<<grid, 256, 0, st>>>(m, n, rps, alpha, A, lda, x, beta, y, part);
   else
-    gemv_t_kernel<false><<<grid, 256, 0, st>>>(m, n, rps, alpha, A, lda, x, beta, y, part);
+    gemv_t_kernel<false, 1><<<grid, 256, 0, st>>>(m, n, rps, alpha, A, lda, x, beta, y, part);
   PAMD_LAUNCH_CHECK();
   if (part) {
     gemv_t_reduce_kernel<<<(unsigned)pamd_cdiv(n, 256), 256, 0, st>>>(n, slices, alpha, part, beta, y);

@@ -29,7 +29,7 @@ def _randn(*shape, seed=0):
 
 
 @pytest.mark.parametrize("m,n", [(1, 1), (3, 511), (5, 512), (5, 513), (2048, 2047), (2048, 2048), (2049, 2048),
-                                 (7, 20001), (31, 65), (32, 64), (33, 63), (5000, 200), (70000, 512)])
+                                 (7, 20001), (31, 65), (32, 64), (33, 63), (5000, 200), (70000, 512), (35, 65472), (35, 65473)])
 def test_gemv(ops, m, n):
     print(f"[gpu-passes] gemv {m} x {n}", flush=True)
     sys.stdout.flush()
