@@ -160,7 +160,8 @@ __global__ __launch_bounds__(BW_THREADS) void mlp_bwd_kernel(int64_t rows, doubl
   __shared__ float sum[MLP_NPARAM + 1];                // the wavefronts' sums over up to BW_TILES tiles each
   __shared__ double tot[LONG ? MLP_NPARAM + 1 : 1];    // the sums before those
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
-  const int wave = tid >> 6;
+  // scalar where that saves a spilled register (13 -> 11; with LONG it costs eight more)
+  const int wave = LONG ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint16_t* wb2 = wb + MLP_IN * MLP_H;
   for (int e = tid; e < 4 * 4 * 64; e += BW_THREADS) {
     const int hi = e >> 8, lo = (e >> 6) & 3, l = e & 63, lc = l & 15, lg = l >> 4;
