@@ -325,8 +325,8 @@ def main():
         ("sketch_SA_f64", 2.0 * dl * ml * nl, FP64_PEAK_TFLOPS * 1e12),
         ("qr_of_sketch", 2.0 * dl * (nl + 1) ** 2 - 2.0 * (nl + 1) ** 3 / 3, FP64_PEAK_TFLOPS * 1e12),
         ("lsqr_two_passes_per_iter", ls_iters * 2 * 8.0 * ml * nl, HBM_PEAK_GBS * 1e9)], t_ls)
-    ls_roof["dominant_kernels"] = "lsqr_tail_kernel (one workgroup, latency) and lsqr_pass_kernel (HBM); " \
-                                  "see profiles/ls_plain_20000x200_kernel_stats.md"
+    ls_roof["dominant_kernels"] = "lsqr_tailp_kernel (one workgroup, latency), lsqr_pass_kernel (cache) and " \
+                                  "lsqr_reduce_kernel; see spo_gauss in profiles/cases_kernel_stats.md"
 
     # the chosen path on the same problem: exact BF16 sketch + FP64 refinement
     # until eta <= 1e-10 (the metric's threshold)
@@ -356,7 +356,7 @@ def main():
     ls_chosen_roof["cg_iterations"] = int(lgc.inner_iterations)
     ls_chosen_roof["dominant_kernels"] = "normal_pass_kernel + its partial reduction and CG update per CG step " \
                                          "(three launches), the 200 x 200 triangular solves, potrf_reg; see " \
-                                         "profiles/ls_chosen_20000x200_kernel_stats.md"
+                                         "mixed_mid in profiles/cases_kernel_stats.md"
 
     # ------------------------------------------------------------- mixed LS
     mixed_extra = {}

@@ -98,8 +98,10 @@ int pamd_trsv_upper_f64(int trans, int64_t n, const double* R, int64_t ldr,
  * solved with more than once: pack writes both directions' blocks in the order
  * the solve reads them (query the size first; R may be freed afterwards, and
  * the packed copy serves any number of solves on any stream ordered after the
- * packing).  x <- R^{-1} x (trans = 0) or R^{-T} x in place; same rounding
- * bound as pamd_trsv_upper_f64.  Only R's upper triangle is read. */
+ * packing).  x <- R^{-1} x (trans = 0) or R^{-T} x in place.  The 8 x 8 blocks
+ * on R's diagonal are applied through their inverses, so the backward error is
+ * of order u times the largest condition number of those blocks, where
+ * pamd_trsv_upper_f64's is of order u.  Only R's upper triangle is read. */
 int pamd_trsv_pack_workspace(int64_t n, int64_t* bytes);
 int pamd_trsv_pack_f64(int64_t n, const double* R, int64_t ldr, void* packed,
                        void* stream);

@@ -600,8 +600,8 @@ extern "C" int pamd_trsv_upper_f64(int trans, int64_t n, const double* R, int64_
 }
 
 // The packed form (trsv_pack.h) for a triangle that is solved with more than
-// once, or once at n >= 192: one wide packing launch, then solves bound by the
-// chain through the diagonal.
+// once, or once where packing pays for itself (from n of about 144: ops.trsv_):
+// one wide packing launch, then solves bound by the chain through the diagonal.
 extern "C" int pamd_trsv_pack_workspace(int64_t n, int64_t* bytes) {
   PAMD_ARG_CHECK(n >= 0 && n <= TP_MAX_N, 1);
   PAMD_ARG_CHECK(bytes != nullptr, 2);

@@ -321,8 +321,8 @@ __device__ __forceinline__ void potrf_reg(int n, double* __restrict__ A, int64_t
 // columns), A22 -= R12^T R12 (one wavefront per 16 x 16 tile), then the
 // trailing matrix.  The middle steps use the whole chip and take about 8 us
 // each; one workgroup's matrix cores would need 40 us for the updates of n =
-// 266 alone (n = 266: 74 us this way, 87 with all of it in one workgroup's
-// registers, 150 in one with the matrix in memory; n = 512: 160 against 730).
+// 266 alone (n = 266: 78 us this way, 87 with all of it in one workgroup's
+// registers, 150 in one with the matrix in memory; n = 512: 165 against 736).
 // ---------------------------------------------------------------------------
 constexpr int PR_LEAD = 128;
 constexpr int PR_LT = PR_LEAD / PR_B;

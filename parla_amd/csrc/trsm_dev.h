@@ -1,5 +1,6 @@
-// Right triangular solve X = Y R^{-1} (R upper k x k, k <= 512) on FP64
-// MFMA, shared by the single-problem and the batched entry points.
+// Right triangular solve X = Y R^{-1} (R upper k x k) on FP64 MFMA, shared by
+// the single-problem and the batched entry points (k <= 512) and by the sketch
+// factorisation (k <= 1024: the strip then takes 142 of the 160 KB of LDS).
 #pragma once
 
 #include "common.h"
@@ -9,7 +10,7 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 namespace {
 
 // ---------------------------------------------------------------------------
-// X = Y R^{-1} for tall Y (m x k, k <= 512) on FP64 MFMA: one workgroup per
+// X = Y R^{-1} for tall Y (m x k) on FP64 MFMA: one workgroup per
 // 16-row strip, held in LDS and solved in place left to right in 16-column
 // blocks J:  X_J = (Y_J - X_{<J} R_{<J,J}) D_J  with D_J the inverse of the
 // diagonal block R_JJ (from trsm_dinv_body).  The update's K range is split

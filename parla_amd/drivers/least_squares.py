@@ -8,9 +8,10 @@ SPO (qr mode) on the device:
      buffer gets the rows [sqrt(delta) I | 0] (least_squares.py:309-310).
   2. R of the first n columns and z = Q^T [S b; 0] = Q[:d].T @ S b from the
      last one (least_squares.py:311-315): CholeskyQR2, its shifted form for an
-     ill-conditioned sketch, Householder QR otherwise (ops.sketch_rz_).
+     ill-conditioned sketch, Householder QR otherwise (ops.sketch_rz_; a host
+     read per form tried, two where the second round needs potrf).
   3. x_ske = R^{-1} z and the presolve test ||A x_ske - b|| / ||b|| < 1
-     (least_squares.py:316, 343-351) -- the one host synchronisation.
+     (least_squares.py:316, 343-351): another host read.
   4. PcSS2 -> device LSQR on [A; sqrt(delta) I] R^{-1} from z (or from 0).
   5. With logging: errors = [||R^{-T} A^T b||, arnorms...] (least_squares.py:360-367).
 """
