@@ -139,14 +139,16 @@ __device__ __forceinline__ bool jac_in_range(double al) { return !(al > 0x1p480 
 
 // The slow path for a round with columns outside that (1e-60 .. 1e72 in
 // length): whether the pair is to be rotated, with al, be and ga scaled by a
-// power of two where their products do not fit, and d, g by the one that makes
-// the larger of them about 1, with their h^2.
+// power of two where their products overflow, and d, g by the one that makes
+// the larger of them about 1, with their h^2.  Where the products underflow the
+// test stays as it is: a pair whose ga^2 is 0 is left alone, which ends the
+// sweeps on the columns of a rank-one triangle (1e-16, 1e-32, .. in length) that
+// cannot be made orthogonal to a relative tolerance among subnormal numbers.
 __device__ __forceinline__ bool jac_wide(double al, double be, double ga, double tol2, double& d, double& g,
                                          double& h2) {
   d = be - al;
   g = 2.0 * ga;
-  const double p = al * be;
-  int e = (p > 0x1p-800 && p < 0x1p1000) ? 0 : -__builtin_amdgcn_frexp_exp(fmax(al, be));
+  int e = al * be < 0x1p1000 ? 0 : -__builtin_amdgcn_frexp_exp(fmax(al, be));
   const double c = ldexp(ga, e);
   const bool rot = c * c > tol2 * (ldexp(al, e) * ldexp(be, e));
   e = -__builtin_amdgcn_frexp_exp(fmax(fabs(d), fabs(g)));

@@ -106,6 +106,23 @@ def test_rotations_over_a_wide_range(ops, scale):
         assert abs(s[0] - ref[0]) <= tol * ref[0]
 
 
+@pytest.mark.parametrize("m,n", [(17, 16), (40, 12), (300, 30), (30, 300), (200, 100)])
+@pytest.mark.parametrize("kind", ["one column repeated", "ones", "outer", "two of each"])
+def test_rank_deficient_matrices_down_to_underflow(ops, m, n, kind):
+    """Equal columns leave a QR factor with rows of length 1e-16, 1e-32, ..,
+    down to subnormal numbers: the sweeps end, the singular values that are
+    not rounding errors are right, and so is the product."""
+    print(f"[gpu-jacobi-rounds] {kind} {m} x {n}", flush=True)
+    rng = np.random.default_rng(0)
+    X = rng.standard_normal((m, n))
+    A = {"one column repeated": np.repeat(X[:, :1], n, axis=1), "ones": np.ones((m, n)),
+         "outer": np.outer(X[:, 0], X[0]), "two of each": np.repeat(X[:, :(n + 1) // 2], 2, axis=1)[:, :n]}[kind]
+    U, s, Vh = (t.cpu().numpy() for t in ops.thin_svd(torch.from_numpy(np.ascontiguousarray(A)).cuda()))
+    tol = 50 * EPS * max(m, n, 16)
+    assert np.max(np.abs(s - np.linalg.svd(A, compute_uv=False))) <= tol * s[0]
+    assert np.linalg.norm((U * s) @ Vh - A) <= tol * np.linalg.norm(A)
+
+
 def test_orthogonal_columns_are_left_alone(ops):
     n = 40
     A = np.zeros((n + 3, n))
